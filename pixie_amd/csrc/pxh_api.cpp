@@ -146,10 +146,6 @@ struct Ctx {
   // own blur temporary and scene row scratch, so that work issued on
   // different lanes (by different host threads) overlaps on the device.
   hipStream_t lane[kLanes] = {};
-  // per lane: a second stream and fork / join events for phase A's two
-  // concurrent launches
-  hipStream_t laneAux[kLanes] = {};
-  hipEvent_t laneFork[kLanes] = {}, laneJoin[kLanes] = {};
   DevBuf laneTmp[kLanes];
   DevBuf laneScratch[kLanes];
   std::mutex lutMu;
@@ -224,11 +220,6 @@ int init() {
   PXH_HIP(hipStreamCreate(&g.stream));
   g.lane[0] = g.stream;
   for (int l = 1; l < kLanes; l++) PXH_HIP(hipStreamCreate(&g.lane[l]));
-  for (int l = 0; l < kLanes; l++) {
-    PXH_HIP(hipStreamCreate(&g.laneAux[l]));
-    PXH_HIP(hipEventCreateWithFlags(&g.laneFork[l], hipEventDisableTiming));
-    PXH_HIP(hipEventCreateWithFlags(&g.laneJoin[l], hipEventDisableTiming));
-  }
   PXH_HIP(hipEventCreateWithFlags(&g.stageFree, hipEventDisableTiming));
   PXH_HIP(hipEventRecord(g.stageFree, g.stream));
   PXH_HIP(hipMalloc((void**)&g.errFlag, sizeof(int32_t)));
@@ -849,7 +840,7 @@ int scene_alloc(pxh_scene* sc) {
   size_t oParts = carve((size_t)sc->bandCap * sizeof(PartInfo)), oBI = carve((size_t)sc->bandCap * 4);
   size_t oEnt = carve((size_t)sc->entryCap * sizeof(Entry)), oEW = carve((size_t)sc->entryCap);
   size_t oTask = carve((size_t)sc->taskCap * sizeof(RowRuns)), oRun = carve((size_t)sc->runCap * 8);
-  size_t oTaskItem = carve((size_t)sc->taskCap * 4), oTaskOrd = carve((size_t)sc->taskCap * 4);
+  size_t oTaskItem = carve((size_t)sc->taskCap * 4), oTaskOrd = carve((size_t)sc->taskCap * 8);
   size_t oTaskCls = carve((size_t)sc->taskCap);
   size_t oRows = carve(nI * sizeof(int4)), oBinC = carve((size_t)sc->binSlots * 4);
   size_t oPaint = carve(nI * sizeof(int4)), oSpan = carve(nI * sizeof(int4));
@@ -1074,9 +1065,7 @@ int scene_launch(pxh_scene* sc, pxh_image* img, int lane, bool checked = false) 
   p.dashes = sc->dDashes;
   const RowShape shape = kRowShapes[sc->rowShape];
   p.ldsCap = shape.ldsCap;
-  // tasks of bands of more than ldsCap entries go to the large-band launch;
-  // a single-launch shape has none (class 32 is never reached)
-  p.bigClass = shape.mode ? 32 - __builtin_clz((unsigned)shape.ldsCap) : kCostClasses;
+  p.heavyClass = shape.heavyClass;
   DevBuf& scr = g.laneScratch[lane];
   if (int e = scr.ensure(scene_gscratch_bytes(scene_scratch_slots(shape, g.numCUs), sc->gcap)))
     return fail(e, "scene row scratch allocation failed");
@@ -1096,7 +1085,7 @@ int scene_launch(pxh_scene* sc, pxh_image* img, int lane, bool checked = false) 
   }
   if (!r) {
     LaunchTimer t("scene_rows_kernel", st);
-    r = scene_launch_rows(p, shape, g.numCUs, st, g.laneAux[lane], g.laneFork[lane], g.laneJoin[lane]);
+    r = scene_launch_rows(p, shape, g.numCUs, st);
   }
   if (!r) {
     LaunchTimer t("scene_compose_kernel", st);

@@ -43,9 +43,8 @@ struct RowLds {
   float* tx0;        // cap: trapezoid x at scanTop (by selection position)
   float* tx1;        // cap: trapezoid x at scanBottom
   int cap, ww;
-  uint64_t* wide;    // LDS staging of the wide path's hit keys (wideCap of
-  int wideCap;       // them; 0 turns it off): AX, which coverage rows leave
-                     // free, and the cap arrays after it when they are in LDS
+  uint32_t* stage;   // LDS staging of the wide path's hit keys: AX, which
+  int stageCap;      // coverage rows leave free
 };
 
 PXH_HD size_t row_lds_fixed_bytes(int ww) { return (size_t)(ww + 4) * 4 + (size_t)ww * 4; }
@@ -63,8 +62,8 @@ __device__ __forceinline__ RowLds row_lds_carve(char* fixed, char* arr, int cap,
   L.B = L.A + cap;
   L.tx0 = (float*)(L.B + cap);
   L.tx1 = L.tx0 + cap;
-  L.wide = nullptr;
-  L.wideCap = 0;
+  L.stage = L.AX;
+  L.stageCap = ww;
   return L;
 }
 
@@ -78,7 +77,7 @@ __device__ __forceinline__ uint64_t ballot(bool p) { return __ballot(p); }
 // identity.  No LDS traffic, about two VALU operations per step.
 constexpr int kDppRowShr1 = 0x111, kDppRowShr2 = 0x112, kDppRowShr4 = 0x114,
               kDppRowShr8 = 0x118, kDppRowBcast15 = 0x142, kDppRowBcast31 = 0x143,
-              kDppWaveShr1 = 0x138;
+              kDppWaveShr1 = 0x138, kDppWaveShl1 = 0x130;
 
 __device__ __forceinline__ int32_t wave_incl_sum(int32_t v) {
   v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr1, 0xf, 0xf, false);
@@ -120,30 +119,145 @@ __device__ __forceinline__ int32_t wave_max(int32_t v) {
   return __builtin_amdgcn_readlane(wave_incl_max(v), kWave - 1);
 }
 
-// Scans inside independent SEG-lane segments of the wave (SEG = 16 or 32).
-template <int SEG>
-__device__ __forceinline__ int32_t seg_incl_sum(int32_t v) {
-  v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr1, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr2, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr4, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, kDppRowShr8, 0xf, 0xf, false);
-  if (SEG == 32) v += __builtin_amdgcn_update_dpp(0, v, kDppRowBcast15, 0xa, 0xf, false);
-  return v;
+// Orders the wave's own LDS and scratch accesses: one lane's stores before
+// the fence are seen by every lane's loads after it (a wave's memory
+// operations run in order).  Not a workgroup barrier, so the waves of a
+// larger workgroup may run row programs independently.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-template <int SEG>
-__device__ __forceinline__ int32_t seg_excl_max(int32_t v) {
-  const int32_t lo = INT32_MIN;
-  v = imax(v, __builtin_amdgcn_update_dpp(lo, v, kDppRowShr1, 0xf, 0xf, false));
-  v = imax(v, __builtin_amdgcn_update_dpp(lo, v, kDppRowShr2, 0xf, 0xf, false));
-  v = imax(v, __builtin_amdgcn_update_dpp(lo, v, kDppRowShr4, 0xf, 0xf, false));
-  v = imax(v, __builtin_amdgcn_update_dpp(lo, v, kDppRowShr8, 0xf, 0xf, false));
-  if (SEG == 32) v = imax(v, __builtin_amdgcn_update_dpp(lo, v, kDppRowBcast15, 0xa, 0xf, false));
-  v = __builtin_amdgcn_update_dpp(lo, v, kDppWaveShr1, 0xf, 0xf, false);
-  return (lane_id() & (SEG - 1)) == 0 ? lo : v;
+// ---- 32-bit key sorts in registers ----
+// Value of the lane whose number differs in bit S (S = 1, 2, 4, 8), by DPP
+// moves inside a 16-lane row.
+constexpr int kDppQuadXor1 = 0xB1, kDppQuadXor2 = 0x4E, kDppQuadXor3 = 0x1B, kDppHalfMirror = 0x141,
+              kDppRowRor8 = 0x128;
+template <int S>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v) {
+  if (S == 1) return __builtin_amdgcn_mov_dpp(v, kDppQuadXor1, 0xf, 0xf, true);
+  if (S == 2) return __builtin_amdgcn_mov_dpp(v, kDppQuadXor2, 0xf, 0xf, true);
+  if (S == 4)  // i -> 7 - i inside eight lanes, then i -> 3 - i inside four
+    return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, kDppHalfMirror, 0xf, 0xf, true), kDppQuadXor3,
+                                    0xf, 0xf, true);
+  return __builtin_amdgcn_mov_dpp(v, kDppRowRor8, 0xf, 0xf, true);
+}
+// Compare-exchange with the lane at distance S: the lower lane of the pair
+// keeps the smaller key.  At 16 and 32 the lane swaps of gfx950 give every
+// lane both keys of its pair.
+template <int S>
+__device__ __forceinline__ uint32_t cmp_exchange(uint32_t k, bool lower) {
+  uint32_t a = k, b;
+  if (S == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(k, k, false, false);
+    a = r[0];
+    b = r[1];
+  } else if (S == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(k, k, false, false);
+    a = r[0];
+    b = r[1];
+  } else {
+    b = lane_xor<S>(k);
+  }
+  const uint32_t mn = a < b ? a : b, mx = a < b ? b : a;
+  return lower ? mn : mx;
 }
 
-__device__ __forceinline__ void wave_sync() { __syncthreads(); }
+// Ascending bitonic sort inside every SEG-lane segment of the wave.
+template <int SEG>
+__device__ __forceinline__ uint32_t seg_sort32(uint32_t k) {
+  const int lane = threadIdx.x & (kWave - 1);
+  uint32_t held = 0;
+#pragma unroll
+  for (int size = 2; size <= SEG; size <<= 1) {
+    const uint32_t want = size < SEG ? (uint32_t)-(int32_t)((lane & size) != 0) : 0u;
+    k ^= held ^ want;
+    held = want;
+#pragma unroll
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      const bool lower = (lane & stride) == 0;
+      if (stride == 16) k = cmp_exchange<16>(k, lower);
+      if (stride == 8) k = cmp_exchange<8>(k, lower);
+      if (stride == 4) k = cmp_exchange<4>(k, lower);
+      if (stride == 2) k = cmp_exchange<2>(k, lower);
+      if (stride == 1) k = cmp_exchange<1>(k, lower);
+    }
+  }
+  return k;
+}
+
+// Ascending bitonic sort of the 64 * NS keys k[s] of lane l (key s * 64 + l).
+// Blocks a stage sorts downwards are held complemented meanwhile, so every
+// exchange keeps the minimum in the lower place: 3 to 5 VALU instructions
+// per exchange and no LDS traffic, against two LDS permutes and about ten
+// VALU instructions for 64-bit keys.
+template <int NS>
+__device__ __forceinline__ void wave_sort32(uint32_t (&k)[NS]) {
+  const int lane = threadIdx.x & (kWave - 1);
+  uint32_t held = 0;  // complement now applied by lane
+#pragma unroll
+  for (int size = 2; size <= kWave * NS; size <<= 1) {
+    const uint32_t want = size < kWave ? (uint32_t)-(int32_t)((lane & size) != 0) : 0u;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+      const uint32_t slotWas = size > kWave && (((s * kWave) & (size >> 1)) != 0) ? ~0u : 0u;
+      const uint32_t slotNow = size >= kWave && size < kWave * NS && (((s * kWave) & size) != 0) ? ~0u : 0u;
+      k[s] ^= held ^ want ^ slotWas ^ slotNow;
+    }
+    held = want;
+#pragma unroll
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      if (stride >= kWave) {
+        const int d = stride / kWave;
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+          if (s & d) continue;
+          const uint32_t a = k[s], b = k[s | d];
+          k[s] = a < b ? a : b;
+          k[s | d] = a < b ? b : a;
+        }
+        continue;
+      }
+      const bool lower = (lane & stride) == 0;
+#pragma unroll
+      for (int s = 0; s < NS; s++) {
+        if (stride == 32) k[s] = cmp_exchange<32>(k[s], lower);
+        if (stride == 16) k[s] = cmp_exchange<16>(k[s], lower);
+        if (stride == 8) k[s] = cmp_exchange<8>(k[s], lower);
+        if (stride == 4) k[s] = cmp_exchange<4>(k[s], lower);
+        if (stride == 2) k[s] = cmp_exchange<2>(k[s], lower);
+        if (stride == 1) k[s] = cmp_exchange<1>(k[s], lower);
+      }
+    }
+  }
+}
+
+// Ascending sort of n keys in memory by one wave, any n: a bitonic network
+// whose every exchange points upwards (each merge starts with a mirrored
+// pass), so keys past n act as the largest and are left out.
+__device__ __forceinline__ void wave_sort32_mem(uint32_t* keys, int n) {
+  const int lane = threadIdx.x & (kWave - 1);
+  int np = 2;
+  while (np < n) np <<= 1;
+  for (int size = 2; size <= np; size <<= 1) {
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      const bool mirror = stride == (size >> 1);
+      for (int t = lane; t < np / 2; t += kWave) {
+        const int r = t & (stride - 1);
+        const int i = 2 * t - r;
+        const int j = mirror ? i + 2 * (stride - r) - 1 : i + stride;
+        if (j < n) {
+          const uint32_t a = keys[i], b = keys[j];
+          if (a > b) {
+            keys[i] = b;
+            keys[j] = a;
+          }
+        }
+      }
+      wave_sync();
+    }
+  }
+}
 
 // Bitonic sort of n keys in L.keys (n <= cap, cap a power of two).  Keys
 // beyond n are padded with UINT64_MAX.  The whole wave participates.
@@ -315,41 +429,6 @@ __device__ void wave_walk(RowLds& L, int n, int32_t rule, SpanFn& span) {
   }
 }
 
-// wave_walk<true> for at most 64 sorted hits held in registers (hit i in
-// lane i, padding keys ~0 beyond n), the next hit taken from the next lane.
-template <class SpanFn>
-__device__ __forceinline__ void wave_walk_reg(uint64_t k, int n, int32_t rule, SpanFn& span) {
-  const int lane = lane_id();
-  const bool valid = lane < n;
-  const bool hasNext = valid && lane < n - 1;
-  const uint64_t kn = __shfl(k, lane + 1 < kWave ? lane + 1 : lane, kWave);
-  WalkCarry c;
-  walk_chunk(valid ? key_at(k) : 0, valid ? key_winding(k) : 0, valid, hasNext,
-             hasNext ? key_at(kn) : 0, hasNext ? key_winding(kn) : 0, rule, c, span);
-}
-
-// One odd-even transposition step over the wave's keys (pairs (2m, 2m+1), or
-// with odd (2m+1, 2m+2)); the lower lane of a pair keeps the smaller key.
-// Returns whether this lane took its partner's key.
-__device__ __forceinline__ bool wave_transpose(uint64_t& k, bool odd) {
-  const int lane = lane_id();
-  bool lower, has;
-  int src;
-  if (!odd) {
-    lower = (lane & 1) == 0;
-    has = true;
-    src = lane ^ 1;
-  } else {
-    lower = (lane & 1) == 1;
-    has = lower ? lane + 1 < kWave : lane > 0;
-    src = lower ? (lane + 1 < kWave ? lane + 1 : lane) : (lane > 0 ? lane - 1 : lane);
-  }
-  const uint64_t o = __shfl(k, src, kWave);
-  const bool take = has && (lower ? o < k : o > k);
-  if (take) k = o;
-  return take;
-}
-
 // Coverage contributions of one span (computeCoverage 1390-1431).
 struct CovSpan {
   const RowCtx* C;
@@ -453,103 +532,217 @@ __device__ __forceinline__ int row_hits(const RowCtx& C, RowLds& L, int ne, floa
   return nh;
 }
 
-// The 5-sample coverage of a row whose selection holds at most SEG entries
-// (computeCoverage 1350-1431 with walk 1298-1334), 64 / SEG sample lines at a
-// time, one per SEG-lane segment of the wave: two passes for SEG = 16, three
-// for SEG = 32, instead of five.  Lane SEG*g + i works on entry i for sample
-// line g of the pass.  A segment holds one whole sample line, so the walk
-// needs no carries between chunks.  S holds selection i in lane i.
+// ---- sample lines by 32-bit keys ----
+// A window's walk needs only the hits inside it: the windings of the hits
+// left of it give the count it starts with, and a span open at its end is
+// known to end later when the windings of the whole line sum to 0 (the count
+// then returns to 0 at a hit that no skip consumes).  So a hit's key is 32
+// bits: its 24.8 position from the window's start, its place in the selection
+// (pixie's stable order of equal x) and the sign of its winding; the keys
+// sort in registers, with no LDS traffic.  A line whose windings do not sum
+// to 0 is walked whole (row_hits and wave_walk).
+//
+// Every span (p, a) of the walk is added as two independent parts, one at
+// its start and one at its end: with L = floor((256 - frac p) * sc / 256) and
+// R = floor(frac a * sc / 256), D gets L and sc - L at p's pixel and the
+// next, R - sc and -R at a's pixel and the next, which sum to what
+// computeCoverage (1390-1431) adds.  Only when p and a share a pixel do the
+// two roundings differ from the one of (a - p) * sc; the end then adds the
+// difference.  Positions are clamped to the columns the coverage may write,
+// which clips spans as computeCoverage clips them.
+//
+// The row program is bound by instruction issue; per 64 hits the 64-bit form
+// of this path took about 250 instructions to sort (LDS permutes) and 250 to
+// walk (scans, up to six LDS atomics a span), this one 110 and 90 (lane masks,
+// two atomics an event): rows of the 4096 x 4096 scene 957 -> 636 us, of the
+// 10,000-glyph atlas 617 -> 515 us.
+constexpr int kSampleCov = 255 / 5;
+
+// Lanes below this one in its SEG-lane segment, as a 64-bit lane mask.
 template <int SEG>
-__device__ __forceinline__ void row_coverage_small(const RowCtx& C, RowLds& L, int ne, SelCache S, float y0,
-                                   float y1, float y2, float y3, float y4, int32_t rule,
-                                   CovSpan& span) {
-  constexpr int kPer = kWave / SEG;                 // sample lines per pass
+__device__ __forceinline__ uint64_t seg_below() {
+  const int lane = lane_id();
+  return ((1ull << lane) - 1ull) & ~((1ull << (lane & ~(SEG - 1))) - 1ull);
+}
+// Set bits of m below this lane in its segment, plus acc.
+template <int SEG>
+__device__ __forceinline__ int32_t seg_rank(uint64_t m) {
+  if (SEG == kWave) return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+  return __popcll(m & seg_below<SEG>());
+}
+
+struct Walk32 {
+  int32_t count = 0;      // winding count before the chunk (per segment)
+  int32_t prev = -1;      // position of the last event before the chunk
+  bool consumed = false;  // the chunk's first hit was consumed by a skip
+};
+
+// One chunk of the walk over sorted keys (position << IB | order << 1 |
+// winding is 1): lane i of a segment holds hit i when valid, kn the key
+// after it when hasNext.  Positions are relative to the pixel D points at,
+// [lo, hi) are the pixels that may be written.
+template <int IB, int SEG>
+__device__ __forceinline__ void walk32(uint32_t k, uint32_t kn, bool valid, bool hasNext, int32_t rule, int32_t* D,
+                                       int32_t lo, int32_t hi, Walk32& c) {
+  const int lane = lane_id();
+  const bool up = (k & 1u) != 0;
+  const uint64_t pos = ballot(valid && up), neg = ballot(valid && !up);
+  const int32_t cb = c.count + seg_rank<SEG>(pos) - seg_rank<SEG>(neg);
+  const bool filling = should_fill(rule, cb);
+  // a hit and the next at the same x whose windings cancel are skipped
+  uint64_t cm = ballot(valid && filling && hasNext && ((k ^ kn) >> IB) == 0 && ((k ^ kn) & 1u));
+  bool off = false;
+  if (cm != 0 || c.consumed) {
+    uint64_t skip = 0, cons = c.consumed ? 1ull : 0ull;
+    bool carry = false;
+    while (cm) {
+      const int b = __builtin_ctzll(cm);
+      cm &= cm - 1;
+      if (!((cons >> b) & 1ull)) {
+        skip |= 1ull << b;
+        if (b + 1 < kWave) cons |= 1ull << (b + 1);
+        else carry = true;
+      }
+    }
+    off = ((skip | cons) >> lane) & 1ull;
+    c.consumed = carry;
+  }
+  const bool act = valid && !off;
+  const bool start = act && !filling;
+  const bool end = act && filling && !(rule == kNonZero && cb + (up ? 1 : -1) != 0);
+  const int32_t rel = (int32_t)(k >> IB);
+  int32_t r = rel > (lo << 8) ? rel : (lo << 8);
+  r = r < (hi << 8) ? r : (hi << 8);
+  const int32_t f = r & 255, px = r >> 8;
+  int32_t v0 = ((start ? 256 - f : f) * kSampleCov) >> 8;
+  if (!start) v0 -= kSampleCov;
+  int32_t v1 = (start ? kSampleCov : -kSampleCov) - v0;
+  // ends whose start may share their pixel: the hit before them does
+  const uint64_t em = ballot(start || end);
+  const uint32_t kp = __builtin_amdgcn_update_dpp(~0u, k, kDppWaveShr1, 0xf, 0xf, false);
+  const bool first = (lane & (SEG - 1)) == 0;
+  const bool near = end && (first ? c.prev >> 8 == rel >> 8 : ((kp ^ k) >> (IB + 8)) == 0);
+  if (ballot(near)) {
+    const uint64_t before = em & seg_below<SEG>();
+    const int src = before ? 63 - __builtin_clzll(before) : lane;
+    const int32_t ps = __shfl(rel, src, kWave);
+    const int32_t p = before ? ps : c.prev;
+    if (near && (p >> 8) == (rel >> 8) && p >= 0 && r == rel && px < hi) {
+      const int32_t left = ((256 - (p & 255)) * kSampleCov) >> 8;  // what p's start added
+      const int32_t whole = ((rel - p) * kSampleCov) >> 8;
+      const int32_t fix = whole - (left + v0);
+      v0 += fix;
+      v1 -= fix;
+    }
+  }
+  if (start || end) {
+    atomicAdd(&D[px], v0);
+    atomicAdd(&D[px + 1], v1);
+  }
+  if (SEG == kWave) {
+    c.count += __popcll(pos) - __popcll(neg);
+    if (em) c.prev = __builtin_amdgcn_readlane(rel, 63 - __builtin_clzll(em));
+  }
+}
+
+// What a line filled at the window's start or end adds there.
+__device__ __forceinline__ void walk32_borders(bool fillStart, bool fillEnd, int32_t* D, int32_t lo, int32_t hi) {
+  if (fillStart) atomicAdd(&D[lo], kSampleCov);
+  if (fillEnd) atomicAdd(&D[hi], -kSampleCov);
+}
+
+// A row window's place for the 32-bit walks.
+struct Win32 {
+  int32_t A, A1, B;  // 24.8 bounds of its hits (a hit at or left of x = 0 only counts)
+  int32_t lo, hi;    // columns the coverage may write, from the window's start
+};
+__device__ __forceinline__ Win32 window32(const RowCtx& C) {
+  const int32_t covLo = C.F->startX, covHi = covLo + C.F->pathWidth;
+  Win32 w;
+  w.A = C.wx0 * 256;
+  w.A1 = w.A > 1 ? w.A : 1;
+  w.B = C.wx1 * 256;
+  w.lo = (covLo > C.wx0 ? covLo : C.wx0) - C.wx0;
+  w.hi = (covHi < C.wx1 ? covHi : C.wx1) - C.wx0;
+  return w;
+}
+constexpr int kKeyBits = 15;  // order (14 bits) and winding below the position (17 bits in 512 px)
+
+// 24.8 x of an entry's hit on a sample line (1373-1388).
+__device__ __forceinline__ int32_t hit_at(const Entry& e, float yLine, float Wf) {
+  const float x = e.m == 0.0f ? e.b : (yLine - e.b) / e.m;
+  return fixed32(nim_minf(x, Wf));
+}
+
+// The 5-sample coverage of a row that selects at most SEG entries (held by
+// lanes 0..ne-1 of S): 64 / SEG sample lines at a time, one per segment of
+// the wave -- all five for SEG = 8, two passes for 16, three for 32, five for
+// 64.  A segment holds one whole line, so the walk needs no carries.  yLine
+// is one step before the first line.  Returns the lines whose windings do
+// not sum to 0 (bit m: line m), which are left to be
+// walked whole.
+template <int SEG>
+__device__ __forceinline__ uint32_t row_coverage_seg(const RowCtx& C, RowLds& L, int ne, SelCache S, float yLine,
+                                                     float offset, int32_t rule) {
+  constexpr int kPer = kWave / SEG;
   constexpr int kPasses = (5 + kPer - 1) / kPer;
   const int lane = lane_id();
   const int grp = lane / SEG, i = lane & (SEG - 1);
   const float Wf = (float)C.F->canvasW;
-  // entry i of the selection in every segment
-  Entry e;
-  e.aty = __shfl(S.e.aty, i, kWave);
-  e.toy = __shfl(S.e.toy, i, kWave);
-  e.m = __shfl(S.e.m, i, kWave);
-  e.b = __shfl(S.e.b, i, kWave);
-  const int32_t ew = __shfl(S.w, i, kWave);
-  uint64_t* sorted = (uint64_t*)L.tx0;  // 64 sorted keys (tx0/tx1 are free here)
-  const int base = SEG * grp;
+  const Win32 w = window32(C);
+  Entry e = S.e;
+  int32_t ew = S.w;
+  if (SEG < kWave) {
+    e.aty = __shfl(S.e.aty, i, kWave);
+    e.toy = __shfl(S.e.toy, i, kWave);
+    e.m = __shfl(S.e.m, i, kWave);
+    e.b = __shfl(S.e.b, i, kWave);
+    ew = __shfl(S.w, i, kWave);
+  }
+  uint32_t whole = 0;
+  const uint64_t segMask = SEG == kWave ? ~0ull : ((1ull << (SEG & 63)) - 1ull) << (grp * SEG);
+#pragma unroll 1
   for (int pass = 0; pass < kPasses; pass++) {
     const int sample = pass * kPer + grp;
-    // the sample line of this segment, selected from registers
-    const float yl = sample == 0 ? y0 : sample == 1 ? y1 : sample == 2 ? y2 : sample == 3 ? y3 : y4;
-    // hits (1373-1388), compacted per segment in entry order
-    bool hit = false;
-    int32_t at = 0;
-    if (sample < 5 && i < ne && e.aty <= yl && e.toy >= yl) {
-      float x = e.m == 0.0f ? e.b : (yl - e.b) / e.m;
-      at = fixed32(nim_minf(x, Wf));
-      hit = true;
+    float y = yLine;
+#pragma unroll
+    for (int g = 0; g < kPer && g < 5; g++) {
+      yLine += offset;
+      y = grp == g ? yLine : y;
     }
-    const uint64_t m = ballot(hit);
-    const uint64_t segMask = (m >> base) & (SEG == 32 ? 0xffffffffull : 0xffffull);
-    const int nh = __popcll(segMask);
-    const int pos = __popcll(segMask & ((1ull << i) - 1ull));
-    // (x, position << 8 | winding): the winding rides in the low byte
-    const uint64_t key = ((uint64_t)((uint32_t)at ^ 0x80000000u) << 32) |
-                         ((uint32_t)pos << 8) | (uint32_t)(uint8_t)ew;
-    if (hit) L.keys[base + pos] = key;
-    wave_sync();
-    // stable sort by (x, position): rank among the segment's hits
-    if (hit) {
-      int rank = 0;
-      for (int j = 0; j < nh; j++) rank += L.keys[base + j] < key ? 1 : 0;
-      sorted[base + rank] = key;
+    const bool hit = sample < 5 && i < ne && e.aty <= y && e.toy >= y;
+    const int32_t at = hit_at(e, y, Wf);
+    const uint64_t up = ballot(hit && ew > 0), down = ballot(hit && ew <= 0);
+    const bool isLeft = hit && at < w.A1, in = hit && !isLeft && at < w.B;
+    const uint64_t inM = ballot(in), leftM = ballot(isLeft);
+    const bool open = __popcll(up & segMask) != __popcll(down & segMask);  // the windings do not sum to 0
+    const uint64_t openM = ballot(open);
+    if (w.lo < w.hi) {
+      const int32_t left = __popcll(leftM & up & segMask) - __popcll(leftM & down & segMask);
+      const int32_t after = left + __popcll(inM & up & segMask) - __popcll(inM & down & segMask);
+      const int n = __popcll(inM & segMask);
+      uint32_t k = in ? ((uint32_t)(at - w.A) << kKeyBits) | ((uint32_t)i << 1) | (ew > 0 ? 1u : 0u) : ~0u;
+      uint32_t ks[1] = {k};
+      if (SEG == kWave) wave_sort32<1>(ks);
+      k = SEG == kWave ? ks[0] : seg_sort32<SEG>(k);
+      const uint32_t kn = __builtin_amdgcn_update_dpp(~0u, k, kDppWaveShl1, 0xf, 0xf, false);
+      Walk32 c;
+      c.count = left;
+      walk32<kKeyBits, SEG>(k, kn, i < n && !open, i < n - 1, rule, L.D, w.lo, w.hi, c);
+      if (i == 0 && !open) walk32_borders(should_fill(rule, left), should_fill(rule, after), L.D, w.lo, w.hi);
     }
-    wave_sync();
-    // walk: lane SEG*g + p holds the p-th hit of segment g
-    const bool valid = i < nh;
-    const uint64_t k = valid ? sorted[base + i] : 0ull;
-    const int32_t hat = valid ? key_at(k) : 0;
-    const int32_t w = valid ? key_winding(k) : 0;
-    const int32_t countBefore = seg_incl_sum<SEG>(w) - w;
-    const bool filling = should_fill(rule, countBefore);
-    const bool hasNext = valid && i < nh - 1;
-    const uint64_t kn = hasNext ? sorted[base + i + 1] : 0ull;
-    const int32_t nextAt = hasNext ? key_at(kn) : 0;
-    const int32_t nextW = hasNext ? key_winding(kn) : 0;
-    const bool canSkip = valid && hat > 0 && filling && hasNext && nextAt == hat && w + nextW == 0;
-    uint64_t cm = ballot(canSkip);
-    uint64_t skipMask = 0, consMask = 0;
-    while (cm) {
-      const int b = __builtin_ctzll(cm);
-      cm &= cm - 1;
-      if (!((consMask >> b) & 1ull)) {
-        skipMask |= 1ull << b;
-        if (((b + 1) & (SEG - 1)) != 0) consMask |= 1ull << (b + 1);  // stays in its segment
-      }
-    }
-    const bool consumed = (consMask >> lane) & 1ull;
-    const bool skipStart = (skipMask >> lane) & 1ull;
-    int ev = 0;  // 0 none, 1 start, 2 end (yield)
-    if (valid && !consumed && !skipStart && hat > 0) {
-      if (filling) {
-        const bool cont = (rule == kNonZero) && hasNext && (countBefore + w != 0);
-        ev = cont ? 0 : 2;
-      } else {
-        ev = 1;
-      }
-    }
-    int32_t prevAt = seg_excl_max<SEG>(ev ? hat : INT32_MIN);
-    if (prevAt < 0) prevAt = 0;  // prevAt starts at 0 (walk 1300)
-    if (ev == 2) span(prevAt, hat);
-    wave_sync();
+    if (openM)
+#pragma unroll
+      for (int g = 0; g < kPer && g < 5; g++)
+        if ((openM >> (g * SEG)) & 1ull) whole |= 1u << (pass * kPer + g);
   }
+  return whole;
 }
 
 // Finishes sorting n distinct keys that are nearly in order: odd-even
 // transposition passes until one swaps nothing, and a full sort once
-// kFixPasses passes have not been enough.
-constexpr int kFixPasses = 8;     // keys in registers
-constexpr int kFixPassesMem = 16;  // keys in LDS or global memory (more than 64 hits)
+// kFixPassesMem passes have not been enough.
+constexpr int kFixPassesMem = 16;
 __device__ void wave_fix_keys(uint64_t* keys, int n, int cap) {
   const int lane = lane_id();
   for (int pass = 0;; pass++) {
@@ -573,7 +766,7 @@ __device__ void wave_fix_keys(uint64_t* keys, int n, int cap) {
   }
 }
 
-// The 5-sample coverage of a row with any number of selected entries
+// The 5-sample coverage of a row of more entries than the wide path takes
 // (computeCoverage 1350-1431).  pixie sorts each sample line's hits from
 // scratch (sort 1373-1388).  Here the selection is sorted once, by x where
 // each entry is nearest the row's middle; every sample line then collects
@@ -582,8 +775,8 @@ __device__ void wave_fix_keys(uint64_t* keys, int n, int cap) {
 // the selection index as tie-break, which orders equal x like pixie's
 // insertion sort over hits collected in selection order, and the winding in
 // their low byte, so the walk reads it from the key.
-__device__ __forceinline__ void row_coverage_presorted(const RowCtx& C, RowLds& L, int ne, SelCache S,
-                                       float yLine, float offset, int32_t rule, CovSpan& span) {
+__device__ __forceinline__ void row_coverage_presorted(const RowCtx& C, RowLds& L, int ne, float yLine,
+                                                       float offset, int32_t rule, CovSpan& span) {
   const int lane = lane_id();
   const float Wf = (float)C.F->canvasW;
   const float yMid = (float)C.y + 0.5f;
@@ -592,39 +785,21 @@ __device__ __forceinline__ void row_coverage_presorted(const RowCtx& C, RowLds& 
   int32_t* order = (int32_t*)L.tx0;
   int32_t* entry = (int32_t*)L.tx1;
   for (int i = lane; i < ne; i += kWave) {
-    Entry e;
-    int32_t w;
-    if (S.inReg) {
-      e = S.e;
-      w = S.w;
-    } else {
-      const int k = L.A[i];
-      e = C.E[k];
-      w = C.EW[k];
-    }
+    const int k = L.A[i];
+    const Entry e = C.E[k];
     const float yc = yMid < e.aty ? e.aty : (yMid > e.toy ? e.toy : yMid);
     L.keys[i] = ((uint64_t)float_key(solve_x(e.m, e.b, yc)) << 32) | (uint32_t)i;
-    L.B[i] = w;
+    L.B[i] = C.EW[k];
   }
   wave_sync();
-  if (ne > 1) wave_sort_keys(L.keys, ne, L.cap);
+  wave_sort_keys(L.keys, ne, L.cap);
   for (int j = lane; j < ne; j += kWave) {
     const int s = (int)(uint32_t)L.keys[j];
     order[j] = (s << 8) | (int32_t)(uint8_t)L.B[s];
-    if (!S.inReg) entry[j] = L.A[s];
+    entry[j] = L.A[s];
   }
   wave_sync();
-  // a selection held in registers moves to its presorted lanes
-  Entry er = S.e;
-  int32_t sr = 0;
-  if (S.inReg) {
-    sr = lane < ne ? order[lane] : 0;
-    const int src = sr >> 8;
-    er.aty = __shfl(S.e.aty, src, kWave);
-    er.toy = __shfl(S.e.toy, src, kWave);
-    er.m = __shfl(S.e.m, src, kWave);
-    er.b = __shfl(S.e.b, src, kWave);
-  }
+#pragma unroll 1
   for (int m = 0; m < 5; m++) {
     yLine += offset;
     int nh = 0;
@@ -633,17 +808,10 @@ __device__ __forceinline__ void row_coverage_presorted(const RowCtx& C, RowLds& 
       bool hit = false;
       int32_t at = 0, s = 0;
       if (j < ne) {
-        Entry e;
-        if (S.inReg) {
-          e = er;
-          s = sr;
-        } else {
-          e = C.E[entry[j]];
-          s = order[j];
-        }
+        const Entry e = C.E[entry[j]];
+        s = order[j];
         if (e.aty <= yLine && e.toy >= yLine) {
-          const float x = e.m == 0.0f ? e.b : (yLine - e.b) / e.m;
-          at = fixed32(nim_minf(x, Wf));
+          at = hit_at(e, yLine, Wf);
           hit = true;
         }
       }
@@ -653,97 +821,68 @@ __device__ __forceinline__ void row_coverage_presorted(const RowCtx& C, RowLds& 
       nh += __popcll(mk);
     }
     wave_sync();
-    if (nh <= kWave) {
-      // the hits fit the wave: finish the sort and walk in registers
-      uint64_t k = lane < nh ? L.keys[lane] : ~0ull;  // padding sorts last
-      bool done = false;
-      for (int t = 0; t < kFixPasses; t++) {
-        bool sw = wave_transpose(k, false);
-        sw = wave_transpose(k, true) || sw;
-        if (ballot(sw) == 0) {
-          done = true;
-          break;
-        }
-      }
-      if (!done) {
-        wave_sync();
-        if (lane < nh) L.keys[lane] = k;
-        wave_sync();
-        wave_sort_keys(L.keys, nh, L.cap);
-        k = lane < nh ? L.keys[lane] : ~0ull;
-      }
-      wave_walk_reg(k, nh, rule, span);
-    } else {
-      wave_fix_keys(L.keys, nh, L.cap);
-      wave_walk<true>(L, nh, rule, span);
-    }
+    wave_fix_keys(L.keys, nh, L.cap);
+    wave_walk<true>(L, nh, rule, span);
     wave_sync();
   }
 }
 
-// Bitonic sort of the 64 * NS keys held in slots k[0..NS) (key s * 64 + lane
-// in slot s of that lane).  Compare-exchanges at strides below 64 move keys
-// between lanes; strides of 64 and more pair two slots of the same lane.
-constexpr int kWideSlots = 4;
-template <int SS>
-__device__ __forceinline__ void slots_exchange(uint64_t (&k)[kWideSlots], int size) {
-#pragma unroll
-  for (int s = 0; s < kWideSlots; s++) {
-    if (s & SS) continue;
-    const bool up = ((s * kWave) & size) == 0;
-    const uint64_t a = k[s], b = k[s | SS];
-    const uint64_t mn = a < b ? a : b, mx = a < b ? b : a;
-    k[s] = up ? mn : mx;
-    k[s | SS] = up ? mx : mn;
-  }
-}
+// Sorts n <= 64 * NS staged keys in NS register slots.
 template <int NS>
-__device__ __forceinline__ void slots_sort(uint64_t (&k)[kWideSlots]) {
+__device__ __forceinline__ void sort32_staged(uint32_t* stage, int n) {
   const int lane = lane_id();
+  uint32_t k[NS];
 #pragma unroll
-  for (int size = 2; size <= kWave * NS; size <<= 1) {
+  for (int s = 0; s < NS; s++) k[s] = s * kWave + lane < n ? stage[s * kWave + lane] : ~0u;  // padding sorts last
+  wave_sort32<NS>(k);
 #pragma unroll
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      if (stride >= 2 * kWave) {
-        slots_exchange<2>(k, size);
-      } else if (stride >= kWave) {
-        slots_exchange<1>(k, size);
-      } else {
-        const bool lower = (lane & stride) == 0;
-#pragma unroll
-        for (int s = 0; s < NS; s++) {
-          const uint64_t o = __shfl_xor(k[s], stride, kWave);
-          const bool up = (((s * kWave) | lane) & size) == 0;
-          const uint64_t mn = k[s] < o ? k[s] : o, mx = k[s] < o ? o : k[s];
-          k[s] = lower == up ? mn : mx;
-        }
-      }
-    }
+  for (int s = 0; s < NS; s++)
+    if (s * kWave + lane < n) stage[s * kWave + lane] = k[s];
+}
+
+// Sorts and walks n staged keys, any n.  One copy of the walk serves every
+// size: the sorted keys go back to the stage.
+template <int IB>
+__device__ __forceinline__ void walk32_staged(uint32_t* stage, int n, int32_t rule, int32_t* D, int32_t lo,
+                                              int32_t hi, Walk32& c) {
+  if (n > 4 * kWave)
+    wave_sort32_mem(stage, n);
+  else if (n > 2 * kWave)
+    sort32_staged<4>(stage, n);
+  else if (n > kWave)
+    sort32_staged<2>(stage, n);
+  else
+    sort32_staged<1>(stage, n);
+  wave_sync();
+#pragma unroll 1
+  for (int base = 0; base < n; base += kWave) {
+    const int i = base + lane_id();
+    const uint32_t k = i < n ? stage[i] : ~0u, kn = i < n - 1 ? stage[i + 1] : ~0u;
+    walk32<IB, kWave>(k, kn, i < n, i < n - 1, rule, D, lo, hi, c);
   }
 }
 
-// The 5-sample coverage of an anti-aliased row that selects 65 to
-// kWideMax entries (computeCoverage 1350-1431 with walk 1298-1334), with no
-// per-row arrays in memory.  A selection of at most 256 entries is held in
-// registers (selection j in slot j / 64 of lane j % 64); a larger one is
-// read from the band for every sample line (C.E / C.EW start at the band,
-// count entries; a hit implies the selection test, which is repeated so
-// that the two agree at any y).  Either way each line's hits are compacted
-// in selection order, their keys (x, hit position << 8 | winding) staged in
-// L.wide, and sorted, which gives pixie's stable insertion order: up to 256
-// hits in four 64-key register slots, walked slot by slot with the walk's
-// carries; more in the stage itself (LDS), whose kWideMax keys hold the
-// sort's padding.  The selection indices are in L.A when ne <= L.cap.
+// The 5-sample coverage of an anti-aliased row that selects 65 to kWideMax
+// entries (computeCoverage 1350-1431 with walk 1298-1334).  A selection of at
+// most 256 is held in registers (selection j in slot j / 64 of lane j % 64);
+// a larger one is read from the band for every sample line (C.E / C.EW start
+// at the band, count entries; a hit implies the selection test, which is
+// repeated so that the two agree at any y).  Each line's hits inside the
+// window are compacted in selection order into L.stage (LDS) as 32-bit keys,
+// sorted in register slots and walked.  Returns the lines to be walked
+// whole, as row_coverage_seg does.
+constexpr int kWideSlots = 4;
 constexpr int kWideMax = 8 * kWave;
-__device__ __forceinline__ int wide_limit(const RowLds& L) {
-  return L.wideCap >= kWideMax ? kWideMax : (L.wideCap < kWideSlots * kWave ? L.wideCap : kWideSlots * kWave);
+__device__ __forceinline__ bool wide_fits(const RowLds& L, int ne, int count) {
+  return ne <= L.stageCap && (ne <= kWideSlots * kWave || (ne <= kWideMax && count <= 1 << (kKeyBits - 1)));
 }
-__device__ __forceinline__ void row_coverage_wide(const RowCtx& C, RowLds& L, int count, int ne, float scanTop,
-                                                  float scanBottom, float yLine, float offset, int32_t rule,
-                                                  CovSpan& span) {
+__device__ __forceinline__ uint32_t row_coverage_wide(const RowCtx& C, RowLds& L, int count, int ne, float scanTop,
+                                                      float scanBottom, float yLine, float offset, int32_t rule) {
   const int lane = lane_id();
   const float Wf = (float)C.F->canvasW;
-  uint64_t* stage = L.wide;
+  const Win32 win = window32(C);
+  uint32_t* stage = L.stage;
+  uint32_t whole = 0;
   const bool inReg = ne <= kWideSlots * kWave;
   Entry e[kWideSlots];
   int32_t w[kWideSlots];
@@ -751,117 +890,60 @@ __device__ __forceinline__ void row_coverage_wide(const RowCtx& C, RowLds& L, in
   for (int s = 0; s < kWideSlots; s++) {
     e[s] = Entry{0.0f, 0.0f, 0.0f, 0.0f};
     w[s] = 0;
-  }
-  if (inReg) {
-    const int32_t* selIdx = L.A;
-    if (ne > L.cap) {  // select again, into the stage
-      int32_t* idx = (int32_t*)stage;
-      int n = 0;
-      for (int base = 0; base < count; base += kWave) {
-        const int i = base + lane;
-        bool sel = false;
-        if (i < count) {
-          const Entry ei = C.E[i];
-          sel = !(ei.toy <= scanTop || ei.aty >= scanBottom);
-        }
-        const uint64_t m = ballot(sel);
-        if (sel) idx[n + __popcll(m & ((1ull << lane) - 1ull))] = i;
-        n += __popcll(m);
-      }
-      wave_sync();
-      selIdx = idx;
+    const int j = s * kWave + lane;
+    if (inReg && j < ne) {
+      const int k = L.A[j];
+      e[s] = C.E[k];
+      w[s] = C.EW[k];
     }
-#pragma unroll
-    for (int s = 0; s < kWideSlots; s++) {
-      const int j = s * kWave + lane;
-      if (j < ne) {
-        const int k = selIdx[j];
-        e[s] = C.E[k];
-        w[s] = C.EW[k];
-      }
-    }
-    wave_sync();  // the stage now takes the hit keys
   }
+#pragma unroll 1
   for (int m = 0; m < 5; m++) {
     yLine += offset;
-    int nh = 0;
+    int n = 0, left = 0, total = 0, in = 0;  // keys, and winding sums
+    auto put = [&](const Entry& ei, int32_t wi, bool sel, int order) {
+      const bool hit = sel && ei.aty <= yLine && ei.toy >= yLine;
+      const int32_t at = hit_at(ei, yLine, Wf);
+      const bool isLeft = hit && at < win.A1, inW = hit && !isLeft && at < win.B;
+      const uint64_t up = ballot(hit && wi > 0), down = ballot(hit && wi <= 0), lm = ballot(isLeft), im = ballot(inW);
+      total += __popcll(up) - __popcll(down);
+      left += __popcll(lm & up) - __popcll(lm & down);
+      in += __popcll(im & up) - __popcll(im & down);
+      if (inW)
+        stage[n + seg_rank<kWave>(im)] =
+            ((uint32_t)(at - win.A) << kKeyBits) | ((uint32_t)order << 1) | (wi > 0 ? 1u : 0u);
+      n += __popcll(im);
+    };
     if (inReg) {
 #pragma unroll
-      for (int s = 0; s < kWideSlots; s++) {
-        bool hit = false;
-        int32_t at = 0;
-        if (s * kWave + lane < ne && e[s].aty <= yLine && e[s].toy >= yLine) {
-          const float x = e[s].m == 0.0f ? e[s].b : (yLine - e[s].b) / e[s].m;
-          at = fixed32(nim_minf(x, Wf));
-          hit = true;
-        }
-        const uint64_t mk = ballot(hit);
-        const int pos = nh + __popcll(mk & ((1ull << lane) - 1ull));
-        if (hit)
-          stage[pos] = ((uint64_t)((uint32_t)at ^ 0x80000000u) << 32) | ((uint32_t)pos << 8) |
-                       (uint32_t)(uint8_t)w[s];
-        nh += __popcll(mk);
-      }
+      for (int s = 0; s < kWideSlots; s++)
+        if (s * kWave < ne) put(e[s], w[s], s * kWave + lane < ne, s * kWave + lane);
     } else {
 #pragma unroll 2
       for (int base = 0; base < count; base += kWave) {
         const int i = base + lane;
-        bool hit = false;
-        int32_t at = 0, wi = 0;
+        Entry ei = {0.0f, 0.0f, 0.0f, 0.0f};
+        int32_t wi = 0;
         if (i < count) {
-          const Entry ei = C.E[i];
-          if (!(ei.toy <= scanTop || ei.aty >= scanBottom) && ei.aty <= yLine && ei.toy >= yLine) {
-            const float x = ei.m == 0.0f ? ei.b : (yLine - ei.b) / ei.m;
-            at = fixed32(nim_minf(x, Wf));
-            wi = C.EW[i];
-            hit = true;
-          }
+          ei = C.E[i];
+          wi = C.EW[i];
         }
-        const uint64_t mk = ballot(hit);
-        const int pos = nh + __popcll(mk & ((1ull << lane) - 1ull));
-        if (hit)
-          stage[pos] = ((uint64_t)((uint32_t)at ^ 0x80000000u) << 32) | ((uint32_t)pos << 8) |
-                       (uint32_t)(uint8_t)wi;
-        nh += __popcll(mk);
+        put(ei, wi, i < count && !(ei.toy <= scanTop || ei.aty >= scanBottom), i);
       }
     }
     wave_sync();
-    if (nh > kWideSlots * kWave) {
-      RowLds Ls = L;
-      Ls.keys = stage;
-      wave_sort_keys(stage, nh, kWideMax);
-      wave_walk<true>(Ls, nh, rule, span);
-      wave_sync();
-      continue;
-    }
-    uint64_t k[kWideSlots];
-#pragma unroll
-    for (int s = 0; s < kWideSlots; s++) {
-      const int j = s * kWave + lane;
-      k[s] = j < nh ? stage[j] : ~0ull;  // padding sorts last
-    }
-    if (nh <= kWave)
-      slots_sort<1>(k);
-    else if (nh <= 2 * kWave)
-      slots_sort<2>(k);
-    else
-      slots_sort<4>(k);
-    WalkCarry c;
-#pragma unroll
-    for (int s = 0; s < kWideSlots; s++) {
-      if (s * kWave >= nh) break;
-      const int j = s * kWave + lane;
-      const bool valid = j < nh, hasNext = j < nh - 1;
-      uint64_t kn = __shfl(k[s], lane + 1 < kWave ? lane + 1 : lane, kWave);
-      if (s + 1 < kWideSlots) {
-        const uint64_t first = __shfl(k[s + 1], 0, kWave);
-        if (lane == kWave - 1) kn = first;
-      }
-      walk_chunk(valid ? key_at(k[s]) : 0, valid ? key_winding(k[s]) : 0, valid, hasNext,
-                 hasNext ? key_at(kn) : 0, hasNext ? key_winding(kn) : 0, rule, c, span);
+    if (total != 0) {
+      whole |= 1u << m;
+    } else if (win.lo < win.hi) {
+      Walk32 c;
+      c.count = left;
+      walk32_staged<kKeyBits>(stage, n, rule, L.D, win.lo, win.hi, c);
+      if (lane == 0)
+        walk32_borders(should_fill(rule, left), should_fill(rule, left + in), L.D, win.lo, win.hi);
     }
     wave_sync();
   }
+  return whole;
 }
 
 // Entries row C.y selects (row_program's selection), so that a caller can
@@ -961,22 +1043,10 @@ __device__ int32_t row_program(const RowCtx& C, RowLds& L) {
     }
   }
   wave_sync();
-  // An anti-aliased row of more than 64 selected entries that is not a
-  // trapezoid candidate takes the wide path when its selection fits it.
-  const bool wide = aa && !two && !(allSpan && (ne % 2) == 0) && ne > kWave && ne <= wide_limit(L);
   // the row's arrays hold the selection (not the whole band); D is untouched
   // so far, so a selection too large for them leaves nothing behind
-  if (!wide && ne > L.cap) return -1;
+  if (ne > L.cap) return -1;
   if (mask && lane == 0) add_run(C, L, 0, W, kClear);  // default for mask rows
-  if (wide) {  // computeCoverage 1350-1431 at quality 5
-    const float offset = 1.0f / 5.0f;
-    const float yLine = (float)y + (offset / 2.0f + 0.00031415926535897936f) - offset;
-    const int64_t covLo = F.startX, covHi = (int64_t)F.startX + F.pathWidth;
-    if (mask && lane == 0) add_run(C, L, covLo, covHi, -kClear);  // coverage range
-    CovSpan cs{&C, &L, 255 / 5, (int32_t)covLo, (int32_t)covHi};
-    row_coverage_wide(Cp, L, P.count, ne, scanTop, scanBottom, yLine, offset, F.rule, cs);
-    return kRowCoverage;
-  }
   const bool inReg = ne <= kWave;
   float sAty = 0.0f, sToy = 0.0f, sM = 0.0f, sB = 0.0f;
   int32_t sW = 0;
@@ -1116,23 +1186,35 @@ __device__ int32_t row_program(const RowCtx& C, RowLds& L) {
 
   // computeCoverage 1350-1431 / fillHits 1898
   const int quality = aa ? 5 : 1;
-  const int32_t sampleCoverage = 255 / quality;
   const float offset = 1.0f / (float)quality;
   const float initialOffset = offset / 2.0f + 0.00031415926535897936f;
   float yLine = (float)y + initialOffset - offset;
   const int64_t covLo = F.startX, covHi = (int64_t)F.startX + F.pathWidth;
   if (aa) {
     if (mask && lane == 0) add_run(C, L, covLo, covHi, -kClear);  // coverage range
-    CovSpan cs{&C, &L, sampleCoverage, (int32_t)covLo, (int32_t)covHi};
-    // (two sample lines per pass for selections of 17-32 entries measured
-    // slower than the five single passes, so only 16-entry rows take it)
-    if (S.inReg && ne <= 16 && L.cap >= kWave) {
-      const float y0 = yLine + offset, y1 = y0 + offset, y2 = y1 + offset, y3 = y2 + offset,
-                  y4 = y3 + offset;
-      row_coverage_small<16>(Cp, L, ne, S, y0, y1, y2, y3, y4, F.rule, cs);
-      return kRowCoverage;
+    CovSpan cs{&C, &L, kSampleCov, (int32_t)covLo, (int32_t)covHi};
+    uint32_t whole;
+    if (ne <= 8) {
+      whole = row_coverage_seg<8>(Cp, L, ne, S, yLine, offset, F.rule);
+    } else if (ne <= 16) {
+      whole = row_coverage_seg<16>(Cp, L, ne, S, yLine, offset, F.rule);
+    } else if (ne <= 32) {
+      whole = row_coverage_seg<32>(Cp, L, ne, S, yLine, offset, F.rule);
+    } else if (ne <= kWave) {
+      whole = row_coverage_seg<64>(Cp, L, ne, S, yLine, offset, F.rule);
+    } else if (wide_fits(L, ne, P.count)) {
+      whole = row_coverage_wide(Cp, L, P.count, ne, scanTop, scanBottom, yLine, offset, F.rule);
+    } else {
+      whole = 0;
+      row_coverage_presorted(Cp, L, ne, yLine, offset, F.rule, cs);
     }
-    row_coverage_presorted(Cp, L, ne, S, yLine, offset, F.rule, cs);
+    for (int m = 0; whole != 0; m++, whole >>= 1) {
+      yLine += offset;
+      if (whole & 1u) {  // pixie's walk of the whole line
+        wave_walk(L, row_hits(Cp, L, ne, yLine, S), F.rule, cs);
+        wave_sync();
+      }
+    }
     return kRowCoverage;
   }
   yLine += offset;

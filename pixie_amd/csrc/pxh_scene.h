@@ -121,8 +121,9 @@ enum SceneCounter {
   kCntRuns,      // run-pool entries handed out in chunks
   kCntRunsUsed,  // run entries written
   kCntError, kCntMaxBand, kCntBinEntries,
-  kCntBigTasks,  // phase-A work items of the large-band launch (the first in their order)
+  kCntHeavy,     // phase-A work items of the heavy kernel (the first in their order)
   kCntGroups,    // phase-A work items (set by the class scan)
+  kCntLeft,      // rows the heavy kernel leaves to the rows kernel
   kNumCounters
 };
 
@@ -155,7 +156,7 @@ constexpr int kBinRows = 16;
 // every fetch.
 constexpr int kQueues = 16;
 constexpr int kQueueStride = 64;  // ints between queue heads (256 B)
-// Queue sets: phase A's large-band launch, its small-band launch, phase B.
+// Queue sets: phase A's heavy rows, its other rows, phase B.
 constexpr int kQueueSets = 3;
 
 // Grid of a queue-fed kernel: at least one wave per queue, a multiple of
@@ -213,7 +214,8 @@ struct ScenePools {
   int32_t entryCap;
   RowRuns* tasks;
   int32_t* taskItem;         // call of each work item
-  int32_t* taskOrder;        // work items in the order phase A takes them (longest first)
+  int32_t* taskOrder;        // work items in the order phase A takes them (longest first),
+                             // then from taskCap on the rows the heavy kernel leaves
   int8_t* taskClass;         // cost class of each work item
   int32_t taskCap;
   int2* runs;
@@ -232,51 +234,36 @@ struct ScenePools {
   char* gscratch;
   int32_t gcap;              // entries per wave slot
   int32_t ldsCap;            // entries that fit in LDS
-  int32_t bigClass;          // first cost class of the large-band launch
+  int32_t heavyClass;        // first cost class of the heavy kernel's rows
 };
 
-// Phase-A launch shapes.  The row program is latency-bound, so each launch
-// keeps about as many waves resident as LDS and registers allow for the
-// band entries its waves keep in LDS.
-//   kRowsSingle      one launch of every task: ldsCap entries in LDS, larger
-//                    selections in the global row scratch
-//   kRowsConcurrent  tasks whose band holds more than ldsCap entries (their
-//                    cost class is above it; they come first in the task
-//                    order) run in a second launch of bigWaves waves per CU
-//                    with bigCap entries in LDS, beside the first launch
-//   kRowsSequential  the same two launches, one after the other
-// Only waves whose tasks may exceed their LDS capacity get global row
-// scratch slots.  A scene's autotuner picks one shape; run-pool sizing
-// assumes the most waves any shape has.
-enum RowMode { kRowsSingle = 0, kRowsConcurrent = 1, kRowsSequential = 2 };
+// Phase-A launch shapes: the band entries the rows kernel's waves keep in LDS
+// (larger selections in the global row scratch), its waves per CU, and the
+// first cost class of the heavy kernel.  16 waves per CU are what 128 VGPRs
+// allow; 20 waves of 96 spilled 39 of them and ran no faster (scene of 2,000
+// paths on 4096 x 4096 1,742 and 1,749 us, paragraph of 820 glyphs 576 and
+// 541 us).  A scene's autotuner picks one;
+// run-pool sizing assumes the most waves any shape has.
+constexpr int kHeavyWins = 2;          // windows of a heavy row's work item
+constexpr int kHeavyWavesPerGroup = 4;  // waves of a heavy kernel workgroup
+constexpr int kHeavyGroupsPerCU = 5;
 struct RowShape {
-  int ldsCap, wavesPerCU;
-  int mode;
-  int bigCap, bigWaves;
+  int ldsCap, wavesPerCU, heavyClass;
 };
 constexpr RowShape kRowShapes[] = {
-    {128, 20, kRowsSingle, 0, 0},
-    {128, 20, kRowsConcurrent, 512, 6},
-    {128, 20, kRowsSequential, 512, 9},
-    {128, 16, kRowsConcurrent, 256, 10},
-    {64, 24, kRowsSingle, 0, 0},
-    {256, 14, kRowsSingle, 0, 0},
+    {128, 16, 10}, {128, 16, 9}, {128, 16, 11}, {64, 16, 10}, {256, 14, 10}, {128, 12, 10},
 };
 constexpr int kNumRowShapes = 6;
 constexpr int kDefaultRowShape = 0;
-// Waves of a shape's phase-A launches together, and the most of any shape.
-inline int scene_shape_waves(const RowShape& s, int numCUs) {
-  return scene_queue_grid(numCUs * s.wavesPerCU) + (s.mode ? scene_queue_grid(numCUs * s.bigWaves) : 0);
-}
+// Waves of phase A that take run chunks: the heavy kernel's and the rows
+// kernel's of the shape with the most.
 inline int scene_row_waves(int numCUs) {
   int m = 0;
-  for (const RowShape& s : kRowShapes) m = m > scene_shape_waves(s, numCUs) ? m : scene_shape_waves(s, numCUs);
-  return m;
+  for (const RowShape& s : kRowShapes) m = m > s.wavesPerCU ? m : s.wavesPerCU;
+  return scene_queue_grid(numCUs * m) + kHeavyWavesPerGroup * scene_queue_grid(numCUs * kHeavyGroupsPerCU);
 }
 // Wave slots of global row scratch a shape uses.
-inline int scene_scratch_slots(const RowShape& s, int numCUs) {
-  return s.mode ? scene_queue_grid(numCUs * s.bigWaves) : scene_queue_grid(numCUs * s.wavesPerCU);
-}
+inline int scene_scratch_slots(const RowShape& s, int numCUs) { return scene_queue_grid(numCUs * s.wavesPerCU); }
 
 int scene_set_lds_limits(size_t bytes);
 size_t scene_gscratch_bytes(int rowGrid, int gcap);  // global row scratch of scene_launch_rows
@@ -286,10 +273,8 @@ int scene_launch_clear(const ScenePools& p, hipStream_t s);
 int scene_launch_geometry(const ScenePools& p, hipStream_t s);
 int scene_launch_bands(const ScenePools& p, int grid, hipStream_t s);
 int scene_launch_bins(const ScenePools& p, int grid, hipStream_t s);
-// Phase A in the given shape; a concurrent shape forks its small-band
-// launch onto aux (fork / join through the two events).
-int scene_launch_rows(const ScenePools& p, const RowShape& shape, int numCUs, hipStream_t s,
-                      hipStream_t aux, hipEvent_t fork, hipEvent_t join);
+// Phase A in the given shape: the heavy rows, then the others.
+int scene_launch_rows(const ScenePools& p, const RowShape& shape, int numCUs, hipStream_t s);
 int scene_launch_compose(const ScenePools& p, void* canvas, bool a8, unsigned long long* touched,
                          int32_t* errOut, int grid, hipStream_t s);
 

@@ -1678,10 +1678,21 @@ __device__ __forceinline__ int band_of_row(const FillInfo& F, int y) {
   const int pi = (y - F.startY) / F.bandH;
   return pi > F.nParts - 1 ? F.nParts - 1 : pi;
 }
-// Cost class of band pi of a call: the bit length of its entry count.
-__device__ __forceinline__ int band_class(const ScenePools& P, const ItemGeom& g, int pi) {
-  const int cnt = P.parts[g.bandBase + pi].count;
-  return cnt <= 0 ? 0 : 32 - __clz(cnt);
+// First cost class of the heavy kernel: one later for a scene of many tasks,
+// whose other rows keep the chip busy beside a row that takes one wave long
+// (the heavy kernel runs more instructions per row: its benefit is latency).
+// 1,023 x 767 with 100 paths (13 k tasks): 694 us from class 10, 928 from 11;
+// 4096 x 4096 with 2,000 paths (291 k): 1,849 and 1,741 us.
+constexpr int kManyTasks = 1 << 16;
+__device__ __forceinline__ int heavy_class(const ScenePools& P) {
+  return P.heavyClass + (P.counters[kCntTasks] > kManyTasks ? 1 : 0);
+}
+// Cost class of band pi of a call: the bit length of its entry count (below
+// the heavy classes when the band needs no anti-aliasing).
+__device__ __forceinline__ int band_class(const ScenePools& P, const ItemGeom& g, int pi, int heavyClass) {
+  const PartInfo p = P.parts[g.bandBase + pi];
+  const int c = p.count <= 0 ? 0 : 32 - __clz(p.count);
+  return (p.flags & 1) || c < heavyClass ? c : heavyClass - 1;
 }
 
 // Maps work items to calls and records their cost classes, counting them
@@ -1694,6 +1705,7 @@ __global__ void __launch_bounds__(kTaskMapBlock) scene_task_map_kernel(ScenePool
   __shared__ int8_t cls[kLdsBandClasses];
   const int tid = threadIdx.x, lane = tid & 63;
   if (P.counters[kCntError]) return;
+  const int heavyClass = heavy_class(P);
   if (tid < kCostClasses) hist[tid] = 0;
   __syncthreads();
   for (int it = blockIdx.x; it < P.nItems; it += gridDim.x) {
@@ -1704,8 +1716,7 @@ __global__ void __launch_bounds__(kTaskMapBlock) scene_task_map_kernel(ScenePool
     const bool banded = F.nParts > 0 && F.bandH > 0;
     const int nb = banded ? F.nParts : 0;
     for (int b = tid; b < nb && b < kLdsBandClasses; b += kTaskMapBlock) {
-      const int cnt = P.parts[g.bandBase + b].count;
-      cls[b] = (int8_t)(cnt <= 0 ? 0 : 32 - __clz(cnt));
+      cls[b] = (int8_t)band_class(P, g, b, heavyClass);
     }
     __syncthreads();
     for (int t0 = 0; t0 < nt; t0 += kTaskMapBlock) {
@@ -1724,13 +1735,15 @@ __global__ void __launch_bounds__(kTaskMapBlock) scene_task_map_kernel(ScenePool
           const int pr = band_of_row(F, g.rowStart + r), p0 = band_of_row(F, g.rowStart + rg),
                     p1 = band_of_row(F, g.rowStart + re);
           for (int pi = p0; pi <= p1; pi++) {
-            const int rc = pi < kLdsBandClasses ? cls[pi] : band_class(P, g, pi);
+            const int rc = pi < kLdsBandClasses ? cls[pi] : band_class(P, g, pi, heavyClass);
             if (pi == pr) own = rc;
             chunk = rc > chunk ? rc : chunk;
           }
         }
         grouped = chunk <= kGroupMaxClass;
-        c = !grouped ? own : (r == rg ? chunk : -1);
+        // a heavy row's item takes kHeavyWins windows at a time
+        if (own >= heavyClass) c = (t % g.nWin) % kHeavyWins == 0 ? own : -1;
+        else c = !grouped ? own : (r == rg ? chunk : -1);
         P.taskItem[g.taskBase + t] = grouped ? (int32_t)((uint32_t)it | 0x80000000u) : it;
         P.taskClass[g.taskBase + t] = (int8_t)c;
       }
@@ -1758,16 +1771,17 @@ __device__ __forceinline__ int2 task_share(int ntasks) {
 }
 
 // Start of each cost class in the work-item order, largest class first, and
-// the number of items in classes >= bigClass (the large-band launch's share).
-__global__ void scene_task_scan_kernel(int32_t* counters, int bigClass) {
+// the number of items in the heavy classes.
+__global__ void scene_task_scan_kernel(ScenePools P) {
   if (threadIdx.x != 0) return;
+  int32_t* const counters = P.counters;
+  const int heavyClass = heavy_class(P);
   int off = 0;
   for (int c = kCostClasses - 1; c >= 0; c--) {
-    if (c == bigClass - 1) counters[kCntBigTasks] = off;
+    if (c == heavyClass - 1) counters[kCntHeavy] = off;
     counters[kCntClassCursor + c] = off;
     off += counters[kCntClassHist + c];
   }
-  if (bigClass <= 0) counters[kCntBigTasks] = off;
   counters[kCntGroups] = off;
 }
 
@@ -1790,35 +1804,434 @@ __global__ void __launch_bounds__(64) scene_task_order_kernel(ScenePools P) {
     if (P.taskClass[t] >= 0) P.taskOrder[atomicAdd(&cur[P.taskClass[t]], 1)] = t;
 }
 
-// kBig: the large-band launch (tasks [0, nBig) of the task order), else the
-// small-band one; two instantiations so that profiles tell them apart.
-template <bool kBig>
-__global__ void __launch_bounds__(64, 5) scene_rows_kernel(ScenePools P) {
+// A wave's place in the run pool: it appends its runs to chunks it takes one
+// at a time (one atomic per chunk, not per task).
+struct RunCursor {
+  int at = 0, end = 0, used = 0;
+};
+
+// Writes a window's codes D[0..wlen] as runs -- the nonzero deltas and, for
+// ops rows, the area factors of the pixels whose code is an area code -- in
+// one pass, and clears D.  The wave's run chunk is first made to hold the
+// most the row can write (wlen + 1 deltas, and wlen area factors on ops
+// rows).  D has kWinA + 4 entries and is zero beyond wlen, so a lane with
+// i0 <= wlen moves its 4 entries as one 16-byte access.  Returns the number
+// of runs and their place in *off.
+__device__ __forceinline__ int emit_runs(const ScenePools& P, int32_t* D, const uint32_t* AX, int wx0, int wlen,
+                                         bool ops, RunCursor* rc, int* off) {
+  const int lane = threadIdx.x & 63;
+  wave_sync();
+  const int most = ops ? 2 * wlen + 1 : wlen + 1;
+  if (rc->at + most > rc->end) {
+    rc->at = queue_take(&P.counters[kCntRuns], kRunChunk);
+    rc->end = rc->at + kRunChunk;
+  }
+  *off = rc->at;
+  if (rc->end > P.runCap) {
+    atomicOr(&P.counters[kCntError], 16);
+    for (int i = lane; i <= wlen; i += 64) D[i] = 0;
+    wave_sync();
+    return 0;
+  }
+  int carry = 0, written = 0;
+  for (int base = 0; base <= wlen; base += 4 * kWave) {
+    const int i0 = base + 4 * lane;
+    int4 dv = make_int4(0, 0, 0, 0);
+    if (i0 <= wlen) dv = *(const int4*)(D + i0);
+    const int32_t d[4] = {dv.x, dv.y, dv.z, dv.w};
+    bool area[4] = {false, false, false, false};
+    if (ops) {
+      const int32_t c0 = d[0], c1 = c0 + d[1], c2 = c1 + d[2], c3 = c2 + d[3];
+      int32_t tot;
+      const int32_t ofs = carry + wave_excl_scan(c3, &tot);
+      carry += tot;
+      const int32_t code[4] = {ofs + c0, ofs + c1, ofs + c2, ofs + c3};
+#pragma unroll
+      for (int q = 0; q < 4; q++) area[q] = i0 + q < wlen && code[q] >= kArea && code[q] < kClear;
+    }
+    int n = 0;
+#pragma unroll
+    for (int q = 0; q < 4; q++) n += (d[q] != 0 ? 1 : 0) + (area[q] ? 1 : 0);
+    int ntot;
+    const int p = wave_excl_scan(n, &ntot);
+    if (i0 <= wlen) {
+      int2* out = P.runs + *off + written + p;
+      int w = 0;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int x = wx0 + i0 + q;
+        if (d[q] != 0) out[w++] = make_int2(x, d[q]);
+        if (area[q]) out[w++] = make_int2(x | kRunArea, (int32_t)AX[i0 + q]);
+      }
+      *(int4*)(D + i0) = make_int4(0, 0, 0, 0);
+    }
+    written += ntot;
+  }
+  rc->at += written;
+  rc->used += written;
+  wave_sync();
+  return written;
+}
+
+// ---------------------------------------------------------------------------
+// heavy rows: one workgroup per (call, row, kHeavyWins windows)
+// ---------------------------------------------------------------------------
+// A row of a band of hundreds of entries (a line of text, a stroke with round
+// joins) is a long serial chain for one wave, and each of its windows would
+// scan the band and sort every hit of the row again.  Here the waves of a
+// workgroup share the row: they scan its band once for kHeavyWins windows,
+// keep the places of the entries that can meet those windows in LDS, deal the hits of all
+// five sample lines into buckets of 4 to 64 pixels, and each wave sorts and
+// walks whole buckets.
+//
+// Walking a bucket [A, B) by itself gives the pixels of pixie's walk over the
+// whole line (paths.nim:1298-1330): skipped pairs and equal-x groups share
+// one x, so they lie in one bucket; a span that crosses a bucket border
+// covers the pixels on both sides as the two spans cut at the border do (the
+// border is a whole pixel); before the bucket's first hit only the winding
+// count matters, which is the sum over the hits left of A; and a span open at
+// B ends at some later hit whenever the windings of the whole line sum to 0
+// (the count then returns to 0 at a hit that is not skipped).  A row with a
+// line whose windings do not sum to 0 (a sample line through a vertex, where
+// float32 leaves no room between them) or with more hits than the key space
+// is left to the rows kernel, as is a trapezoid candidate.
+//
+// An entry's hit position is monotone in y (every float operation of it is),
+// so the positions on the first and the last sample line tell whether it can
+// meet the windows at all; entries left of them only add to the counts.
+//
+// Keys are 32 bits: x inside the bucket in 24.8 (14 bits), the entry's place
+// in the band (17 bits: pixie's stable order), the winding's sign.
+//
+// Measured (kernel trace): a 4096-px page of 33,000 glyphs, rows kernel alone
+// 2,888 us, heavy rows 139 us + rows kernel 48 us; 100 paths on 1,023 x 767,
+// 647 us and 45 us + 140 us.  An item takes 70 thousand cycles when the chip
+// is not full (scan 16, deal 14, buckets 24, runs 9), bound by the latency of
+// the loads and of the short dependent chains between its barriers.
+constexpr int kHeavyThreads = kHeavyWavesPerGroup * 64;
+constexpr int kHeavyPx = kHeavyWins * kWinA;
+constexpr int kBucketKeyBits = 18;  // order and winding below a bucket's positions
+constexpr int kHeavyBuckets = 64;  // most buckets of a line (a wave scans them)
+constexpr int kHeavyKeys = 4096;   // hits of the lines dealt together
+constexpr int kHeavySel = 1280;    // entries kept
+constexpr int kHeavyMaxBand = 65535;  // a bucket's hit count is 16 bits
+constexpr int kHeavyMaxWidth = 1 << 22;  // 24.8 positions of a row item stay below 2^31
+
+// What the workgroup needs to know of a work item.
+struct HeavyItem {
+  int32_t first;       // task of its first window; -1 ends the kernel
+  int32_t y, gx0, nw;  // row, first pixel, windows
+  PartInfo part;       // the row's band
+  int32_t mode, rule, xhi, covLo, covHi;
+};
+
+// Wave 0 reads the records of the next item while the workgroup is busy with
+// this one: each step's loads (order -> task -> call -> band) are issued a
+// phase before the next step needs them.  The items go round the workgroups
+// in their order, longest first; a shared queue would cost each item the
+// round trip of an atomic (8 to 14 thousand cycles of 70).
+struct HeavyFetch {
+  int q;  // place of the next item
+  int first, it;
+  ItemGeom g;
+  FillInfo F;
+  PartInfo part;
+  __device__ __forceinline__ void step_order(const ScenePools& P, int n) {
+    first = q < n ? P.taskOrder[q] : -1;
+  }
+  __device__ __forceinline__ void step_task(const ScenePools& P) {
+    it = first >= 0 ? P.taskItem[first] & 0x7fffffff : 0;
+  }
+  __device__ __forceinline__ void step_call(const ScenePools& P) {
+    g = P.geo[it];
+    F = P.fills[it];
+  }
+  __device__ __forceinline__ void step_band(const ScenePools& P, HeavyItem* h) {
+    h->first = first;  // every lane stores the same values
+    if (first < 0) return;
+    const int local = first - g.taskBase, win0 = local % g.nWin, y = g.rowStart + local / g.nWin;
+    part = P.parts[g.bandBase + band_of_row(F, y)];
+    h->y = y;
+    h->gx0 = g.winBase + win0 * kWinA;
+    h->nw = g.nWin - win0 < kHeavyWins ? g.nWin - win0 : kHeavyWins;
+    h->mode = F.mode;
+    h->rule = F.rule;
+    h->xhi = F.mode == kMask ? P.W : F.xhi;
+    h->covLo = F.startX;
+    h->covHi = F.startX + F.pathWidth;
+  }
+};
+
+__global__ void __launch_bounds__(kHeavyThreads, 5) scene_heavy_kernel(ScenePools P) {
+  __shared__ __align__(16) int32_t D[kHeavyWins][kWinA + 4];
+  __shared__ uint32_t sel[kHeavySel];  // kept entries: place in the band << 1 | winding is 1
+  __shared__ uint32_t keys[kHeavyKeys];
+  // per line and bucket: hits | windings << 16, then the place of the
+  // bucket's next key in its line; and the winding count left of the bucket
+  __shared__ uint32_t bkt[5][kHeavyBuckets];
+  __shared__ int32_t left0[5][kHeavyBuckets];
+  // per line: the winding sums of the hits left of the windows and of all
+  // hits, and its hits in the buckets
+  __shared__ int32_t sLeft[5], sTotal[5], sHits[5];
+  __shared__ int32_t sNe, sNotSpan, sSel;
+  __shared__ HeavyItem sItems[2];  // this item's record and the next one's
+  const int tid = threadIdx.x, lane = tid & 63, wave = uni(tid >> 6);
+  for (int i = tid; i < kHeavyWins * (kWinA + 4); i += kHeavyThreads) ((int32_t*)D)[i] = 0;
+  // read once, so that every wave takes the same way when another workgroup
+  // sets the error meanwhile
+  if (tid == 0) sNe = P.counters[kCntError];
+  __syncthreads();
+  if (uni(sNe)) return;
+  const int nHeavy = P.counters[kCntHeavy];
+  RunCursor rc;
+  HeavyFetch nx;
+  if (wave == 0) {
+    nx.q = blockIdx.x;
+    nx.step_order(P, nHeavy);
+    nx.step_task(P);
+    nx.step_call(P);
+    nx.step_band(P, &sItems[0]);
+  }
+  for (int cur = 0;; cur ^= 1) {
+    HeavyItem& sItem = sItems[cur];
+    HeavyItem* const next = &sItems[cur ^ 1];
+    __syncthreads();  // the item before is done with the shared words
+    if (wave == 0) {
+      sItem.part = nx.part;
+      if (lane == 0) sNe = sNotSpan = sSel = 0;
+      if (lane < 5) sLeft[lane] = sTotal[lane] = 0;
+      nx.q += gridDim.x;
+      nx.step_order(P, nHeavy);
+    }
+    for (int i = tid; i < 5 * kHeavyBuckets; i += kHeavyThreads) (&bkt[0][0])[i] = 0;
+    __syncthreads();
+    const int first = uni(sItem.first);
+    if (first < 0) break;
+    const int y = uni(sItem.y), nw = uni(sItem.nw), count = uni(sItem.part.count);
+    const int32_t mode = uni(sItem.mode), rule = uni(sItem.rule);
+    const bool mask = mode == kMask;
+    const Entry* E = P.entries + uni(sItem.part.entryBase);
+    const int8_t* EW = P.entW + uni(sItem.part.entryBase);
+    const float scanTop = (float)y, scanBottom = (float)(y + 1);
+    const int32_t gx0 = uni(sItem.gx0), cx1 = uni(sItem.xhi);
+    const int32_t covLo = uni(sItem.covLo), covHi = uni(sItem.covHi);
+    const int32_t A = gx0 * 256, A1 = A > 1 ? A : 1, B = (gx0 + nw * kWinA) * 256;
+    const float Wf = (float)P.W;
+    float yl[5];
+    {
+      const float offset = 1.0f / 5.0f;
+      float v = (float)y + (offset / 2.0f + 0.00031415926535897936f) - offset;
+#pragma unroll
+      for (int m = 0; m < 5; m++) yl[m] = v += offset;
+    }
+    // Buckets of a width that puts 24 to 48 hits into each, at most
+    // kHeavyBuckets of them: a row selects about half of its band's entries,
+    // half of those meet a sample line, and the windows hold their share of
+    // the path's width.
+    const int extent = covHi < gx0 + nw * kWinA ? covHi - gx0 : nw * kWinA;
+    const int est = covHi - covLo > extent ? (int)((int64_t)count * extent / (covHi - covLo)) : count;
+    int sh = 6;
+    while (sh > 2 && (extent >> (sh - 1)) < kHeavyBuckets && (est << sh) > 192 * extent) sh--;
+    const int px = 1 << sh;
+    int nb = (extent + px - 1) >> sh;
+    nb = nb < 1 ? 1 : (nb < kHeavyBuckets ? nb : kHeavyBuckets);
+    // hits at Bk or beyond lie right of the coverage range: they cover no
+    // pixel, and what they end covers the range to its border either way
+    const int32_t Bk = A + nb * (px << 8) < B ? A + nb * (px << 8) : B;
+    bool leave = !(uni(sItem.part.flags) & 1) || count > P.gcap || count > kHeavyMaxBand || P.W > kHeavyMaxWidth;
+    // Scan of the band: the row's selection (paths.nim:1673-1689) with its
+    // size and whether every entry spans the row, each line's winding sums and
+    // bucket counts, and the list of the entries that can meet the windows.
+    // kLoads entries per thread are in flight at a time.
+    constexpr int kLoads = 4;
+    int ne = 0;
+    if (!leave) {
+      bool notSpan = false;
+      int32_t left[5] = {0, 0, 0, 0, 0}, total[5] = {0, 0, 0, 0, 0};
+      auto scan = [&](const Entry& e, int32_t w, bool in) -> bool {
+        if (!in || e.toy <= scanTop || e.aty >= scanBottom) return false;
+        ne++;
+        notSpan |= e.aty > scanTop || e.toy < scanBottom;
+        const int32_t a0 = hit_at(e, yl[0], Wf), a4 = hit_at(e, yl[4], Wf);
+        const bool isLeft = a0 < A && a4 < A, isRight = a0 >= B && a4 >= B;
+#pragma unroll
+        for (int m = 0; m < 5; m++) {
+          if (!(e.aty <= yl[m] && e.toy >= yl[m])) continue;
+          total[m] += w;
+          if (isLeft) left[m] += w;
+          if (isLeft || isRight) continue;
+          const int32_t at = m == 0 ? a0 : m == 4 ? a4 : hit_at(e, yl[m], Wf);
+          if (at < A1) left[m] += w;  // (a hit at x = 0 only counts)
+          else if (at < Bk) atomicAdd(&bkt[m][(at - A) >> (sh + 8)], 1u + ((uint32_t)w << 16));
+        }
+        return !isLeft && !isRight;
+      };
+      for (int i0 = 0; i0 < count; i0 += kLoads * kHeavyThreads) {
+        Entry e[kLoads];
+        int32_t w[kLoads];
+#pragma unroll
+        for (int u = 0; u < kLoads; u++) {
+          const int i = i0 + u * kHeavyThreads + tid;
+          e[u] = Entry{0.0f, 0.0f, 0.0f, 0.0f};
+          w[u] = 0;
+          if (i < count) {
+            e[u] = E[i];
+            w[u] = EW[i];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kLoads; u++) {
+          const int i = i0 + u * kHeavyThreads + tid;
+          if (scan(e[u], w[u], i < count)) {
+            const int at = atomicAdd(&sSel, 1);
+            if (at < kHeavySel) sel[at] = ((uint32_t)i << 1) | (w[u] > 0 ? 1u : 0u);
+          }
+        }
+      }
+      ne = wave_incl_sum(ne);
+      if (lane == 63 && ne) atomicAdd(&sNe, ne);
+      if (ballot(notSpan) && lane == 0) sNotSpan = 1;
+#pragma unroll
+      for (int m = 0; m < 5; m++) {
+        left[m] = wave_incl_sum(left[m]);
+        total[m] = wave_incl_sum(total[m]);
+        if (lane == 63 && left[m]) atomicAdd(&sLeft[m], left[m]);
+        if (lane == 63 && total[m]) atomicAdd(&sTotal[m], total[m]);
+      }
+    }
+    if (wave == 0) nx.step_task(P);
+    __syncthreads();
+    if (wave == 0) nx.step_call(P);
+    ne = uni(sNe);
+    leave = leave || (ne > 0 && !uni(sNotSpan) && (ne % 2) == 0) ||
+            (uni(sTotal[0]) | uni(sTotal[1]) | uni(sTotal[2]) | uni(sTotal[3]) | uni(sTotal[4])) != 0;
+    if (!leave) {
+      if (mask && wave < nw && lane == 0) {
+        // a mask row is cleared but for its coverage range
+        const int32_t wx0 = gx0 + wave * kWinA, wx1 = wx0 + kWinA < cx1 ? wx0 + kWinA : cx1;
+        const int32_t lo = covLo > wx0 ? covLo : wx0, hi = covHi < wx1 ? covHi : wx1;
+        atomicAdd(&D[wave][0], kClear);
+        atomicAdd(&D[wave][wx1 - wx0], -kClear);
+        if (ne > 0 && lo < hi) {
+          atomicAdd(&D[wave][lo - wx0], -kClear);
+          atomicAdd(&D[wave][hi - wx0], kClear);
+        }
+      }
+      // places of the buckets in their line, and the counts left of them
+      for (int m = wave; m < 5; m += kHeavyWavesPerGroup) {
+        const uint32_t v = bkt[m][lane];
+        int nHit, wAll;
+        const int at = wave_excl_scan((int)(v & 0xffffu), &nHit);
+        const int cw = uni(sLeft[m]) + wave_excl_scan((int32_t)v >> 16, &wAll);
+        bkt[m][lane] = (uint32_t)at;
+        left0[m][lane] = cw;
+        if (lane == 0) sHits[m] = nHit;
+      }
+      // the listed entries, or the band's when they do not fit the list
+      const int nSel = uni(sSel);
+      const bool kept = nSel <= kHeavySel;
+      const int nList = kept ? nSel : count;
+      for (int l0 = 0; ne > 0 && l0 < 5;) {
+        __syncthreads();
+        // as many lines at a time as the key space holds
+        int base[5], nKeys = 0, l1 = l0;
+#pragma unroll
+        for (int m = 0; m < 5; m++) {
+          base[m] = nKeys;
+          const int h = uni(sHits[m]);
+          if (m == l1 && nKeys + h <= kHeavyKeys) {
+            nKeys += h;
+            l1++;
+          }
+        }
+        if (l1 == l0) {  // a line alone exceeds it (the same in every wave)
+          leave = true;
+          break;
+        }
+        auto deal = [&](const Entry& e, uint32_t k) {
+          if (e.toy <= scanTop || e.aty >= scanBottom) return;
+#pragma unroll
+          for (int m = 0; m < 5; m++) {
+            if (m < l0 || m >= l1 || !(e.aty <= yl[m] && e.toy >= yl[m])) continue;
+            const int32_t at = hit_at(e, yl[m], Wf);
+            if (at < A1 || at >= Bk) continue;
+            const uint32_t rel = (uint32_t)(at - A);
+            keys[base[m] + atomicAdd(&bkt[m][rel >> (sh + 8)], 1u)] = ((rel & ((1u << (sh + 8)) - 1u)) << 18) | k;
+          }
+        };
+#pragma unroll 2
+        for (int i = tid; i < nList; i += kHeavyThreads) {
+          const uint32_t k = kept ? sel[i] : ((uint32_t)i << 1) | (EW[i] > 0 ? 1u : 0u);
+          deal(E[k >> 1], k);
+        }
+        if (wave == 0 && l0 == 0) nx.step_band(P, next);
+        __syncthreads();
+        // a bucket's place now points past its keys, at the next one's.  The
+        // buckets go round the waves: a shared counter read by one lane would
+        // put that lane on a path of its own from here to the next round.
+        for (int j = wave; j < (l1 - l0) * nb; j += kHeavyWavesPerGroup) {
+          const int m = l0 + j / nb, b = j % nb;
+          const int o1 = uni((int)bkt[m][b]), o0 = b > 0 ? uni((int)bkt[m][b - 1]) : 0;
+          const int32_t cb = uni(left0[m][b]);
+          if (o1 == o0 && !should_fill(rule, cb)) continue;
+          const int32_t bx0 = gx0 + b * px;
+          const int win = (b * px) / kWinA;
+          const int32_t wx0 = gx0 + win * kWinA, wx1 = wx0 + kWinA < cx1 ? wx0 + kWinA : cx1;
+          const int32_t lo = (bx0 > covLo ? bx0 : covLo) - bx0;
+          int32_t hi = bx0 + px < covHi ? bx0 + px : covHi;
+          hi = (hi < wx1 ? hi : wx1) - bx0;
+          if (lo >= hi) continue;
+          const int kb = m == 0 ? base[0] : m == 1 ? base[1] : m == 2 ? base[2] : m == 3 ? base[3] : base[4];
+          int32_t* const Db = D[win] + (bx0 - wx0);
+          Walk32 c;
+          c.count = cb;
+          walk32_staged<kBucketKeyBits>(keys + kb + o0, o1 - o0, rule, Db, lo, hi, c);
+          if (lane == 0) walk32_borders(should_fill(rule, cb), should_fill(rule, c.count), Db, lo, hi);
+        }
+        l0 = l1;
+        __syncthreads();
+      }
+      __syncthreads();
+    }
+    if (leave) {  // to the rows kernel, window by window
+      if (wave == 0) nx.step_band(P, next);
+      for (int i = tid; i < kHeavyWins * (kWinA + 4); i += kHeavyThreads) ((int32_t*)D)[i] = 0;
+      if (tid < nw) P.taskOrder[P.taskCap + atomicAdd(&P.counters[kCntLeft], 1)] = first + tid;
+      continue;
+    }
+    if (ne == 0 && wave == 0) nx.step_band(P, next);
+    if (wave < nw) {
+      const int32_t wx0 = gx0 + wave * kWinA, wx1 = wx0 + kWinA < cx1 ? wx0 + kWinA : cx1;
+      RowRuns rr;
+      rr.kind = ne > 0 ? kRowCoverage : kRowOps;
+      rr.pad = 0;
+      rr.off = 0;
+      rr.n = emit_runs(P, D[wave], nullptr, wx0, wx1 - wx0, false, &rc, &rr.off);
+      P.tasks[first + wave] = rr;  // every lane stores the same value
+    }
+  }
+  if (lane == 0 && rc.used) atomicAdd(&P.counters[kCntRunsUsed], rc.used);
+}
+
+__global__ void __launch_bounds__(64, 4) scene_rows_kernel(ScenePools P) {
   extern __shared__ __align__(16) char smem[];
   const int lane = threadIdx.x;
   const size_t fixedBytes = row_lds_fixed_bytes(kWinA);
   RowLds Ll = row_lds_carve(smem, smem + fixedBytes, P.ldsCap, kWinA);
   RowLds Lg = row_lds_carve(smem, P.gscratch + (size_t)blockIdx.x * row_cap_bytes(P.gcap), P.gcap, kWinA);
-  // the wide path stages its keys through AX and the LDS arrays, which follow it
-  Ll.wide = Lg.wide = (uint64_t*)Ll.AX;
-  Ll.wideCap = Lg.wideCap = (int)((kWinA * 4 + row_cap_bytes(P.ldsCap)) / 8);
   for (int i = lane; i < kWinA + 4; i += 64) Ll.D[i] = 0;
   __syncthreads();
   if (P.counters[kCntError]) return;
-  // this launch's share of the work-item order: the large-band items come first
-  const int nBig = P.counters[kCntBigTasks];
-  const int tBegin = kBig ? 0 : nBig;
-  const int tEnd = kBig ? nBig : P.counters[kCntGroups];
-  int32_t* heads = P.queues + (kBig ? 0 : kQueues * kQueueStride);
-  // Each wave appends its runs to chunks of the run pool it takes one at a
-  // time (one atomic per chunk, not per task).
-  int cursor = 0, chunkEnd = 0, used = 0;
+  // the rows the heavy kernel left, then the work items after its own
+  const int nHeavy = P.counters[kCntHeavy], nLeft = P.counters[kCntLeft];
+  const int nItems = nLeft + P.counters[kCntGroups] - nHeavy;
+  RunCursor rc;
   for (;;) {
-    const int q = tBegin + queue_next<kRowGranule>(heads, tEnd - tBegin);
-    if (q >= tEnd) break;
+    const int q = queue_next<kRowGranule>(P.queues + kQueues * kQueueStride, nItems);
+    if (q >= nItems) break;
     // Work item, call and the call's records are the same in every lane:
     // read them into scalar registers.
-    const int first = uni(P.taskOrder[q]);
+    const int first = uni(q < nLeft ? P.taskOrder[P.taskCap + q] : P.taskOrder[nHeavy + q - nLeft]);
     const int itw = uni(P.taskItem[first]);
     const int it = itw & 0x7fffffff;
     ItemGeom g = P.geo[it];
@@ -1876,70 +2289,13 @@ __global__ void __launch_bounds__(64, 5) scene_rows_kernel(ScenePools P) {
       if (kind < 0) {
         atomicOr(&P.counters[kCntError], 8);
       } else if (kind != kRowNone) {
-        // compact D[0..wlen] (nonzero deltas) and, for ops rows, the area
-        // factors of the pixels whose code is an area code, in one pass.
-        // Coverage rows need no codes, only the nonzero deltas.  The wave's
-        // run chunk is first made to hold the most the row can write (wlen + 1
-        // deltas, and wlen area factors on ops rows).  D has ww + 4 entries
-        // and is zero beyond wlen, so a lane with i0 <= wlen moves its 4
-        // entries as one 16-byte access.
         const int wlen = C.wx1 - C.wx0;
-        const bool ops = kind == kRowOps;
-        const int most = ops ? 2 * wlen + 1 : wlen + 1;
-        if (cursor + most > chunkEnd) {
-          cursor = queue_take(&P.counters[kCntRuns], kRunChunk);
-          chunkEnd = cursor + kRunChunk;
-        }
-        rr.off = cursor;
-        int written = 0;
-        if (chunkEnd > P.runCap) {
-          atomicOr(&P.counters[kCntError], 16);
-          for (int i = lane; i <= wlen; i += 64) L.D[i] = 0;
-        } else {
-          int carry = 0;
-          for (int base = 0; base <= wlen; base += 4 * kWave) {
-            const int i0 = base + 4 * lane;
-            int4 dv = make_int4(0, 0, 0, 0);
-            if (i0 <= wlen) dv = *(const int4*)(Ll.D + i0);
-            const int32_t d[4] = {dv.x, dv.y, dv.z, dv.w};
-            bool area[4] = {false, false, false, false};
-            if (ops) {
-              const int32_t c0 = d[0], c1 = c0 + d[1], c2 = c1 + d[2], c3 = c2 + d[3];
-              int32_t tot;
-              const int32_t off = carry + wave_excl_scan(c3, &tot);
-              carry += tot;
-              const int32_t code[4] = {off + c0, off + c1, off + c2, off + c3};
-#pragma unroll
-              for (int q = 0; q < 4; q++) area[q] = i0 + q < wlen && code[q] >= kArea && code[q] < kClear;
-            }
-            int n = 0;
-#pragma unroll
-            for (int q = 0; q < 4; q++) n += (d[q] != 0 ? 1 : 0) + (area[q] ? 1 : 0);
-            int ntot;
-            const int p = wave_excl_scan(n, &ntot);
-            if (i0 <= wlen) {
-              int2* out = P.runs + rr.off + written + p;
-              int w = 0;
-#pragma unroll
-              for (int q = 0; q < 4; q++) {
-                const int x = C.wx0 + i0 + q;
-                if (d[q] != 0) out[w++] = make_int2(x, d[q]);
-                if (area[q]) out[w++] = make_int2(x | kRunArea, (int32_t)L.AX[i0 + q]);
-              }
-              *(int4*)(Ll.D + i0) = make_int4(0, 0, 0, 0);
-            }
-            written += ntot;
-          }
-        }
-        rr.n = written;
-        cursor += written;
-        used += written;
-        __syncthreads();
+        rr.n = emit_runs(P, Ll.D, L.AX, C.wx0, wlen, kind == kRowOps, &rc, &rr.off);
       }
       P.tasks[task] = rr;  // every lane stores the same value
     }
   }
-  if (threadIdx.x == 0 && used) atomicAdd(&P.counters[kCntRunsUsed], used);
+  if (threadIdx.x == 0 && rc.used) atomicAdd(&P.counters[kCntRunsUsed], rc.used);
 }
 
 // ---------------------------------------------------------------------------
@@ -2200,10 +2556,7 @@ __global__ void __launch_bounds__(64) scene_compose_kernel(ScenePools P, void* c
 // launcher
 // ---------------------------------------------------------------------------
 int scene_set_lds_limits(size_t bytes) {
-  // the kernel's static LDS (its task slot) counts against the same limit
-  if (hipFuncSetAttribute((const void*)scene_rows_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)(bytes - 1024)) != hipSuccess ||
-      hipFuncSetAttribute((const void*)scene_rows_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+  if (hipFuncSetAttribute((const void*)scene_rows_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)(bytes - 1024)) != hipSuccess)
     return kErrDevice;
   return 0;
@@ -2336,7 +2689,7 @@ int scene_launch_bands(const ScenePools& p, int grid, hipStream_t s) {
 
 int scene_launch_bins(const ScenePools& p, int grid, hipStream_t s) {
   hipLaunchKernelGGL(scene_task_map_kernel, dim3(grid / 4 > 0 ? grid / 4 : 1), dim3(kTaskMapBlock), 0, s, p);
-  hipLaunchKernelGGL(scene_task_scan_kernel, dim3(1), dim3(64), 0, s, p.counters, p.bigClass);
+  hipLaunchKernelGGL(scene_task_scan_kernel, dim3(1), dim3(64), 0, s, p);
   hipLaunchKernelGGL(scene_task_order_kernel, dim3(grid >= 8 ? grid / 4 : grid), dim3(64), 0, s, p);
   hipLaunchKernelGGL(scene_bin_kernel<false>, dim3(grid), dim3(64), 0, s, p);
   hipLaunchKernelGGL(scene_bin_scan_kernel, dim3(1), dim3(kScanBlock), 0, s, p);
@@ -2344,36 +2697,11 @@ int scene_launch_bins(const ScenePools& p, int grid, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
 }
 
-int scene_launch_rows(const ScenePools& p, const RowShape& shape, int numCUs, hipStream_t s,
-                      hipStream_t aux, hipEvent_t fork, hipEvent_t join) {
-  const int gridSmall = scene_queue_grid(numCUs * shape.wavesPerCU);
-  ScenePools small = p;
-  small.ldsCap = shape.ldsCap;
-  const size_t smallLds = row_lds_fixed_bytes(kWinA) + row_cap_bytes(shape.ldsCap);
-  if (shape.mode == kRowsSingle) {  // every task; big ones use the row scratch
-    hipLaunchKernelGGL(scene_rows_kernel<false>, dim3(gridSmall), dim3(64), smallLds, s, small);
-    return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
-  }
-  const int gridBig = scene_queue_grid(numCUs * shape.bigWaves);
-  ScenePools big = p;
-  big.ldsCap = shape.bigCap;
-  const size_t bigLds = row_lds_fixed_bytes(kWinA) + row_cap_bytes(shape.bigCap);
-  // the small-band launch never needs global row scratch (its bands hold
-  // fewer entries than its LDS capacity); with no slots, a row that did would
-  // report a capacity error instead of reaching another wave's slot
-  small.gscratch = nullptr;
-  small.gcap = 0;
-  if (shape.mode == kRowsSequential) {
-    hipLaunchKernelGGL(scene_rows_kernel<true>, dim3(gridBig), dim3(64), bigLds, s, big);
-    hipLaunchKernelGGL(scene_rows_kernel<false>, dim3(gridSmall), dim3(64), smallLds, s, small);
-    return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
-  }
-  if (hipEventRecord(fork, s) != hipSuccess || hipStreamWaitEvent(aux, fork, 0) != hipSuccess)
-    return kErrDevice;
-  hipLaunchKernelGGL(scene_rows_kernel<false>, dim3(gridSmall), dim3(64), smallLds, aux, small);
-  hipLaunchKernelGGL(scene_rows_kernel<true>, dim3(gridBig), dim3(64), bigLds, s, big);
-  if (hipEventRecord(join, aux) != hipSuccess || hipStreamWaitEvent(s, join, 0) != hipSuccess)
-    return kErrDevice;
+int scene_launch_rows(const ScenePools& p, const RowShape& shape, int numCUs, hipStream_t s) {
+  hipLaunchKernelGGL(scene_heavy_kernel, dim3(scene_queue_grid(numCUs * kHeavyGroupsPerCU)), dim3(kHeavyThreads), 0,
+                     s, p);
+  const size_t lds = row_lds_fixed_bytes(kWinA) + row_cap_bytes(shape.ldsCap);
+  hipLaunchKernelGGL(scene_rows_kernel, dim3(scene_queue_grid(numCUs * shape.wavesPerCU)), dim3(64), lds, s, p);
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
 }
 
