@@ -69,6 +69,7 @@ struct pxh_scene {
   pxh::ScenePoly* dPolys = nullptr;
   int32_t* dOrder = nullptr;  // geometry workgroup -> call, longest call first
   int32_t nBig = 0;           // calls of more than 256 commands (first in order)
+  int32_t nStrokes = 0;       // strokes (their calls end the order)
   int32_t bigCmds = 0;        // their commands
   float* dDashes = nullptr;
   size_t dItemsCap = 0, dCmdsCap = 0, dPolysCap = 0, dOrderCap = 0, dDashesCap = 0;
@@ -831,20 +832,23 @@ int scene_alloc(pxh_scene* sc) {
   size_t oPts = carve((size_t)sc->ptCap * 8), oPtP = carve((size_t)sc->ptCap * 4);
   size_t oPtS = carve((size_t)sc->ptCap * 4);
   const size_t nChunk = (size_t)sc->ptCap / kBigChunk + (size_t)sc->nBig + 1;
-  size_t oBCS = carve(((size_t)sc->nBig + 1) * 4), oBGS = carve(((size_t)sc->nBig + 1) * 4);
+  size_t oBCS = carve(((size_t)sc->nBig + 1) * 4);
+  const size_t nStrokeChunk = sc->nStrokes ? (size_t)sc->ptCap / 64 + (size_t)sc->nStrokes + 1 : 1;
+  size_t oStr = carve(sc->nStrokes ? nI * sizeof(StrokeCall) : sizeof(StrokeCall)), oStC = carve(nStrokeChunk * 8);
+  size_t oGrp = carve(((size_t)sc->segCap / 64 + 1) * 4);
   size_t oBPS = carve(((size_t)sc->nBig + 1) * 4);
   size_t oBPC = carve((nP / kBigPolyChunk + (size_t)sc->nBig + 1) * 16);
   size_t oBCC = carve(nChunk * 8), oBCB = carve(nChunk * 16);
   size_t oSeg = carve((size_t)sc->segCap * 16), oSegW = carve((size_t)sc->segCap);
   size_t oSegB = carve((size_t)sc->segCap * 8), oSegC = carve(((size_t)sc->segCap / 64 + 1) * 8);
   size_t oParts = carve((size_t)sc->bandCap * sizeof(PartInfo)), oBI = carve((size_t)sc->bandCap * 4);
+  size_t oTile = carve(kBandTilesMax * 4), oQuart = carve(kBandTilesMax * 16);
   size_t oEnt = carve((size_t)sc->entryCap * sizeof(Entry)), oEW = carve((size_t)sc->entryCap);
   size_t oTask = carve((size_t)sc->taskCap * sizeof(RowRuns)), oRun = carve((size_t)sc->runCap * 8);
-  size_t oTaskItem = carve((size_t)sc->taskCap * 4), oTaskOrd = carve((size_t)sc->taskCap * 8);
-  size_t oTaskCls = carve((size_t)sc->taskCap);
+  size_t oTaskChunk = carve(((size_t)sc->taskCap / 64 + nI + 1) * 8), oTaskOrd = carve((size_t)sc->taskCap * 16);
   size_t oRows = carve(nI * sizeof(int4)), oBinC = carve((size_t)sc->binSlots * 4);
   size_t oPaint = carve(nI * sizeof(int4)), oSpan = carve(nI * sizeof(int4));
-  size_t oBinO = carve(((size_t)sc->binSlots + 1) * 4), oBinL = carve((size_t)sc->binCap * 4);
+  size_t oBinO = carve((size_t)sc->binSlots * 4), oBinL = carve((size_t)sc->binCap * 4);
   size_t oQ = carve(kQueueSets * kQueues * kQueueStride * 4);
   size_t oCnt = carve(kCounterInts * 4);
   if (off > sc->dMemBytes) {
@@ -863,6 +867,8 @@ int scene_alloc(pxh_scene* sc) {
   p.nBig = sc->nBig;
   p.bigCmdStart = sc->dOrder + sc->items.size();
   p.bigCmds = sc->bigCmds;
+  p.strokeItems = sc->dOrder + sc->items.size() + sc->nBig + 1;
+  p.nStrokes = sc->nStrokes;
   p.dashes = sc->dDashes;
   p.nItems = (int32_t)nI;
   p.geo = (ItemGeom*)(b + oGeo);
@@ -876,7 +882,9 @@ int scene_alloc(pxh_scene* sc) {
   p.ptSeg = (int32_t*)(b + oPtS);
   p.ptCap = sc->ptCap;
   p.bigChunkStart = (int32_t*)(b + oBCS);
-  p.bigGroupStart = (int32_t*)(b + oBGS);
+  p.strokes = (StrokeCall*)(b + oStr);
+  p.strokeChunk = (int2*)(b + oStC);
+  p.groupItem = (int32_t*)(b + oGrp);
   p.bigPolyStart = (int32_t*)(b + oBPS);
   p.bigPolyChunk = (int4*)(b + oBPC);
   p.bigChunkCnt = (int2*)(b + oBCC);
@@ -889,13 +897,14 @@ int scene_alloc(pxh_scene* sc) {
   p.parts = (PartInfo*)(b + oParts);
   p.bandItem = (int32_t*)(b + oBI);
   p.bandCap = sc->bandCap;
+  p.tileSum = (int32_t*)(b + oTile);
+  p.bandQuarter = (int4*)(b + oQuart);
   p.entries = (Entry*)(b + oEnt);
   p.entW = (int8_t*)(b + oEW);
   p.entryCap = sc->entryCap;
   p.tasks = (RowRuns*)(b + oTask);
-  p.taskItem = (int32_t*)(b + oTaskItem);
-  p.taskOrder = (int32_t*)(b + oTaskOrd);
-  p.taskClass = (int8_t*)(b + oTaskCls);
+  p.taskChunk = (int2*)(b + oTaskChunk);
+  p.taskOrder = (int2*)(b + oTaskOrd);
   p.taskCap = sc->taskCap;
   p.runs = (int2*)(b + oRun);
   p.runCap = sc->runCap;
@@ -1022,6 +1031,13 @@ int scene_upload(pxh_scene* sc, int lane) {
       sc->bigCmds += sc->items[sc->order[k]].cmdCount;
     }
     sc->order.push_back(sc->bigCmds);
+    // then the strokes
+    sc->nStrokes = 0;
+    for (size_t i = 0; i < n; i++)
+      if (sc->items[i].stroke) {
+        sc->order.push_back((int32_t)i);
+        sc->nStrokes++;
+      }
     const size_t m = sc->order.size();
     if (int r = scene_buf(&sc->dOrder, &sc->dOrderCap, m)) return r;
     PXH_HIP(hipMemcpyAsync(sc->dOrder, sc->order.data(), m * sizeof(int32_t), hipMemcpyHostToDevice, st));
@@ -1062,6 +1078,8 @@ int scene_launch(pxh_scene* sc, pxh_image* img, int lane, bool checked = false) 
   p.nBig = sc->nBig;
   p.bigCmdStart = sc->dOrder + sc->items.size();
   p.bigCmds = sc->bigCmds;
+  p.strokeItems = sc->dOrder + sc->items.size() + sc->nBig + 1;
+  p.nStrokes = sc->nStrokes;
   p.dashes = sc->dDashes;
   const RowShape shape = kRowShapes[sc->rowShape];
   p.ldsCap = shape.ldsCap;
@@ -1077,11 +1095,11 @@ int scene_launch(pxh_scene* sc, pxh_image* img, int lane, bool checked = false) 
   }
   if (!r) {
     LaunchTimer t("scene_bands", st);
-    r = scene_launch_bands(p, g.numCUs * 64, st);
+    r = scene_launch_bands(p, st);
   }
   if (!r) {
     LaunchTimer t("scene_bins", st);
-    r = scene_launch_bins(p, g.numCUs * 4, st);
+    r = scene_launch_tasks(p, st);
   }
   if (!r) {
     LaunchTimer t("scene_rows_kernel", st);

@@ -80,6 +80,14 @@ struct ItemGeom {
   int32_t pad;
 };
 
+// A stroke's point chunks (scene_stroke_*): its first chunk, their number, the
+// error its counting met, and its bounds as ordered unsigned keys.
+struct StrokeCall {
+  int32_t chunkBase, nChunks;
+  int32_t err, pad;
+  uint32_t bd[4];  // xMin, xMax, yMin, yMax
+};
+
 // Phase-A output of one (call, row, window).
 struct RowRuns {
   int32_t off, n;    // run entries in the run pool
@@ -124,6 +132,8 @@ enum SceneCounter {
   kCntHeavy,     // phase-A work items of the heavy kernel (the first in their order)
   kCntGroups,    // phase-A work items (set by the class scan)
   kCntLeft,      // rows the heavy kernel leaves to the rows kernel
+  kCntStrokeChunks,  // point chunks of the strokes
+  kCntChunks,        // 64-unit chunks of the work items
   kNumCounters
 };
 
@@ -134,22 +144,18 @@ enum SceneCounter {
 // or else a single row, so that no item is long.  Items run longest first:
 // an item's cost class is the bit length of the largest band entry count
 // among its rows, and the items are ordered by class, descending.  Work
-// items are named by the task of their first row; the task map marks
-// grouped items (taskItem bit 31) and gives the other rows of a group no
-// class (-1).
+// items are named by the task of their first row; grouped items are marked
+// (bit 31 of the call).
 // The class histogram and the scatter cursors follow the counters.
 constexpr int kCostClasses = 32;
 constexpr int kCntClassHist = kNumCounters;                  // kCostClasses ints
 constexpr int kCntClassCursor = kNumCounters + kCostClasses;  // kCostClasses ints
-// The band-entry scan runs over kEntryTiles contiguous tiles of bands; the
-// tile sums, then the tile offsets, follow the class cursors.
-constexpr int kEntryTiles = 256;
-constexpr int kCntTileSum = kNumCounters + 2 * kCostClasses;  // kEntryTiles ints
-constexpr int kCounterInts = kNumCounters + 2 * kCostClasses + kEntryTiles;
+constexpr int kCounterInts = kNumCounters + 2 * kCostClasses;
 
 // Phase B looks calls up by row bins of kBinRows canvas rows: each bin lists,
 // in call order, the calls whose rows meet it.
 constexpr int kBinRows = 16;
+constexpr int kBandTilesMax = 4096;
 
 // Phase A and B deal out work through kQueues independent queues (queue q
 // serves work items q, q + kQueues, ...), so that no single counter takes
@@ -177,6 +183,8 @@ struct ScenePools {
   int32_t nBig;              // calls of more than 256 commands, first in itemOrder
   const int32_t* bigCmdStart;  // their command counts' exclusive prefix (nBig + 1)
   int32_t bigCmds;           // bigCmdStart[nBig]
+  const int32_t* strokeItems;  // the strokes among the calls
+  int32_t nStrokes;
   int32_t W, H;              // target size
   // per-call outputs
   ItemGeom* geo;
@@ -189,18 +197,19 @@ struct ScenePools {
   // pools
   float2* pts;
   int32_t* ptPoly;
-  int32_t* ptSeg;            // segments each point emits (geometry scratch)
+  int32_t* ptSeg;            // segments each point of a stroke emits (a byte per lane of four)
+  StrokeCall* strokes;       // per call (strokes only)
+  int2* strokeChunk;         // per point chunk: call, segment count then offset in the call
+  int32_t* groupItem;        // call of each 64-segment group
   int32_t ptCap;
   // segments of the big fill calls, in chunks of kBigChunk points spread
   // over the device: chunk prefix per big call (nBig + 1), per chunk
-  // (segment count, segment offset in the call) and bounds, and the prefix
-  // of their 64-segment groups (nBig + 1)
+  // (segment count, segment offset in the call) and bounds
   int32_t* bigChunkStart;
   int32_t* bigPolyStart;     // subpath-chunk prefix of the big calls (nBig + 1)
   int4* bigPolyChunk;        // per subpath chunk: points, error, point offset
   int2* bigChunkCnt;
   float4* bigChunkBd;
-  int32_t* bigGroupStart;
   float4* segs;
   int8_t* segW;
   int2* segBand;             // per segment: first band, last band | kSegAA
@@ -208,15 +217,17 @@ struct ScenePools {
   int32_t segCap;
   PartInfo* parts;
   int32_t* bandItem;
+  int32_t* tileSum;          // entries of each tile of bands (kBandTilesMax)
+  int4* bandQuarter;         // few bands: each one's entries by quarter of its groups
   int32_t bandCap;
   Entry* entries;
   int8_t* entW;
   int32_t entryCap;
   RowRuns* tasks;
-  int32_t* taskItem;         // call of each work item
-  int32_t* taskOrder;        // work items in the order phase A takes them (longest first),
-                             // then from taskCap on the rows the heavy kernel leaves
-  int8_t* taskClass;         // cost class of each work item
+  int2* taskChunk;           // per 64 units (row group, window) of a call: call, chunk in it
+  int2* taskOrder;           // work items in the order phase A takes them (longest first):
+                             // first task, call (bit 31: a group of rows); then from
+                             // taskCap on the rows the heavy kernel leaves
   int32_t taskCap;
   int2* runs;
   int32_t runCap;
@@ -224,7 +235,7 @@ struct ScenePools {
   int4* itemPaint;           // per call: rgbx, mode, first task, windows per row
   int4* itemSpan;            // per call: rowStart, rowCount, xlo, xhi
   int32_t* binCount;         // nBins
-  int32_t* binOff;           // nBins + 1
+  int32_t* binOff;           // nBins
   int32_t* binList;          // call indices per bin
   int32_t binCap;
   int32_t binSlots;          // capacity of binCount / binOff (bins)
@@ -271,8 +282,8 @@ int scene_launch_expand(const GlyphInst* inst, int32_t n, const SceneCmd* arenaC
                         const ScenePoly* arenaPolys, SceneCmd* cmds, ScenePoly* polys, hipStream_t s);
 int scene_launch_clear(const ScenePools& p, hipStream_t s);
 int scene_launch_geometry(const ScenePools& p, hipStream_t s);
-int scene_launch_bands(const ScenePools& p, int grid, hipStream_t s);
-int scene_launch_bins(const ScenePools& p, int grid, hipStream_t s);
+int scene_launch_bands(const ScenePools& p, hipStream_t s);  // band entries and row bins
+int scene_launch_tasks(const ScenePools& p, hipStream_t s);  // phase A's work items and their order
 // Phase A in the given shape: the heavy rows, then the others.
 int scene_launch_rows(const ScenePools& p, const RowShape& shape, int numCUs, hipStream_t s);
 int scene_launch_compose(const ScenePools& p, void* canvas, bool a8, unsigned long long* touched,

@@ -12,9 +12,11 @@
 namespace pxh {
 
 constexpr int kBlock = 256;
-constexpr int kBigGeomBlock = 1024;  // geometry workgroup of a call of more than kBlock commands
 constexpr int kStagePts = 4096;  // LDS points of the geometry stage (32 KB)
 constexpr int kBigSegGrid = 1024;  // workgroups of the big-fill segment kernels (grid-stride)
+constexpr int kStrokeGrid = 2048;  // workgroups of the stroke segment kernels (grid-stride)
+constexpr int kSegBandBlocks = 2048;  // workgroups of the band ranges (a wave per 64 segments)
+constexpr int kTaskBlocks = 1024;     // workgroups of the work-item kernels (a wave per 64 units)
 
 // A value that is the same in every lane, moved to a scalar register.
 __device__ __forceinline__ int32_t uni(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -44,19 +46,9 @@ __device__ __forceinline__ int block_excl_scan_n(int v, int* total, int* sh) {
   return off + x;
 }
 
-__device__ __forceinline__ int block_excl_scan(int v, int* total, int* sh) {
-  return block_excl_scan_n<kBlock>(v, total, sh);
-}
-
-// Single-workgroup scans over every band / call / bin use the largest
-// workgroup so that they take few serial steps.
+// Single-workgroup scans over the big calls use the largest workgroup so that
+// they take few serial steps.
 constexpr int kScanBlock = 1024;
-
-__device__ int block_sum(int v, int* sh) {
-  int t;
-  block_excl_scan(v, &t, sh);
-  return t;
-}
 
 // ---------------------------------------------------------------------------
 // commands (SceneCmd) -> points, commandsToShapes (paths.nim:654-1057)
@@ -99,15 +91,18 @@ struct StageEmit {
   }
 };
 
-// flatten_cubic (paths.nim:677-721) run by a group of kFlatGroup lanes of
-// one wave (lanes gbase .. gbase + kFlatGroup - 1, u = lane - gbase).  Each
+// flatten_cubic (paths.nim:677-721) run by a group of G lanes of one wave
+// (lanes gbase .. gbase + G - 1, u = lane - gbase).  Each
 // round lane u tries the step halved u times; the first candidate in
 // halving order that is accepted, or that reaches epsilon, decides the round,
 // which is the decision the sequential loop reaches after u halvings (each
 // halving and its reuse of the halfway point are exact, so the candidates
 // evaluate the same points).  Every lane of the group calls emit alike.
-constexpr int kFlatGroup = 8;
-template <class Emit>
+template <int G>
+struct Lanes {
+  static constexpr int value = G;
+};
+template <int G, class Emit>
 __device__ __forceinline__ int32_t flatten_cubic_group(V2 at, V2 c1, V2 c2, V2 to, float errSq, Emit& emit, int u,
                                        int gbase) {
   float t = 0.0f, step = 1.0f;
@@ -129,9 +124,9 @@ __device__ __forceinline__ int32_t flatten_cubic_group(V2 at, V2 c1, V2 c2, V2 t
       const float errorTangent = lensq(lineTangent - curveTangentScaled);
       ok = !(error + errorTangent > errSq);
     }
-    const uint64_t bm = (__ballot(eps || ok) >> gbase) & ((1ull << kFlatGroup) - 1ull);
-    if (bm == 0) {  // every candidate was refined: go on from step / 2^kFlatGroup
-      for (int q = 0; q < kFlatGroup; q++) step /= 2.0f;
+    const uint64_t bm = (__ballot(eps || ok) >> gbase) & ((1ull << G) - 1ull);
+    if (bm == 0) {  // every candidate was refined: go on from step / 2^G
+      for (int q = 0; q < G; q++) step /= 2.0f;
       continue;
     }
     const int src = gbase + __builtin_ctzll(bm);
@@ -240,25 +235,26 @@ struct CircleEmit {
   }
 };
 
-__device__ __forceinline__ void circle_segments(V2 at, const SceneItem& I, SegSink& sink) {
+// The quarters [q0, q1) of the circle: quarter q's cubic starts where quarter
+// q - 1's ends (its last flattened point is its end point exactly: the cubic
+// at t = 1 adds zeros to it), so the quarters are independent.
+__device__ __forceinline__ void circle_segments(V2 at, int q0, int q1, const SceneItem& I, SegSink& sink) {
   const double K = 4.0 * (-1.0 + 1.4142135623730951) / 3.0;  // splineCircleK (float64)
-  float cx = at.x, cy = at.y, rx = I.halfStroke, ry = I.halfStroke;
-  double mx = K * (double)rx, my = K * (double)ry;
-  V2 s = v2(cx + rx, cy);
-  V2 st = I.identity ? s : mat_apply(I.mat, s);
-  CircleEmit ce{&sink, &I, v2(st.x, quantize_y(st.y))};
-  V2 a = s;
-  V2 c1 = v2(cx + rx, (float)((double)cy + my)), c2 = v2((float)((double)cx + mx), cy + ry), to = v2(cx, cy + ry);
-  flatten_cubic(a, c1, c2, to, I.errSq, ce);
-  a = to;
-  c1 = v2((float)((double)cx - mx), cy + ry); c2 = v2(cx - rx, (float)((double)cy + my)); to = v2(cx - rx, cy);
-  flatten_cubic(a, c1, c2, to, I.errSq, ce);
-  a = to;
-  c1 = v2(cx - rx, (float)((double)cy - my)); c2 = v2((float)((double)cx - mx), cy - ry); to = v2(cx, cy - ry);
-  flatten_cubic(a, c1, c2, to, I.errSq, ce);
-  a = to;
-  c1 = v2((float)((double)cx + mx), cy - ry); c2 = v2(cx + rx, (float)((double)cy - my)); to = v2(cx + rx, cy);
-  flatten_cubic(a, c1, c2, to, I.errSq, ce);
+  const float cx = at.x, cy = at.y, rx = I.halfStroke, ry = I.halfStroke;
+  const double mx = K * (double)rx, my = K * (double)ry;
+  const float right = cx + rx, left = cx - rx, low = cy + ry, high = cy - ry;
+  const float yp = (float)((double)cy + my), yn = (float)((double)cy - my);
+  const float xp = (float)((double)cx + mx), xn = (float)((double)cx - mx);
+#pragma unroll 1
+  for (int q = q0; q < q1; q++) {
+    const V2 a = q == 0 ? v2(right, cy) : q == 1 ? v2(cx, low) : q == 2 ? v2(left, cy) : v2(cx, high);
+    const V2 c1 = q == 0 ? v2(right, yp) : q == 1 ? v2(xn, low) : q == 2 ? v2(left, yn) : v2(xp, high);
+    const V2 c2 = q == 0 ? v2(xp, low) : q == 1 ? v2(left, yp) : q == 2 ? v2(xn, high) : v2(right, yn);
+    const V2 to = q == 0 ? v2(cx, low) : q == 1 ? v2(left, cy) : q == 2 ? v2(cx, high) : v2(right, cy);
+    const V2 st = I.identity ? a : mat_apply(I.mat, a);
+    CircleEmit ce{&sink, &I, v2(st.x, quantize_y(st.y))};
+    flatten_cubic(a, c1, c2, to, I.errSq, ce);
+  }
 }
 
 __device__ __forceinline__ void rect_segments(V2 at, V2 to, const SceneItem& I, SegSink& sink) {  // makeRect
@@ -331,19 +327,29 @@ __device__ __forceinline__ void join_segments(V2 prevPos, V2 pos, V2 nextPos, co
   }
 }
 
-// Stroke polygons attributed to point k of a shape with n points, in
-// strokeShapes order.
-// Segments of point k of a stroked polyline P[0..n): its cap or its
-// segment rectangle and join.  A round cap or round join comes last, so the
-// one circle a point may need is drawn at the end, from a single call site
-// (which keeps I and sink in registers once inlined).
+// The stroke of a call whose joins or caps are circles spreads every point
+// over four lanes, one per quarter of its circle.
+__device__ __forceinline__ int stroke_lanes(const SceneItem& I) { return (I.join == 1 || I.cap == 1) ? 4 : 1; }
+
+// Segments of point k of a stroked polyline P[0..n), in strokeShapes order:
+// its cap or its segment rectangle and join.  A round cap or round join comes
+// last, so the one circle a point may need is drawn at the end, from a single
+// call site (which keeps I and sink in registers once inlined).  Lane `sub` of
+// the point's `lanes` emits its share: lane 0 what precedes the circle, and
+// each lane its quarters of the circle.
 __device__ __forceinline__ void stroke_point(const float2* P, int k, int n, const SceneItem& I,
-                                             const float* dash, SegSink& sink) {
+                                             const float* dash, SegSink& sink, int sub, int lanes) {
   auto pt = [&](int i) { return v2(P[i].x, P[i].y); };
   bool closed = veq(pt(0), pt(n - 1));
   bool circle = false;
   V2 center = v2(0.0f, 0.0f);
-  if (k == 0) {
+  if (sub > 0) {
+    const bool cap = !closed && (k == 0 || k == n - 1) && I.cap == 1;
+    const bool join = k > 0 && (k < n - 1 || (closed && n >= 2)) && I.join == 1;
+    if (join) join_segments(pt(k), pt(k), pt(k), I, sink, &circle);  // a round join only decides on its circle
+    circle = circle || cap;
+    center = pt(k);
+  } else if (k == 0) {
     if (!closed) {
       if (I.cap == 1) {
         circle = true;
@@ -401,21 +407,21 @@ __device__ __forceinline__ void stroke_point(const float2* P, int k, int n, cons
       }
     }
   }
-  if (circle) circle_segments(center, I, sink);
+  if (circle) {
+    const int per = 4 / lanes;
+    circle_segments(center, sub * per, (sub + 1) * per, I, sink);
+  }
 }
 
 // ---------------------------------------------------------------------------
 // geometry: one workgroup per call
 // ---------------------------------------------------------------------------
-// Stages 6-7 of the geometry kernel: the call's bounds (merged from every
-// thread's `bd`) give its fill locals and band layout (fill_locals,
-// band_layout), then every segment gets its band range and AA bit, and every
-// 64-segment chunk the band range of its segments.
+// Stage 6 of a fill: the call's bounds (merged from every thread's `bd`)
+// give its fill locals and band layout (fill_locals, band_layout).
 template <int NB>
-__device__ __forceinline__ void geom_finish(const ScenePools& P, const SceneItem& I, int it, Bounds bd, int nseg, int sBase,
-                            Bounds* sBd, FillInfo& sF) {
+__device__ __forceinline__ void geom_finish(const ScenePools& P, const SceneItem& I, int it, Bounds bd, int nseg,
+                                            Bounds* sBd) {
   const int tid = threadIdx.x;
-  // 6. bounds -> fill locals, band layout
   for (int o = 32; o > 0; o >>= 1) {
     Bounds ob;
     ob.xMin = __shfl_xor(bd.xMin, o, 64);
@@ -426,54 +432,40 @@ __device__ __forceinline__ void geom_finish(const ScenePools& P, const SceneItem
   }
   if ((tid & 63) == 0) sBd[tid >> 6] = bd;
   __syncthreads();
-  if (tid == 0) {
-    Bounds b = sBd[0];
-    for (int w = 1; w < NB / 64; w++) b = bounds_merge(b, sBd[w]);
-    FillInfo f = {};
-    f.rgbx = I.rgbx;
-    f.mode = I.mode;
-    f.rule = I.stroke ? kNonZero : I.rule;
-    int32_t r = fill_locals(b, false, P.W, P.H, &f);
-    f.status = r;
-    if (r == kOk && f.pathWidth > 0) band_layout(&f, nseg);
-    P.fills[it] = f;
-    sF = f;
+  if (tid != 0) return;
+  Bounds b = sBd[0];
+  for (int w = 1; w < NB / 64; w++) b = bounds_merge(b, sBd[w]);
+  FillInfo f = {};
+  f.rgbx = I.rgbx;
+  f.mode = I.mode;
+  f.rule = I.rule;
+  const int32_t r = fill_locals(b, false, P.W, P.H, &f);
+  f.status = r;
+  if (r == kOk && f.pathWidth > 0) band_layout(&f, nseg);
+  P.fills[it] = f;
+}
+
+// Marks the 64-segment groups a call has allocated, for the band-range stage.
+__device__ __forceinline__ void mark_groups(const ScenePools& P, int it, int segBase, int segs) {
+  for (int g = (int)threadIdx.x; g < (segs + 63) / 64; g += (int)blockDim.x) P.groupItem[(segBase >> 6) + g] = it;
+}
+
+// Registers the chunks of a stroke's points (the whole workgroup; none when
+// the call failed).
+__device__ __forceinline__ void stroke_register(const ScenePools& P, const SceneItem& I, int it, int points) {
+  __shared__ int sChunk;
+  const int per = 256 / stroke_lanes(I);
+  const int n = I.strokeNone ? 0 : (points + per - 1) / per;
+  if (threadIdx.x == 0) {
+    sChunk = n ? atomicAdd(&P.counters[kCntStrokeChunks], n) : 0;
+    StrokeCall st = {};
+    st.chunkBase = sChunk;
+    st.nChunks = n;
+    st.err = kOk;
+    P.strokes[it] = st;
   }
   __syncthreads();
-  // 7. band range of every segment (partitionSegments 1201-1213) and its
-  // requiresAntiAliasing bit, and the band range of each 64-segment chunk
-  const FillInfo fl = sF;
-  if (fl.status == kOk && fl.pathWidth > 0) {
-    // four rounds at a time, their loads first
-    for (int j0 = 0; j0 < nseg; j0 += 4 * NB) {
-      float4 sg[4];
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int j = j0 + u * NB + tid;
-        sg[u] = j < nseg ? P.segs[sBase + j] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      }
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const int j = j0 + u * NB + tid;
-        int lo = 0x7fffffff, hi = -1;
-        if (j < nseg) {
-          uint32_t l = 0, h = 0;
-          if (fl.nParts > 1)
-            partition_range(sg[u].y, sg[u].w, (uint32_t)fl.startY, (uint32_t)fl.bandH, (uint32_t)fl.nParts,
-                            &l, &h);
-          const bool aa = seg_requires_aa(v2(sg[u].x, sg[u].y), v2(sg[u].z, sg[u].w));
-          P.segBand[sBase + j] = make_int2((int)l, (int)h | (aa ? kSegAA : 0));
-          lo = (int)l;
-          hi = (int)h;
-        }
-        for (int o = 32; o > 0; o >>= 1) {
-          lo = min(lo, __shfl_xor(lo, o, 64));
-          hi = max(hi, __shfl_xor(hi, o, 64));
-        }
-        if ((tid & 63) == 0 && j < nseg) P.segChunk[(sBase + j) >> 6] = make_int2(lo, hi);
-      }
-    }
-  }
+  for (int c = (int)threadIdx.x; c < n; c += (int)blockDim.x) P.strokeChunk[sChunk + c] = make_int2(it, 0);
 }
 
 // Thread per command of the calls of more than kBlock commands (the first
@@ -557,11 +549,10 @@ __device__ __forceinline__ Bounds block_bounds256(Bounds bd, Bounds* sBd) {
 }
 
 // Prefixes over the big calls: subpath chunks of every call (what = 2),
-// point chunks of the fills whose points were laid out (what = 0), and
-// 64-segment groups of the fills that draw (what = 1).
+// and point chunks of the fills whose points were laid out (what = 0).
 __global__ void __launch_bounds__(kScanBlock) scene_big_plan_kernel(ScenePools P, int what) {
   __shared__ int sh[kScanBlock / 64];
-  int32_t* out = what == 2 ? P.bigPolyStart : what == 1 ? P.bigGroupStart : P.bigChunkStart;
+  int32_t* out = what == 2 ? P.bigPolyStart : P.bigChunkStart;
   int carry = 0;
   for (int i0 = 0; i0 < P.nBig; i0 += kScanBlock) {
     const int i = i0 + threadIdx.x;
@@ -572,10 +563,7 @@ __global__ void __launch_bounds__(kScanBlock) scene_big_plan_kernel(ScenePools P
         n = (P.items[it].polyCount + kBigPolyChunk - 1) / kBigPolyChunk;
       } else {
         const ItemGeom g = P.geo[it];
-        if (!P.items[it].stroke && g.status == kOk) {
-          if (what == 0) n = (g.ptCount + kBigChunk - 1) / kBigChunk;
-          else if (P.fills[it].pathWidth > 0) n = (g.segCount + 63) / 64;
-        }
+        if (!P.items[it].stroke && g.status == kOk) n = (g.ptCount + kBigChunk - 1) / kBigChunk;
       }
     }
     int t;
@@ -714,31 +702,36 @@ __global__ void __launch_bounds__(256) scene_big_front_alloc_kernel(ScenePools P
   for (int o = 32; o > 0; o >>= 1) err = max(err, __shfl_xor(err, o, 64));
   if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = err;
   __syncthreads();
-  if (threadIdx.x != 0) return;
   err = max(max(sh[0], sh[1]), max(sh[2], sh[3]));
   const int total = carry;
-  int base = 0;
-  if (err == kOk) {
-    base = atomicAdd(&P.counters[kCntPoints], total);
-    if (base + total > P.ptCap) {
-      atomicOr(&P.counters[kCntError], 1);
-      err = kErrCapacity;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int base = 0;
+    if (err == kOk) {
+      base = atomicAdd(&P.counters[kCntPoints], total);
+      if (base + total > P.ptCap) {
+        atomicOr(&P.counters[kCntError], 1);
+        err = kErrCapacity;
+      }
+      // strokeShapes checks the dash values once it meets a shape with
+      // points (paths.nim:2029-2031)
+      if (I.stroke && !I.strokeNone && I.dashBad && total > 0 && err == kOk) err = kErrDash;
     }
-    // strokeShapes checks the dash values once it meets a shape with
-    // points (paths.nim:2029-2031)
-    if (I.stroke && !I.strokeNone && I.dashBad && total > 0 && err == kOk) err = kErrDash;
+    ItemGeom g = {};
+    if (err != kOk) {
+      g.status = err;
+      P.fills[it].status = err;
+      P.fills[it].pathWidth = 0;
+    } else {
+      g.ptBase = base;
+      g.ptCount = total;
+      g.status = kOk;
+    }
+    P.geo[it] = g;
+    sh[0] = err;
   }
-  ItemGeom g = {};
-  if (err != kOk) {
-    g.status = err;
-    P.fills[it].status = err;
-    P.fills[it].pathWidth = 0;
-  } else {
-    g.ptBase = base;
-    g.ptCount = total;
-    g.status = kOk;
-  }
-  P.geo[it] = g;
+  __syncthreads();
+  if (I.stroke) stroke_register(P, I, it, sh[0] == kOk ? total : 0);
 }
 
 // Segments and bounds of each chunk (emit = 0), or its segments written at
@@ -829,76 +822,204 @@ __global__ void __launch_bounds__(256) scene_big_seg_alloc_kernel(ScenePools P) 
     __syncthreads();
   }
   const Bounds b = block_bounds256(bd, sBd);
-  if (threadIdx.x != 0) return;
   const int nseg = carry;
-  // segments start on a 64-segment chunk of their own
-  const int base = atomicAdd(&P.counters[kCntSegs], (nseg + 63) & ~63);
-  FillInfo f = {};
-  f.rgbx = I.rgbx;
-  f.mode = I.mode;
-  f.rule = I.rule;
-  if (base + nseg > P.segCap) {
-    atomicOr(&P.counters[kCntError], 1);
-    f.status = kErrCapacity;
-    f.pathWidth = 0;
-    g.segBase = 0;
-    g.segCount = 0;
-    g.status = kErrCapacity;
-  } else {
-    const int32_t r = fill_locals(b, false, P.W, P.H, &f);
-    f.status = r;
-    if (r == kOk && f.pathWidth > 0) band_layout(&f, nseg);
-    g.segBase = base;
-    g.segCount = nseg;
-    g.status = r;
+  if (threadIdx.x == 0) {
+    // segments start on a 64-segment group of their own
+    const int base = atomicAdd(&P.counters[kCntSegs], (nseg + 63) & ~63);
+    FillInfo f = {};
+    f.rgbx = I.rgbx;
+    f.mode = I.mode;
+    f.rule = I.rule;
+    if (base + nseg > P.segCap) {
+      atomicOr(&P.counters[kCntError], 1);
+      f.status = kErrCapacity;
+      f.pathWidth = 0;
+      g.segBase = 0;
+      g.segCount = 0;
+      g.status = kErrCapacity;
+    } else {
+      const int32_t r = fill_locals(b, false, P.W, P.H, &f);
+      f.status = r;
+      if (r == kOk && f.pathWidth > 0) band_layout(&f, nseg);
+      g.segBase = base;
+      g.segCount = nseg;
+      g.status = r;
+    }
+    P.fills[it] = f;
+    P.geo[it] = g;
+    sh[0] = g.status == kErrCapacity ? -1 : base;
   }
-  P.fills[it] = f;
-  P.geo[it] = g;
+  __syncthreads();
+  if (sh[0] >= 0) mark_groups(P, it, sh[0], nseg);
 }
 
-// Stage 7 of the big fills: one wave per 64-segment group.
-__global__ void __launch_bounds__(256) scene_big_band_kernel(ScenePools P) {
-  const int nGroups = P.bigGroupStart[P.nBig];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  for (int gi = blockIdx.x * 4 + wave; gi < nGroups; gi += gridDim.x * 4) {
-    const int bi = big_call_of(P.bigGroupStart, P.nBig, gi);
-    const int it = P.itemOrder[bi];
+// ---- strokes, spread over the device (stages 5-6) ----
+// A stroke makes tens of segments per point (a round join flattens a circle),
+// and segments keep point order.  Its points are cut into chunks of 256 lanes
+// (64 points of four lanes, or 256 of one): the chunks count their segments,
+// one workgroup per stroke scans the counts and allocates, and the chunks
+// write theirs and merge their bounds.  In one workgroup per stroke these
+// stages were the tail of the whole geometry: 630 of the 800 thousand cycles
+// of the longest call (1,303 points, 26,038 segments) of 100 paths on
+// 1,023 x 767, whose geometry took 340 us and now takes 73 + 9 + 7 + 13.
+
+// Order-preserving map of a non-NaN float to an unsigned, for atomic bounds.
+__device__ __forceinline__ uint32_t bound_key(float f) {
+  const uint32_t u = __float_as_uint(f);
+  return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+}
+__device__ __forceinline__ float bound_value(uint32_t k) {
+  return __uint_as_float((k & 0x80000000u) ? (k & 0x7fffffffu) : ~k);
+}
+
+// Without kEmit: the segments of every chunk; with it: the segments written,
+// and the bounds.
+template <bool kEmit>
+__global__ void __launch_bounds__(256) scene_stroke_kernel(ScenePools P) {
+  __shared__ int sh[4];
+  __shared__ Bounds sBd[4];
+  if (P.counters[kCntError]) return;
+  const int nChunks = P.counters[kCntStrokeChunks];
+  for (int c = blockIdx.x; c < nChunks; c += gridDim.x) {
+    const int2 ch = P.strokeChunk[c];
+    const int it = ch.x;
+    const SceneItem& I = P.items[it];
     const ItemGeom g = P.geo[it];
-    const FillInfo fl = P.fills[it];
-    const int j = (gi - P.bigGroupStart[bi]) * 64 + lane;
-    int lo = 0x7fffffff, hi = -1;
-    if (j < g.segCount) {
-      const float4 sg = P.segs[g.segBase + j];
-      uint32_t l = 0, h = 0;
-      if (fl.nParts > 1)
-        partition_range(sg.y, sg.w, (uint32_t)fl.startY, (uint32_t)fl.bandH, (uint32_t)fl.nParts, &l, &h);
-      const bool aa = seg_requires_aa(v2(sg.x, sg.y), v2(sg.z, sg.w));
-      P.segBand[g.segBase + j] = make_int2((int)l, (int)h | (aa ? kSegAA : 0));
-      lo = (int)l;
-      hi = (int)h;
+    if (kEmit && g.status != kOk) continue;  // the same for the whole block
+    const int lanes = stroke_lanes(I), sub = (int)threadIdx.x % lanes;
+    const int j = (c - P.strokes[it].chunkBase) * (256 / lanes) + (int)threadIdx.x / lanes;
+    const float2* pts = P.pts + g.ptBase;
+    int n = 0, pb = 0, np = 0;
+    int32_t err = 0;
+    if (j < g.ptCount) {
+      const int q = I.polyBase + P.ptPoly[g.ptBase + j];
+      pb = P.polyPt[q];
+      np = P.polyN[q];
+      // a lane of four keeps up to 254 of its segments in its byte of ptSeg
+      // (255: counted again); a point of one lane has the whole word
+      if (kEmit) {
+        const uint32_t w = (uint32_t)P.ptSeg[g.ptBase + j];
+        n = lanes == 1 ? (int)w : (int)((w >> (8 * sub)) & 255u);
+      }
+      if (!kEmit || (lanes > 1 && n == 255)) {
+        SegSink sink;
+        stroke_point(pts + pb, j - pb, np, I, P.dashes + I.dashBase, sink, sub, lanes);
+        n = sink.n;
+        err = sink.err;
+      }
     }
-    for (int o = 32; o > 0; o >>= 1) {
-      lo = min(lo, __shfl_xor(lo, o, 64));
-      hi = max(hi, __shfl_xor(hi, o, 64));
+    if (!kEmit) {
+      if (err) atomicMax(&P.strokes[it].err, (int32_t)kErrCapacity);
+      uint32_t w = (uint32_t)n;
+      if (lanes > 1) {  // the same for the whole block
+        w = (uint32_t)(n < 255 ? n : 255) << (8 * sub);
+        w |= (uint32_t)__shfl_xor((int)w, 1, 64);
+        w |= (uint32_t)__shfl_xor((int)w, 2, 64);
+      }
+      if (sub == 0 && j < g.ptCount) P.ptSeg[g.ptBase + j] = (int32_t)w;
     }
-    if (lane == 0) P.segChunk[(g.segBase + j) >> 6] = make_int2(lo, hi);
+    int t;
+    const int off = block_excl_scan_n<256>(n, &t, sh);
+    if (!kEmit) {
+      if (threadIdx.x == 0) P.strokeChunk[c].y = t;
+    } else {
+      SegSink out;
+      out.bd = bounds_init();
+      if (n > 0) {
+        const int w = g.segBase + ch.y + off;
+        out.out = P.segs + w;
+        out.outW = P.segW + w;
+        stroke_point(pts + pb, j - pb, np, I, P.dashes + I.dashBase, out, sub, lanes);
+      }
+      const Bounds b = block_bounds256(out.bd, sBd);
+      if (threadIdx.x == 0 && t > 0) {
+        uint32_t* const bd = P.strokes[it].bd;
+        atomicMin(&bd[0], bound_key(b.xMin));
+        atomicMax(&bd[1], bound_key(b.xMax));
+        atomicMin(&bd[2], bound_key(b.yMin));
+        atomicMax(&bd[3], bound_key(b.yMax));
+      }
+    }
+    __syncthreads();
   }
 }
 
-// Geometry kernel stages by MODE: kGeomAll runs every stage for a call.
-// Calls of more than kBlock commands spread their stages over the CUs:
-// scene_big_cmd_kernel counts every command's points, scene_big_front_*
-// lay the points out (stages 2-3), scene_big_cmd_kernel emits them, and the
-// segment stages run in scene_big_seg_* / scene_big_band_kernel for fills
-// and in one kGeomBack workgroup per call for strokes (stages 5-7).
-constexpr int kGeomAll = 0, kGeomBack = 2;
+// One workgroup per stroke: scans its chunk counts and allocates its segments.
+__global__ void __launch_bounds__(256) scene_stroke_alloc_kernel(ScenePools P) {
+  __shared__ int sh[4];
+  __shared__ int sBase;
+  const int it = P.strokeItems[blockIdx.x];
+  const SceneItem& I = P.items[it];
+  ItemGeom g = P.geo[it];
+  if (g.status != kOk) return;  // the point layout wrote the error
+  const int chunkBase = P.strokes[it].chunkBase, nChunks = P.strokes[it].nChunks;
+  int carry = 0;
+  for (int k0 = 0; k0 < nChunks; k0 += 256) {
+    const int k = k0 + threadIdx.x;
+    const int n = k < nChunks ? P.strokeChunk[chunkBase + k].y : 0;
+    int t;
+    const int off = block_excl_scan_n<256>(n, &t, sh);
+    if (k < nChunks) P.strokeChunk[chunkBase + k].y = carry + off;
+    carry += t;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    int32_t status = P.strokes[it].err;
+    int base = 0;
+    if (status == kOk) {
+      // segments start on a 64-segment group of their own
+      base = atomicAdd(&P.counters[kCntSegs], (carry + 63) & ~63);
+      if (base + carry > P.segCap) {
+        atomicOr(&P.counters[kCntError], 1);
+        status = kErrCapacity;
+      }
+    }
+    const Bounds b = bounds_init();
+    uint32_t* const bd = P.strokes[it].bd;
+    bd[0] = bound_key(b.xMin);
+    bd[1] = bound_key(b.xMax);
+    bd[2] = bound_key(b.yMin);
+    bd[3] = bound_key(b.yMax);
+    g.segBase = status == kOk ? base : 0;
+    g.segCount = status == kOk ? carry : 0;
+    g.status = status;
+    P.geo[it] = g;
+    // the band-range stage writes the fill of a stroke that has segments
+    FillInfo f = {};
+    f.rgbx = I.rgbx;
+    f.mode = I.mode;
+    f.rule = kNonZero;
+    f.status = status != kOk ? status : fill_locals(b, false, P.W, P.H, &f);
+    P.fills[it] = f;
+    sBase = status == kOk ? base : -1;
+  }
+  __syncthreads();
+  if (sBase >= 0) mark_groups(P, it, sBase, carry);
+}
 
-template <int NB, int MODE>
-__global__ void __launch_bounds__(NB) scene_geom_kernel(ScenePools P, int orderBase) {
+// A stroke's fill from its merged bounds (stage 6).
+__device__ __forceinline__ void stroke_fill(const ScenePools& P, int it, int segCount, FillInfo* f) {
+  const uint32_t* bd = P.strokes[it].bd;
+  Bounds b;
+  b.xMin = bound_value(bd[0]);
+  b.xMax = bound_value(bd[1]);
+  b.yMin = bound_value(bd[2]);
+  b.yMax = bound_value(bd[3]);
+  f->status = fill_locals(b, false, P.W, P.H, f);
+  if (f->status == kOk && f->pathWidth > 0) band_layout(f, segCount);
+}
+
+// Geometry of a call of at most kBlock commands, one workgroup per call: a
+// fill's stages 1-6; a stroke ends here with its points (scene_stroke_*).
+// The other calls spread their stages over the CUs: scene_big_cmd_kernel
+// counts every command's points, scene_big_front_* lay the points out (stages
+// 2-3), scene_big_cmd_kernel emits them, and scene_big_seg_* make the
+// segments of fills.
+__global__ void __launch_bounds__(kBlock) scene_geom_kernel(ScenePools P, int orderBase) {
+  constexpr int NB = kBlock;
   __shared__ int sh[NB / 64];
   __shared__ int sBase;
   __shared__ Bounds sBd[NB / 64];
-  __shared__ FillInfo sF;
   __shared__ int sErr;
   __shared__ float2 sPts[kStagePts];
   __shared__ int sPre[NB + 1];
@@ -909,27 +1030,17 @@ __global__ void __launch_bounds__(NB) scene_geom_kernel(ScenePools P, int orderB
   if (tid == 0) sErr = kOk;
   __syncthreads();
 
-  int total = 0, ptBase = 0;
-  if (MODE == kGeomBack) {
-    const ItemGeom gf = P.geo[it];
-    if (gf.status != kOk) return;  // the front wrote the error
-    if (!I.stroke) return;         // big fills: scene_big_seg_* kernels
-    total = gf.ptCount;
-    ptBase = gf.ptBase;
-    goto segments;
-  }
-  {
-  // 1. points per command.  A call of at most NB commands keeps each
-  // command's points in an LDS slice of its own (thread tid <-> command tid
-  // in stages 1 and 4), so stage 4 copies them unless a slice overflowed.
-  const bool stage = I.cmdCount <= NB;
-  const int slice = stage && I.cmdCount > 0 ? kStagePts / I.cmdCount : 0;
+  int total = 0;
+  // 1. points per command, kept in an LDS slice per command (thread tid <->
+  // command tid in stages 1 and 4), so that stage 4 copies them unless a
+  // slice overflowed.  Few commands take 8, 4 or 2 lanes each, so that a
+  // cubic's adaptive steps are tried that many halvings at a time.
+  const int slice = I.cmdCount > 0 ? kStagePts / I.cmdCount : 0;
   bool staged = false;
   int myN = 0;
-  if (stage && I.cmdCount <= NB / kFlatGroup) {
-    // few commands: kFlatGroup lanes per command, so a cubic's adaptive
-    // steps are tried kFlatGroup halvings at a time
-    const int c = tid / kFlatGroup, u = tid % kFlatGroup;
+  auto group = [&](auto lanesPer) {
+    constexpr int G = decltype(lanesPer)::value;
+    const int c = tid / G, u = tid % G;
     if (c < I.cmdCount) {
       const int i = I.cmdBase + c;
       StageEmit se{sPts + c * slice, slice, I.mat, xf};
@@ -937,8 +1048,8 @@ __global__ void __launch_bounds__(NB) scene_geom_kernel(ScenePools P, int orderB
       int32_t r;
       const SceneCmd& cm = P.cmds[i];
       if ((int)cm.kind == 5)
-        r = flatten_cubic_group(cmd_end(P.cmds[i - 1]), v2(cm.p[0], cm.p[1]), v2(cm.p[2], cm.p[3]),
-                                v2(cm.p[4], cm.p[5]), I.errSq, se, u, tid & 63 & ~(kFlatGroup - 1));
+        r = flatten_cubic_group<G>(cmd_end(P.cmds[i - 1]), v2(cm.p[0], cm.p[1]), v2(cm.p[2], cm.p[3]),
+                                   v2(cm.p[4], cm.p[5]), I.errSq, se, u, tid & 63 & ~(G - 1));
       else
         r = cmd_emit(P.cmds, i, I.errSq, se);
       if (u == 0) {
@@ -952,24 +1063,27 @@ __global__ void __launch_bounds__(NB) scene_geom_kernel(ScenePools P, int orderB
       myN = sPre[tid];
       staged = myN <= slice;
     }
-  } else if (MODE == kGeomAll) {
-    for (int c0 = 0; c0 < I.cmdCount; c0 += NB) {
-      int i = I.cmdBase + c0 + tid;
-      if (c0 + tid < I.cmdCount) {
-        StageEmit se{sPts + tid * slice, slice, I.mat, xf};
-        int32_t r = cmd_emit(P.cmds, i, I.errSq, se);
-        if (r != kOk) atomicMax(&sErr, r);
-        P.cmdCount[i] = se.n;
-        myN = se.n;
-        staged = stage && se.n <= slice;
-      }
-    }
+  };
+  if (I.cmdCount <= NB / 8) {
+    group(Lanes<8>{});
+  } else if (I.cmdCount <= NB / 4) {
+    group(Lanes<4>{});
+  } else if (I.cmdCount <= NB / 2) {
+    group(Lanes<2>{});
+  } else if (tid < I.cmdCount) {
+    const int i = I.cmdBase + tid;
+    StageEmit se{sPts + tid * slice, slice, I.mat, xf};
+    const int32_t r = cmd_emit(P.cmds, i, I.errSq, se);
+    if (r != kOk) atomicMax(&sErr, r);
+    P.cmdCount[i] = se.n;
+    myN = se.n;
+    staged = se.n <= slice;
   }
   __syncthreads();
-  // With one command per thread: points before each command of the call
-  // (sPre[c], and the total in sPre[cmdCount]), so that subpath sums and
-  // command offsets take two LDS reads instead of a loop over commands.
-  if (stage) {
+  // Points before each command of the call (sPre[c], and the total in
+  // sPre[cmdCount]), so that subpath sums and command offsets take two LDS
+  // reads instead of a loop over commands.
+  {
     int tot;
     const int pre = block_excl_scan_n<NB>(tid < I.cmdCount ? myN : 0, &tot, sh);
     if (tid < I.cmdCount) sPre[tid] = pre;
@@ -982,13 +1096,8 @@ __global__ void __launch_bounds__(NB) scene_geom_kernel(ScenePools P, int orderB
     int np = 0;
     if (q0 + tid < I.polyCount) {
       ScenePoly sp = P.polys[q];
-      int n = 0;
-      if (stage) {
-        const int cl = sp.firstCmd - I.cmdBase;
-        n = sPre[cl + sp.numCmds] - sPre[cl];
-      } else {
-        for (int c = 0; c < sp.numCmds; c++) n += P.cmdCount[sp.firstCmd + c];
-      }
+      const int cl = sp.firstCmd - I.cmdBase;
+      const int n = sPre[cl + sp.numCmds] - sPre[cl];
       if (n > 0) {
         np = n + 1;
         const SceneCmd& last = P.cmds[sp.firstCmd + sp.numCmds - 1];
@@ -1018,7 +1127,8 @@ __global__ void __launch_bounds__(NB) scene_geom_kernel(ScenePools P, int orderB
     sBase = base;
   }
   __syncthreads();
-  ptBase = sBase;
+  const int ptBase = sBase;
+  if (I.stroke) stroke_register(P, I, it, sErr == kOk ? total : 0);
   if (sErr != kOk) {
     if (tid == 0) {
       P.geo[it].status = sErr;
@@ -1030,9 +1140,8 @@ __global__ void __launch_bounds__(NB) scene_geom_kernel(ScenePools P, int orderB
   }
   float2* pts = P.pts + ptBase;
   int32_t* ptPoly = P.ptPoly + ptBase;
-  int32_t* ptSeg = P.ptSeg + ptBase;  // segments of each point (stage 5)
 
-  // 3. per-command point offsets, start and closing points (thread per subpath)
+  // 3. start and closing points (thread per subpath)
   for (int q0 = 0; q0 < I.polyCount; q0 += NB) {
     int ql = q0 + tid;
     if (ql < I.polyCount) {
@@ -1040,15 +1149,8 @@ __global__ void __launch_bounds__(NB) scene_geom_kernel(ScenePools P, int orderB
       ScenePoly sp = P.polys[q];
       int np = P.polyN[q], pb = P.polyPt[q];
       int off = pb + 1;
-      if (stage) {  // stage 4 derives each command's offset from sPre
-        const int cl = sp.firstCmd - I.cmdBase;
-        off += sPre[cl + sp.numCmds] - sPre[cl];
-      } else {
-        for (int c = 0; c < sp.numCmds; c++) {
-          P.cmdOff[sp.firstCmd + c] = off;
-          off += P.cmdCount[sp.firstCmd + c];
-        }
-      }
+      const int cl = sp.firstCmd - I.cmdBase;  // stage 4 derives each command's offset from sPre
+      off += sPre[cl + sp.numCmds] - sPre[cl];
       if (np > 0) {
         const SceneCmd& mv = P.cmds[sp.firstCmd];
         V2 s = v2(mv.sx, mv.sy);
@@ -1064,46 +1166,30 @@ __global__ void __launch_bounds__(NB) scene_geom_kernel(ScenePools P, int orderB
   }
   __syncthreads();
   // 4. emit points (thread per command)
-  for (int c0 = 0; c0 < I.cmdCount; c0 += NB) {
-    int i = I.cmdBase + c0 + tid;
-    if (c0 + tid < I.cmdCount && P.cmdCount[i] > 0) {
-      // subpath of command i (the host stores it in pad[0] of every command)
-      int ql = P.cmds[i].pad[0];
-      int o;
-      if (stage) {
-        const int q = I.polyBase + ql;
-        o = P.polyPt[q] + 1 + sPre[c0 + tid] - sPre[P.polys[q].firstCmd - I.cmdBase];
-      } else {
-        o = P.cmdOff[i];
+  if (tid < I.cmdCount && myN > 0) {
+    const int i = I.cmdBase + tid;
+    // subpath of command i (the host stores it in pad[0] of every command)
+    const int ql = P.cmds[i].pad[0], q = I.polyBase + ql;
+    const int o = P.polyPt[q] + 1 + sPre[tid] - sPre[P.polys[q].firstCmd - I.cmdBase];
+    if (staged) {
+      const float2* src = sPts + tid * slice;
+      for (int k = 0; k < myN; k++) {
+        pts[o + k] = src[k];
+        ptPoly[o + k] = ql;
       }
-      if (staged) {
-        const int n = P.cmdCount[i];
-        const float2* src = sPts + tid * slice;
-        for (int k = 0; k < n; k++) {
-          pts[o + k] = src[k];
-          ptPoly[o + k] = ql;
-        }
-      } else {
-        StoreEmit se{pts + o, ptPoly + o, ql, I.mat, xf};
-        cmd_emit(P.cmds, i, I.errSq, se);
-      }
+    } else {
+      StoreEmit se{pts + o, ptPoly + o, ql, I.mat, xf};
+      cmd_emit(P.cmds, i, I.errSq, se);
     }
   }
   __syncthreads();
-  }
-segments:
-  float2* pts = P.pts + ptBase;
-  int32_t* ptPoly = P.ptPoly + ptBase;
-  int32_t* ptSeg = P.ptSeg + ptBase;  // segments of each point (stage 5)
 
-  // 5. segments: count, allocate, emit (thread per point).  A fill makes at
-  // most one segment per point, so it allocates that bound and emits in one
-  // pass; a stroke counts first.
+  // 5. segments of a fill, thread per point: it makes at most one per point,
+  // so it allocates that bound and emits in one pass
   int nseg = 0;
-  const bool onePass = !I.stroke;
-  if (onePass) {
+  if (!I.stroke) {
     if (tid == 0) {
-      // segments start on a 64-segment chunk of their own
+      // segments start on a 64-segment group of their own
       int base = atomicAdd(&P.counters[kCntSegs], (total + 63) & ~63);
       if (base + total > P.segCap) {
         atomicOr(&P.counters[kCntError], 1);
@@ -1149,67 +1235,18 @@ segments:
         segOff += t;
       }
       nseg = segOff;
-      geom_finish<NB>(P, I, it, bd, nseg, sBase, sBd, sF);
-    }
-  } else {
-    // a stroke: count the segments of every point, allocate, then emit
-    for (int pass = 0; pass < 2 && sErr == kOk; pass++) {
-      int segOff = 0;
-      Bounds bd = bounds_init();
-      for (int j0 = 0; j0 < total; j0 += NB) {
-        int j = j0 + tid;
-        int cnt = 0;
-        if (pass == 1) {
-          // the counts of pass 0 (this thread wrote them)
-          if (j < total) cnt = ptSeg[j];
-        } else if (j < total && !I.strokeNone) {
-          int q = I.polyBase + ptPoly[j];
-          int pb = P.polyPt[q], np = P.polyN[q];
-          SegSink sink;
-          stroke_point(pts + pb, j - pb, np, I, P.dashes + I.dashBase, sink);
-          cnt = sink.n;
-          if (sink.err) atomicMax(&sErr, kErrCapacity);
-        }
-        if (pass == 0 && j < total) ptSeg[j] = cnt;
-        int t;
-        int off = block_excl_scan_n<NB>(cnt, &t, sh);
-        if (pass == 1 && j < total && cnt > 0) {
-          SegSink out;
-          out.out = P.segs + sBase + segOff + off;
-          out.outW = P.segW + sBase + segOff + off;
-          out.bd = bd;
-          int q = I.polyBase + ptPoly[j];
-          int pb = P.polyPt[q], np = P.polyN[q];
-          stroke_point(pts + pb, j - pb, np, I, P.dashes + I.dashBase, out);
-          bd = out.bd;
-        }
-        segOff += t;
-      }
-      if (pass == 0) {
-        nseg = segOff;
-        __syncthreads();
-        if (tid == 0) {
-          // segments start on a 64-segment chunk of their own
-          int base = atomicAdd(&P.counters[kCntSegs], (nseg + 63) & ~63);
-          if (base + nseg > P.segCap) {
-            atomicOr(&P.counters[kCntError], 1);
-            sErr = kErrCapacity;
-          }
-          sBase = base;
-        }
-        __syncthreads();
-      } else {
-        geom_finish<NB>(P, I, it, bd, nseg, sBase, sBd, sF);
-      }
+      geom_finish<NB>(P, I, it, bd, nseg, sBd);
+      mark_groups(P, it, sBase, total);
     }
   }
   if (tid == 0) {
+    const bool segs = !I.stroke && sErr == kOk;
     ItemGeom g = {};
     g.ptBase = ptBase;
     g.ptCount = total;
-    g.segBase = sErr == kOk ? sBase : 0;
-    g.segCount = sErr == kOk ? nseg : 0;
-    g.status = sErr != kOk ? sErr : P.fills[it].status;
+    g.segBase = segs ? sBase : 0;
+    g.segCount = segs ? nseg : 0;
+    g.status = sErr != kOk ? sErr : (I.stroke ? (int32_t)kOk : P.fills[it].status);
     if (sErr != kOk) {
       P.fills[it].status = sErr;
       P.fills[it].pathWidth = 0;
@@ -1219,21 +1256,31 @@ segments:
 }
 
 // ---------------------------------------------------------------------------
-// planning (one block): bands, phase-A tasks, band -> call map
+// planning: each call's bands, phase-A tasks and work-item chunks
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(kScanBlock) scene_plan_kernel(ScenePools P) {
-  __shared__ int sh[kScanBlock / 64];
-  const int tid = threadIdx.x;
-  int bandTot = 0, taskTot = 0;
-  for (int i0 = 0; i0 < P.nItems; i0 += kScanBlock) {
-    int it = i0 + tid;
-    int nb = 0, nt = 0;
-    ItemGeom g;
-    FillInfo f;
+// 64 calls per workgroup: wave 0 lays them out (one atomic per workgroup and
+// pool: where a call's bands and tasks lie does not matter, only that they
+// are consecutive), then all four waves write the band -> call and
+// chunk -> call maps.
+constexpr int kPlanCalls = 64;
+__device__ void plan_calls(const ScenePools& P, int block) {
+  __shared__ int sBand[kPlanCalls], sBands[kPlanCalls], sChunk[kPlanCalls], sChunks[kPlanCalls];
+  const int lane = threadIdx.x & 63, wave = uni((int)threadIdx.x >> 6);
+  const int it0 = block * kPlanCalls;
+  if (wave == 0) {
+    const int it = it0 + lane;
+    int nb = 0, nt = 0, nc = 0;
+    ItemGeom g = {};
+    FillInfo f = {};
     int4 rows = make_int4(0, 0, 0, 0);
     if (it < P.nItems) {
       g = P.geo[it];
       f = P.fills[it];
+      if (P.items[it].stroke && g.status == kOk && g.segCount > 0) {
+        stroke_fill(P, it, g.segCount, &f);
+        g.status = f.status;
+        P.fills[it] = f;
+      }
       g.rowStart = 0;
       g.rowCount = 0;
       g.nWin = 0;
@@ -1247,31 +1294,101 @@ __global__ void __launch_bounds__(kScanBlock) scene_plan_kernel(ScenePools P) {
         g.winBase = lo;
         g.nWin = hi > lo ? (hi - lo + kWinA - 1) / kWinA : 0;
         nt = g.rowCount * g.nWin;
+        nc = ((g.rowCount + kRowGroup - 1) / kRowGroup * g.nWin + 63) / 64;
         // a mask call touches every row (it clears the rows outside it)
         rows = f.mode == kMask ? make_int4(0, P.H, 0, P.W)
                                : make_int4(g.rowStart, g.rowStart + g.rowCount, f.xlo, f.xhi);
       }
       P.itemRows[it] = rows;
     }
-    int tb, tt;
-    int bOff = block_excl_scan_n<kScanBlock>(nb, &tb, sh);
-    int tOff = block_excl_scan_n<kScanBlock>(nt, &tt, sh);
+    int tb, tt, tc;
+    const int bOff = wave_excl_scan(nb, &tb), tOff = wave_excl_scan(nt, &tt), cOff = wave_excl_scan(nc, &tc);
+    int bBase = 0, tBase = 0, cBase = 0;
+    if (lane == 0) {
+      bBase = atomicAdd(&P.counters[kCntBands], tb);
+      tBase = atomicAdd(&P.counters[kCntTasks], tt);
+      cBase = atomicAdd(&P.counters[kCntChunks], tc);
+    }
+    bBase = uni(bBase);
+    tBase = uni(tBase);
+    cBase = uni(cBase);
+    const bool fits = bBase + tb <= P.bandCap && tBase + tt <= P.taskCap &&
+                      cBase + tc <= P.taskCap / 64 + P.nItems + 1;
+    if (!fits && lane == 0) atomicOr(&P.counters[kCntError], 2);
     if (it < P.nItems) {
-      g.bandBase = bandTot + bOff;
-      g.taskBase = taskTot + tOff;
-      P.geo[it] = g;
+      g.bandBase = bBase + bOff;
+      g.taskBase = tBase + tOff;
+      ItemGeom* const o = &P.geo[it];  // not its segments, which the band ranges read meanwhile
+      o->bandBase = g.bandBase;
+      o->rowStart = g.rowStart;
+      o->rowCount = g.rowCount;
+      o->winBase = g.winBase;
+      o->nWin = g.nWin;
+      o->taskBase = g.taskBase;
+      o->status = g.status;
       // compact per-call record for phase B
       P.itemPaint[it] = make_int4((int)f.rgbx, f.mode, g.taskBase, g.nWin);
       P.itemSpan[it] = make_int4(g.rowStart, g.rowCount, f.xlo, f.xhi);
     }
-    bandTot += tb;
-    taskTot += tt;
+    sBand[lane] = bBase + bOff;
+    sBands[lane] = fits ? nb : 0;
+    sChunk[lane] = cBase + cOff;
+    sChunks[lane] = fits ? nc : 0;
   }
-  if (tid == 0) {
-    P.counters[kCntBands] = bandTot;
-    P.counters[kCntTasks] = taskTot;
-    if (bandTot > P.bandCap || taskTot > P.taskCap) atomicOr(&P.counters[kCntError], 2);
+  __syncthreads();
+  for (int c = wave; c < kPlanCalls; c += 4) {
+    const int b0 = uni(sBand[c]), nb = uni(sBands[c]), c0 = uni(sChunk[c]), nc = uni(sChunks[c]);
+    for (int b = lane; b < nb; b += 64) P.bandItem[b0 + b] = it0 + c;
+    for (int k = lane; k < nc; k += 64) P.taskChunk[c0 + k] = make_int2(it0 + c, k);
   }
+}
+
+// Stage 7 of every call: one wave per 64-segment group finds the band range
+// of each segment (partitionSegments 1201-1213), its requiresAntiAliasing bit
+// and the band range of the group.
+__device__ void seg_bands(const ScenePools& P, int block, int blocks) {
+  const int nGroups = P.counters[kCntSegs] >> 6;
+  const int wave = uni((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+  for (int gi = block * 4 + wave; gi < nGroups; gi += blocks * 4) {
+    const int it = uni(P.groupItem[gi]);
+    const int segBase = uni(P.geo[it].segBase), segCount = uni(P.geo[it].segCount);
+    FillInfo f = {};
+    if (P.items[it].stroke) {
+      stroke_fill(P, it, segCount, &f);
+    } else {
+      const FillInfo& F = P.fills[it];
+      f.status = F.status;
+      f.pathWidth = F.pathWidth;
+      f.startY = F.startY;
+      f.nParts = F.nParts;
+      f.bandH = F.bandH;
+    }
+    const int j = gi * 64 + lane - segBase;
+    int lo = 0x7fffffff, hi = -1;
+    if (j < segCount && f.status == kOk && f.pathWidth > 0) {
+      const float4 sg = P.segs[segBase + j];
+      uint32_t l = 0, h = 0;
+      if (f.nParts > 1)
+        partition_range(sg.y, sg.w, (uint32_t)f.startY, (uint32_t)f.bandH, (uint32_t)f.nParts, &l, &h);
+      const bool aa = seg_requires_aa(v2(sg.x, sg.y), v2(sg.z, sg.w));
+      P.segBand[segBase + j] = make_int2((int)l, (int)h | (aa ? kSegAA : 0));
+      lo = (int)l;
+      hi = (int)h;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      lo = min(lo, __shfl_xor(lo, o, 64));
+      hi = max(hi, __shfl_xor(hi, o, 64));
+    }
+    if (lane == 0) P.segChunk[gi] = make_int2(lo, hi);
+  }
+}
+
+// The plan and the band ranges need the same inputs and not each other.
+__global__ void __launch_bounds__(256) scene_plan_kernel(ScenePools P, int planBlocks) {
+  if ((int)blockIdx.x < planBlocks)
+    plan_calls(P, blockIdx.x);
+  else if (!(P.counters[kCntError] & 1))  // (set by earlier kernels only)
+    seg_bands(P, (int)blockIdx.x - planBlocks, (int)gridDim.x - planBlocks);
 }
 
 // Band b of its call: top / bottom rows (partitionSegments 1183-1192).
@@ -1289,137 +1406,12 @@ constexpr int kXcds = 8;
 struct XcdSpan {
   int begin, end, step;
 };
-__device__ __forceinline__ XcdSpan xcd_span(int n) {
-  const int per = (int)gridDim.x / kXcds;
-  if (per == 0) return XcdSpan{(int)blockIdx.x, n, (int)gridDim.x};
-  const int xcd = (int)blockIdx.x % kXcds, li = (int)blockIdx.x / kXcds;
+__device__ __forceinline__ XcdSpan xcd_span(int n, int block, int blocks) {
+  const int per = blocks / kXcds;
+  if (per == 0) return XcdSpan{block, n, blocks};
+  const int xcd = block % kXcds, li = block / kXcds;
   if (li >= per) return XcdSpan{0, 0, 1};  // beyond the last full round of XCDs
   return XcdSpan{(int)((int64_t)n * xcd / kXcds) + li, (int)((int64_t)n * (xcd + 1) / kXcds), per};
-}
-
-// One wave per band: entry count and requiresAntiAliasing.
-__global__ void __launch_bounds__(64) scene_band_count_kernel(ScenePools P) {
-  const int lane = threadIdx.x;
-  const int nb = P.counters[kCntBands];
-  if (nb > P.bandCap) return;
-  const XcdSpan sp = xcd_span(nb);
-  for (int b = sp.begin; b < sp.end; b += sp.step) {
-    const int it = uni(P.bandItem[b]);
-    ItemGeom g = P.geo[it];
-    g.bandBase = uni(g.bandBase);
-    g.segBase = uni(g.segBase);
-    g.segCount = uni(g.segCount);
-    const int k = b - g.bandBase;
-    int cnt = 0;
-    bool aa = false;
-    const int s0 = g.segBase, s1 = g.segBase + g.segCount;  // s0 is 64-aligned
-    const int cEnd = (s1 + 63) >> 6;
-    for (int cb = s0 >> 6; cb < cEnd; cb += 64) {
-      // chunks that may reach band k, 64 chunk ranges at a time
-      bool may = false;
-      if (cb + lane < cEnd) {
-        const int2 cr = P.segChunk[cb + lane];
-        may = k >= cr.x && k <= cr.y;
-      }
-      uint64_t cm = __ballot(may);
-      while (cm) {  // four candidate chunks at a time: their loads overlap
-        int2 sb[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-          sb[u] = make_int2(1, 0);  // empty band range
-          if (cm) {
-            const int j = ((cb + __builtin_ctzll(cm)) << 6) + lane;
-            cm &= cm - 1;
-            if (j < s1) sb[u] = P.segBand[j];
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-          const bool in = k >= sb[u].x && k <= (sb[u].y & ~kSegAA);
-          cnt += __popcll(__ballot(in));
-          if (__ballot(in && (sb[u].y & kSegAA))) aa = true;
-        }
-      }
-    }
-    if (lane == 0) {
-      PartInfo pi;
-      pi.entryBase = 0;
-      pi.count = cnt;
-      pi.flags = aa ? 1 : 0;
-      pi.pad = 0;
-      P.parts[b] = pi;
-    }
-  }
-}
-
-// One block: entry offsets of all bands, largest band.
-// Band -> call map (a workgroup per call, its bands across the threads).
-__global__ void __launch_bounds__(kBlock) scene_band_map_kernel(ScenePools P) {
-  const int tid = threadIdx.x;
-  for (int it = blockIdx.x; it < P.nItems; it += gridDim.x) {
-    const ItemGeom g = P.geo[it];
-    const FillInfo f = P.fills[it];
-    const int nb = (g.status == kOk && f.pathWidth > 0) ? f.nParts : 0;
-    if (g.bandBase + nb > P.bandCap) continue;
-    for (int b = tid; b < nb; b += kBlock) P.bandItem[g.bandBase + b] = it;
-  }
-}
-
-// Band-entry offsets: a scan of the band entry counts over kEntryTiles
-// contiguous tiles of bands.  1. tile sums (and the largest band).
-__device__ __forceinline__ int2 entry_tile(int nb) {
-  const int per = (nb + kEntryTiles - 1) / kEntryTiles;
-  const int lo = (int)blockIdx.x * per;
-  return make_int2(lo, lo + per < nb ? lo + per : nb);
-}
-
-__global__ void __launch_bounds__(kBlock) scene_entry_tile_kernel(ScenePools P) {
-  __shared__ int sh[kBlock / 64];
-  const int nb = P.counters[kCntBands];
-  if (nb > P.bandCap) return;
-  const int2 r = entry_tile(nb);
-  int sum = 0, mx = 0;
-  for (int b = r.x + (int)threadIdx.x; b < r.y; b += kBlock) {
-    const int c = P.parts[b].count;
-    sum += c;
-    mx = c > mx ? c : mx;
-  }
-  sum = block_sum(sum, sh);
-  mx = wave_max(mx);
-  if ((threadIdx.x & 63) == 0 && mx > 0) atomicMax(&P.counters[kCntMaxBand], mx);
-  if (threadIdx.x == 0) P.counters[kCntTileSum + blockIdx.x] = sum;
-}
-
-// 2. tile offsets (in place of the tile sums) and the entry total.
-__global__ void __launch_bounds__(kEntryTiles) scene_entry_scan_kernel(ScenePools P) {
-  __shared__ int sh[kEntryTiles / 64];
-  const int nb = P.counters[kCntBands];
-  if (nb > P.bandCap) return;
-  const int t = threadIdx.x;
-  int tot;
-  const int off = block_excl_scan_n<kEntryTiles>(P.counters[kCntTileSum + t], &tot, sh);
-  P.counters[kCntTileSum + t] = off;
-  if (t == 0) {
-    P.counters[kCntEntries] = tot;
-    if (tot > P.entryCap) atomicOr(&P.counters[kCntError], 4);
-  }
-}
-
-// 3. entry offset of every band.
-__global__ void __launch_bounds__(kBlock) scene_entry_apply_kernel(ScenePools P) {
-  __shared__ int sh[kBlock / 64];
-  const int nb = P.counters[kCntBands];
-  if (nb > P.bandCap) return;
-  const int2 r = entry_tile(nb);
-  int base = P.counters[kCntTileSum + blockIdx.x];
-  for (int b0 = r.x; b0 < r.y; b0 += kBlock) {
-    const int b = b0 + (int)threadIdx.x;
-    const int c = b < r.y ? P.parts[b].count : 0;
-    int t;
-    const int off = block_excl_scan(c, &t, sh);
-    if (b < r.y) P.parts[b].entryBase = base + off;
-    base += t;
-  }
 }
 
 // Entry of segment s in band [top, bot]: slope-intercept form of the whole
@@ -1441,199 +1433,327 @@ __device__ __forceinline__ Entry band_entry(float4 s, float top, float bot, floa
   return e;
 }
 
-// One wave per band: ordered entries, clipping, two-spanning flag
-// (partitionSegments 1194-1262).  Lanes exchange data only through ballots
-// and shuffles, which every lane executes.
-__global__ void __launch_bounds__(64) scene_band_write_kernel(ScenePools P) {
-  const int lane = threadIdx.x;
+// The segment groups [c0, c1) of a call that may reach band k, four at a
+// time so that their loads overlap: calls fn(segBand of this lane's segment
+// in each of the four, its index) until fn returns false.
+template <class Fn>
+__device__ __forceinline__ void band_groups(const ScenePools& P, int k, int c0, int c1, int s1, Fn fn) {
+  const int lane = threadIdx.x & 63;
+  for (int cb = c0; cb < c1; cb += 64) {
+    bool may = false;
+    if (cb + lane < c1) {
+      const int2 cr = P.segChunk[cb + lane];
+      may = k >= cr.x && k <= cr.y;
+    }
+    uint64_t cm = ballot(may);
+    while (cm) {
+      int2 sb[4];
+      int js[4];
+#pragma unroll
+      for (int u = 0; u < 4; u++) {
+        sb[u] = make_int2(1, 0);  // empty band range
+        js[u] = 0;
+        if (cm) {
+          js[u] = ((cb + __builtin_ctzll(cm)) << 6) + lane;
+          cm &= cm - 1;
+          if (js[u] < s1) sb[u] = P.segBand[js[u]];
+        }
+      }
+      if (!fn(sb, js)) return;
+    }
+  }
+}
+
+// The bands, in a tile per workgroup (tile t holds bands t,
+// t + nTiles, ...: neighbours, which are of one call and about as long, go to
+// different workgroups of one XCD).  One launch counts the entries of every
+// band, with requiresAntiAliasing, and each tile's; the next finds its tile's
+// place by summing the tiles before it (4,096 at most; an atomic per tile on
+// one counter took 40 us) and writes the entries.  A wave takes a band by
+// itself; when there are few bands (a page of text has a couple of hundred
+// with thousands of segment groups), the four waves of a workgroup share one,
+// each a quarter of its call's groups.
+constexpr int kBandBlocks = kBandTilesMax;  // at most one tile per workgroup
+struct BandTiles {
+  bool share;  // four waves per band
+  int tile, n;
+};
+__device__ __forceinline__ BandTiles band_tiling(int nb) {
+  BandTiles t;
+  t.share = nb <= kBandBlocks;
+  t.tile = t.share ? 1 : (nb + kBandBlocks - 1) / kBandBlocks;
+  t.n = (nb + t.tile - 1) / t.tile;
+  return t;
+}
+// The share of groups [c0, c1) of wave w of four.
+__device__ __forceinline__ void quarter(int w, int* c0, int* c1) {
+  const int per = (*c1 - *c0 + 3) / 4;
+  *c0 += w * per;
+  *c1 = *c0 + per < *c1 ? *c0 + per : *c1;
+}
+
+__device__ void band_count(const ScenePools& P, int block, int blocks) {
+  __shared__ int sSum, sCnt[4];
+  const int lane = threadIdx.x & 63, wave = uni((int)threadIdx.x >> 6);
   const int nb = P.counters[kCntBands];
-  if (nb > P.bandCap || P.counters[kCntEntries] > P.entryCap) return;
-  const XcdSpan sp = xcd_span(nb);
-  for (int b = sp.begin; b < sp.end; b += sp.step) {
-    const int it = uni(P.bandItem[b]);
-    ItemGeom g = P.geo[it];
-    g.bandBase = uni(g.bandBase);
-    g.segBase = uni(g.segBase);
-    g.segCount = uni(g.segCount);
-    FillInfo f = P.fills[it];
-    f.startY = uni(f.startY);
-    f.bandH = uni(f.bandH);
-    f.nParts = uni(f.nParts);
-    f.pathHeight = uni(f.pathHeight);
-    const int k = b - g.bandBase;
-    PartInfo pi = P.parts[b];
-    pi.entryBase = uni(pi.entryBase);
-    pi.count = uni(pi.count);
-    pi.flags = uni(pi.flags);
-    float top, bot;
-    band_rows(f, k, &top, &bot);
-    const int s0 = g.segBase, s1 = g.segBase + g.segCount;
-    if (pi.count != 2) {
-      int pos = 0;
-      const int cEnd = (s1 + 63) >> 6;
-      for (int cb = s0 >> 6; cb < cEnd && pos < pi.count; cb += 64) {
-        bool may = false;
-        if (cb + lane < cEnd) {
-          const int2 cr = P.segChunk[cb + lane];
-          may = k >= cr.x && k <= cr.y;
+  const BandTiles bt = band_tiling(nb);
+  const XcdSpan sp = xcd_span(bt.n, block, blocks);
+  for (int t = sp.begin; t < sp.end; t += sp.step) {
+    const int bn = (nb - t + bt.n - 1) / bt.n;
+    if (threadIdx.x < 4) sCnt[threadIdx.x] = 0;
+    if (threadIdx.x == 0) sSum = 0;
+    __syncthreads();
+    int sum = 0;
+    for (int i = bt.share ? 0 : wave; i < bn; i += bt.share ? 1 : 4) {
+      const int b = t + i * bt.n, it = uni(P.bandItem[b]);
+      const ItemGeom g = P.geo[it];
+      const int k = b - uni(g.bandBase), s0 = uni(g.segBase), s1 = s0 + uni(g.segCount);  // s0 is 64-aligned
+      int c0 = s0 >> 6, c1 = (s1 + 63) >> 6;
+      if (bt.share) quarter(wave, &c0, &c1);
+      int cnt = 0;
+      bool aa = false;
+      band_groups(P, k, c0, c1, s1, [&](const int2* sb, const int*) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          const bool in = k >= sb[u].x && k <= (sb[u].y & ~kSegAA);
+          cnt += __popcll(ballot(in));
+          if (ballot(in && (sb[u].y & kSegAA))) aa = true;
         }
-        uint64_t cm = __ballot(may);
-        while (cm && pos < pi.count) {  // four candidate chunks at a time
-          int2 sb[4];
-          int js[4];
-#pragma unroll
-          for (int u = 0; u < 4; u++) {
-            sb[u] = make_int2(1, 0);  // empty band range
-            js[u] = 0;
-            if (cm) {
-              js[u] = ((cb + __builtin_ctzll(cm)) << 6) + lane;
-              cm &= cm - 1;
-              if (js[u] < s1) sb[u] = P.segBand[js[u]];
-            }
-          }
-          bool in[4];
-          float4 sg[4];
-          int8_t sw[4];
-#pragma unroll
-          for (int u = 0; u < 4; u++) {
-            in[u] = k >= sb[u].x && k <= (sb[u].y & ~kSegAA);
-            sg[u] = make_float4(0, 0, 0, 0);
-            sw[u] = 0;
-            if (in[u]) {
-              sg[u] = P.segs[js[u]];
-              sw[u] = P.segW[js[u]];
-            }
-          }
+        return true;
+      });
+      sum += cnt;
+      if (bt.share) {
+        if (lane == 0) sCnt[wave] = cnt | (aa ? 1 << 30 : 0);
+      } else {
+        P.parts[b] = PartInfo{0, cnt, aa ? 1 : 0, 0};  // every lane stores the same value
+        if (cnt > P.gcap && lane == 0) atomicMax(&P.counters[kCntMaxBand], cnt);
+      }
+    }
+    if (lane == 0 && sum) atomicAdd(&sSum, sum);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      P.tileSum[t] = sSum;
+      if (bt.share) {
+        const int m = (1 << 30) - 1;
+        P.parts[t] = PartInfo{0, sSum, ((sCnt[0] | sCnt[1] | sCnt[2] | sCnt[3]) >> 30) & 1, 0};
+        P.bandQuarter[t] = make_int4(sCnt[0] & m, sCnt[1] & m, sCnt[2] & m, sCnt[3] & m);
+        if (sSum > P.gcap) atomicMax(&P.counters[kCntMaxBand], sSum);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+__global__ void __launch_bounds__(256) scene_band_write_kernel(ScenePools P) {
+  __shared__ int sh[4];
+  const int lane = threadIdx.x & 63, wave = uni((int)threadIdx.x >> 6);
+  if (P.counters[kCntError] & 3) return;  // (not set by this kernel)
+  const int nb = P.counters[kCntBands];
+  const BandTiles bt = band_tiling(nb);
+  const XcdSpan sp = xcd_span(bt.n, blockIdx.x, gridDim.x);
+  for (int t = sp.begin; t < sp.end; t += sp.step) {
+    const int bn = (nb - t + bt.n - 1) / bt.n;
+    // entries of the tiles before this one, and of all
+    int before = 0, all = 0;
+    for (int i = (int)threadIdx.x; i < bt.n; i += 256) {
+      const int v = P.tileSum[i];
+      all += v;
+      before += i < t ? v : 0;
+    }
+    int tot;
+    block_excl_scan_n<256>(all, &tot, sh);
+    int base;
+    block_excl_scan_n<256>(before, &base, sh);
+    if (t == 0 && threadIdx.x == 0) {
+      P.counters[kCntEntries] = tot;
+      if (tot > P.entryCap) atomicOr(&P.counters[kCntError], 4);
+    }
+    if (tot > P.entryCap) return;  // the same in every workgroup
+    for (int r0 = 0; r0 < bn; r0 += 64) {  // 64 bands' counts and places at a time
+      const int n64 = bn - r0 < 64 ? bn - r0 : 64;
+      const PartInfo mine = lane < n64 ? P.parts[t + (r0 + lane) * bt.n] : PartInfo{0, 0, 0, 0};
+      int sum64;
+      const int place = base + wave_excl_scan(mine.count, &sum64);
+      base += sum64;
+      for (int i = bt.share ? 0 : wave; i < n64; i += bt.share ? 1 : 4) {
+        const int b = t + (r0 + i) * bt.n, it = uni(P.bandItem[b]);
+        const int eb = __builtin_amdgcn_readlane(place, i);
+        const ItemGeom g = P.geo[it];
+        FillInfo f = P.fills[it];
+        const int k = b - uni(g.bandBase), s0 = uni(g.segBase), s1 = s0 + uni(g.segCount);
+        f.startY = uni(f.startY);
+        f.bandH = uni(f.bandH);
+        f.nParts = uni(f.nParts);
+        f.pathHeight = uni(f.pathHeight);
+        float top, bot;
+        band_rows(f, k, &top, &bot);
+        int c0 = s0 >> 6, c1 = (s1 + 63) >> 6;
+        const int count = __builtin_amdgcn_readlane(mine.count, i), flags = __builtin_amdgcn_readlane(mine.flags, i);
+        if (!bt.share || wave == 0) P.parts[b].entryBase = eb;  // every lane stores the same value
+        int pos = 0, end = count;
+        if (bt.share && count != 2) {
+          const int4 q = P.bandQuarter[b];
+          const int q0 = uni(q.x), q1 = uni(q.y), q2 = uni(q.z);
+          quarter(wave, &c0, &c1);
+          pos = wave == 0 ? 0 : wave == 1 ? q0 : wave == 2 ? q0 + q1 : q0 + q1 + q2;
+          end = wave == 0 ? q0 : wave == 1 ? q0 + q1 : wave == 2 ? q0 + q1 + q2 : count;
+        }
+        if (count != 2) {
           const uint64_t below = (1ull << lane) - 1ull;
+          if (pos < end)
+            band_groups(P, k, c0, c1, s1, [&](const int2* sb, const int* js) {
+              bool in[4];
+              float4 sg[4];
+              int8_t sw[4];
+#pragma unroll
+              for (int u = 0; u < 4; u++) {
+                in[u] = k >= sb[u].x && k <= (sb[u].y & ~kSegAA);
+                sg[u] = make_float4(0, 0, 0, 0);
+                sw[u] = 0;
+                if (in[u]) {
+                  sg[u] = P.segs[js[u]];
+                  sw[u] = P.segW[js[u]];
+                }
+              }
+#pragma unroll
+              for (int u = 0; u < 4; u++) {
+                const uint64_t m = ballot(in[u]);
+                if (in[u]) {
+                  const int p = eb + pos + __popcll(m & below);
+                  float4 cl;
+                  P.entries[p] = band_entry(sg[u], top, bot, &cl);
+                  P.entW[p] = sw[u];
+                }
+                pos += __popcll(m);
+              }
+              return pos < end;
+            });
+          continue;
+        }
+        if (bt.share && wave != 0) continue;
+        // two entries: gather both segments into every lane, decide the
+        // two-spanning flag and order (1250-1262), then write
+        float4 g0 = make_float4(0, 0, 0, 0), g1 = g0;
+        int w0 = 0, w1 = 0, found = 0;
+        band_groups(P, k, c0, c1, s1, [&](const int2* sb, const int* js) {
 #pragma unroll
           for (int u = 0; u < 4; u++) {
-            const uint64_t m = __ballot(in[u]);
-            if (in[u]) {
-              const int p = pos + __popcll(m & below);
-              float4 cl;
-              P.entries[pi.entryBase + p] = band_entry(sg[u], top, bot, &cl);
-              P.entW[pi.entryBase + p] = sw[u];
+            const bool in = k >= sb[u].x && k <= (sb[u].y & ~kSegAA);
+            uint64_t m = ballot(in);
+            if (!m) continue;
+            float4 sg = make_float4(0, 0, 0, 0);
+            int wv = 0;
+            if (in) {
+              sg = P.segs[js[u]];
+              wv = P.segW[js[u]];
             }
-            pos += __popcll(m);
+            while (m != 0 && found < 2) {
+              const int src = __builtin_ctzll(m);
+              m &= m - 1;
+              const float4 t4 = make_float4(__shfl(sg.x, src, 64), __shfl(sg.y, src, 64), __shfl(sg.z, src, 64),
+                                            __shfl(sg.w, src, 64));
+              const int tw = __shfl(wv, src, 64);
+              if (found == 0) {
+                g0 = t4;
+                w0 = tw;
+              } else {
+                g1 = t4;
+                w1 = tw;
+              }
+              found++;
+            }
+          }
+          return found < 2;
+        });
+        float4 a, c;
+        Entry first = band_entry(g0, top, bot, &a);
+        Entry second = band_entry(g1, top, bot, &c);
+        const V2 a0 = v2(a.x, a.y), a1 = v2(a.z, a.w), d0 = v2(c.x, c.y), d1 = v2(c.z, c.w);
+        bool swap = false, two = false;
+        if (!intersects_inside(a0, a1, d0, d1)) {
+          if (a0.y <= top && a1.y >= bot && d0.y <= top && d1.y >= bot) {
+            two = true;
+            swap = midpoint_x(a0, a1) > midpoint_x(d0, d1);
           }
         }
-      }
-      continue;
-    }
-    // two entries: gather both segments into every lane, decide the
-    // two-spanning flag and order (1250-1262), then write
-    float4 g0 = make_float4(0, 0, 0, 0), g1 = g0;
-    int w0 = 0, w1 = 0, found = 0;
-    const int cEnd2 = (s1 + 63) >> 6;
-    for (int cb = s0 >> 6; cb < cEnd2 && found < 2; cb += 64) {
-      bool may = false;
-      if (cb + lane < cEnd2) {
-        const int2 cr = P.segChunk[cb + lane];
-        may = k >= cr.x && k <= cr.y;
-      }
-      uint64_t cm = __ballot(may);
-      while (cm && found < 2) {
-      const int c = cb + __builtin_ctzll(cm);
-      cm &= cm - 1;
-      const int j = (c << 6) + lane;
-      bool in = false;
-      float4 sg = make_float4(0, 0, 0, 0);
-      int wv = 0;
-      if (j < s1) {
-        const int2 sb = P.segBand[j];
-        in = k >= sb.x && k <= (sb.y & ~kSegAA);
-        if (in) {
-          sg = P.segs[j];
-          wv = P.segW[j];
+        // every lane stores the same values (conditional copies, not ?: on the
+        // two lvalues, which would keep both entries in memory)
+        if (swap) {
+          const Entry e = first;
+          first = second;
+          second = e;
         }
-      }
-      uint64_t m = __ballot(in);
-      while (m != 0 && found < 2) {
-        const int src = __builtin_ctzll(m);
-        m &= m - 1;
-        float4 t = make_float4(__shfl(sg.x, src, 64), __shfl(sg.y, src, 64), __shfl(sg.z, src, 64),
-                               __shfl(sg.w, src, 64));
-        int tw = __shfl(wv, src, 64);
-        if (found == 0) {
-          g0 = t;
-          w0 = tw;
-        } else {
-          g1 = t;
-          w1 = tw;
-        }
-        found++;
-      }
+        P.entries[eb] = first;
+        P.entries[eb + 1] = second;
+        P.entW[eb] = (int8_t)(swap ? w1 : w0);
+        P.entW[eb + 1] = (int8_t)(swap ? w0 : w1);
+        if (two) P.parts[b].flags = flags | 2;
       }
     }
-    float4 a, c;
-    Entry e0 = band_entry(g0, top, bot, &a);
-    Entry e1 = band_entry(g1, top, bot, &c);
-    int32_t flags = pi.flags;
-    bool swap = false;
-    V2 a0 = v2(a.x, a.y), a1 = v2(a.z, a.w), c0 = v2(c.x, c.y), c1 = v2(c.z, c.w);
-    if (!intersects_inside(a0, a1, c0, c1)) {
-      if (a0.y <= top && a1.y >= bot && c0.y <= top && c1.y >= bot) {
-        flags |= 2;
-        swap = midpoint_x(a0, a1) > midpoint_x(c0, c1);
-      }
-    }
-    // every lane stores the same values (conditional copies, not ?: on the
-    // two lvalues, which would keep both entries in memory)
-    Entry first = e0, second = e1;
-    if (swap) {
-      first = e1;
-      second = e0;
-    }
-    P.entries[pi.entryBase] = first;
-    P.entries[pi.entryBase + 1] = second;
-    P.entW[pi.entryBase] = (int8_t)(swap ? w1 : w0);
-    P.entW[pi.entryBase + 1] = (int8_t)(swap ? w0 : w1);
-    P.parts[b].flags = flags;
+    __syncthreads();
   }
 }
 
 // ---------------------------------------------------------------------------
-// row bins for phase B: one wave per bin, calls compacted in call order
+// row bins for phase B: a workgroup per bin lists the calls that meet its
+// rows, in call order; wave w takes the w-th quarter of the calls
 // ---------------------------------------------------------------------------
-template <bool kWrite>
-__global__ void __launch_bounds__(64) scene_bin_kernel(ScenePools P) {
-  const int lane = threadIdx.x;
-  const int nBins = (P.H + kBinRows - 1) / kBinRows;
-  if (kWrite && P.counters[kCntBinEntries] > P.binCap) return;
-  for (int bin = blockIdx.x; bin < nBins; bin += gridDim.x) {
-    const int r0 = bin * kBinRows, r1 = r0 + kBinRows;
-    int pos = kWrite ? P.binOff[bin] : 0;
-    for (int i0 = 0; i0 < P.nItems; i0 += 64) {
-      const int it = i0 + lane;
-      bool in = false;
-      if (it < P.nItems) {
-        int4 r = P.itemRows[it];
-        in = r.x < r1 && r.y > r0;
-      }
-      uint64_t m = __ballot(in);
-      if (kWrite && in) P.binList[pos + __popcll(m & ((1ull << lane) - 1ull))] = it;
-      pos += __popcll(m);
+__device__ void fill_bin(const ScenePools& P, int bin) {
+  __shared__ int sCnt[4], sBase;
+  const int lane = threadIdx.x & 63, wave = uni((int)threadIdx.x >> 6);
+  const int r0 = bin * kBinRows, r1 = r0 + kBinRows;
+  const int per = ((P.nItems + 3) / 4 + 63) & ~63;
+  const int i0 = wave * per, i1 = i0 + per < P.nItems ? i0 + per : P.nItems;
+  int cnt = 0;
+#pragma unroll 4
+  for (int i = i0; i < i1; i += 64) {
+    const int it = i + lane;
+    bool in = false;
+    if (it < i1) {
+      const int4 r = P.itemRows[it];
+      in = r.x < r1 && r.y > r0;
     }
-    if (!kWrite) P.binCount[bin] = pos;  // every lane stores the same value
+    cnt += __popcll(ballot(in));
   }
-}
-
-__global__ void __launch_bounds__(kScanBlock) scene_bin_scan_kernel(ScenePools P) {
-  __shared__ int sh[kScanBlock / 64];
-  const int nBins = (P.H + kBinRows - 1) / kBinRows;
-  int tot = 0;
-  for (int b0 = 0; b0 < nBins; b0 += kScanBlock) {
-    int b = b0 + threadIdx.x;
-    int c = b < nBins ? P.binCount[b] : 0;
-    int t;
-    int off = block_excl_scan_n<kScanBlock>(c, &t, sh);
-    if (b < nBins) P.binOff[b] = tot + off;
-    tot += t;
-  }
+  if (lane == 0) sCnt[wave] = cnt;
+  __syncthreads();
+  const int c0 = uni(sCnt[0]), c1 = uni(sCnt[1]), c2 = uni(sCnt[2]), tot = c0 + c1 + c2 + uni(sCnt[3]);
   if (threadIdx.x == 0) {
-    P.binOff[nBins] = tot;
-    P.counters[kCntBinEntries] = tot;
-    if (tot > P.binCap) atomicOr(&P.counters[kCntError], 32);
+    const int base = atomicAdd(&P.counters[kCntBinEntries], tot);
+    if (base + tot > P.binCap) atomicOr(&P.counters[kCntError], 32);
+    P.binOff[bin] = base;
+    P.binCount[bin] = tot;
+    sBase = base;
+  }
+  __syncthreads();
+  const int base = uni(sBase);
+  if (base + tot > P.binCap) return;
+  int pos = base + (wave == 0 ? 0 : wave == 1 ? c0 : wave == 2 ? c0 + c1 : c0 + c1 + c2);
+#pragma unroll 4
+  for (int i = i0; i < i1; i += 64) {
+    const int it = i + lane;
+    bool in = false;
+    if (it < i1) {
+      const int4 r = P.itemRows[it];
+      in = r.x < r1 && r.y > r0;
+    }
+    const uint64_t m = ballot(in);
+    if (in) P.binList[pos + __popcll(m & ((1ull << lane) - 1ull))] = it;
+    pos += __popcll(m);
+  }
+}
+
+// Both need the plan and not each other.  binBlocks is a multiple of kXcds.
+__global__ void __launch_bounds__(256) scene_band_kernel(ScenePools P, int binBlocks) {
+  __shared__ int sErr;
+  // read once: another workgroup may set the error meanwhile
+  if (threadIdx.x == 0) sErr = P.counters[kCntError] & 3;
+  __syncthreads();
+  if (uni(sErr)) return;
+  if ((int)blockIdx.x < binBlocks) {
+    if ((int)blockIdx.x < (P.H + kBinRows - 1) / kBinRows) fill_bin(P, blockIdx.x);
+  } else {
+    band_count(P, (int)blockIdx.x - binBlocks, (int)gridDim.x - binBlocks);
   }
 }
 
@@ -1695,113 +1815,90 @@ __device__ __forceinline__ int band_class(const ScenePools& P, const ItemGeom& g
   return (p.flags & 1) || c < heavyClass ? c : heavyClass - 1;
 }
 
-// Maps work items to calls and records their cost classes, counting them
-// per class (per block in LDS, then one global atomic per class and block).
-// The classes of a call's bands are staged in LDS first.
-constexpr int kLdsBandClasses = 4096;
-constexpr int kTaskMapBlock = 1024;
-__global__ void __launch_bounds__(kTaskMapBlock) scene_task_map_kernel(ScenePools P) {
-  __shared__ int32_t hist[kCostClasses];
-  __shared__ int8_t cls[kLdsBandClasses];
-  const int tid = threadIdx.x, lane = tid & 63;
+// The work items of one (call, row group, window) unit, a lane per unit: fn(r,
+// class, grouped) is called by every lane alike, with a negative class for
+// lanes without an item at row r of their group.
+template <class Fn>
+__device__ __forceinline__ void unit_items(const ScenePools& P, int unit, const ItemGeom& g, const FillInfo& F,
+                                           int heavyClass, Fn fn) {
+  const bool on = unit < (g.rowCount + kRowGroup - 1) / kRowGroup * g.nWin;
+  const int rg = unit / g.nWin * kRowGroup, win = unit % g.nWin;
+  const int rows = !on ? 0 : (rg + kRowGroup < g.rowCount ? kRowGroup : g.rowCount - rg);
+  const bool banded = F.nParts > 0 && F.bandH > 0;
+  // classes of its rows' bands (every row of a call lies in [startY, pathHeight))
+  int cls[kRowGroup], chunk = 0;
+#pragma unroll
+  for (int q = 0; q < kRowGroup; q++) {
+    cls[q] = 0;
+    if (banded && q < rows) {
+      cls[q] = band_class(P, g, band_of_row(F, g.rowStart + rg + q), heavyClass);
+      chunk = cls[q] > chunk ? cls[q] : chunk;
+    }
+  }
+  const bool grouped = chunk <= kGroupMaxClass;
+  if (ballot(on && grouped)) fn(rg, on && grouped ? chunk : -1, true);
+  if (ballot(on && !grouped)) {
+#pragma unroll
+    for (int q = 0; q < kRowGroup; q++) {
+      // a heavy row's item takes kHeavyWins windows at a time
+      const bool own = on && !grouped && q < rows && (cls[q] < heavyClass || win % kHeavyWins == 0);
+      fn(rg + q, own ? cls[q] : -1, false);
+    }
+  }
+}
+
+// Counts the work items per cost class (kPlace = false), or places them in
+// the order, largest class first (kPlace = true): a wave per 64 units, each
+// workgroup a contiguous share of them.  Placing counts the share again and
+// reserves its range of every class with one atomic before it deals the
+// places out in LDS.
+template <bool kPlace>
+__global__ void __launch_bounds__(256) scene_task_kernel(ScenePools P) {
+  __shared__ int32_t hist[kCostClasses], start[kCostClasses];
+  const int lane = threadIdx.x & 63, wave = uni((int)threadIdx.x >> 6);
   if (P.counters[kCntError]) return;
   const int heavyClass = heavy_class(P);
-  if (tid < kCostClasses) hist[tid] = 0;
+  if (threadIdx.x < kCostClasses) hist[threadIdx.x] = 0;
   __syncthreads();
-  for (int it = blockIdx.x; it < P.nItems; it += gridDim.x) {
+  const int nChunks = P.counters[kCntChunks];
+  const int per = (nChunks + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int k0 = (int)blockIdx.x * per, k1 = k0 + per < nChunks ? k0 + per : nChunks;
+  for (int k = k0 + wave; k < k1; k += 4) {
+    const int2 ch = P.taskChunk[k];
+    const int it = uni(ch.x);
+    unit_items(P, uni(ch.y) * 64 + lane, P.geo[it], P.fills[it], heavyClass, [&](int, int c, bool) {
+      if (c >= 0) atomicAdd(&hist[c], 1);
+    });
+  }
+  __syncthreads();
+  if (!kPlace) {
+    if (threadIdx.x < kCostClasses && hist[threadIdx.x])
+      atomicAdd(&P.counters[kCntClassHist + threadIdx.x], hist[threadIdx.x]);
+    return;
+  }
+  if (wave == 0) {  // lane l: class kCostClasses - 1 - l
+    const int c = kCostClasses - 1 - lane;
+    const int n = lane < kCostClasses ? P.counters[kCntClassHist + c] : 0;
+    int tot;
+    const int off = wave_excl_scan(n, &tot);
+    if (lane < kCostClasses) {
+      start[c] = off + (hist[c] ? atomicAdd(&P.counters[kCntClassCursor + c], hist[c]) : 0);
+      if (blockIdx.x == 0 && c == heavyClass - 1) P.counters[kCntHeavy] = off;
+      if (blockIdx.x == 0 && c == 0) P.counters[kCntGroups] = tot;
+    }
+  }
+  __syncthreads();
+  for (int k = k0 + wave; k < k1; k += 4) {
+    const int2 ch = P.taskChunk[k];
+    const int it = uni(ch.x);
     const ItemGeom g = P.geo[it];
-    const FillInfo F = P.fills[it];
-    const int nt = g.rowCount * g.nWin;
-    if (nt <= 0) continue;
-    const bool banded = F.nParts > 0 && F.bandH > 0;
-    const int nb = banded ? F.nParts : 0;
-    for (int b = tid; b < nb && b < kLdsBandClasses; b += kTaskMapBlock) {
-      cls[b] = (int8_t)band_class(P, g, b, heavyClass);
-    }
-    __syncthreads();
-    for (int t0 = 0; t0 < nt; t0 += kTaskMapBlock) {
-      const int t = t0 + tid;
-      const bool on = t < nt;
-      int c = -1;
-      bool grouped = false;
-      if (on) {
-        // classes of this task's row and of its group's rows (the bands
-        // from the group's first row to its last; every row of a call lies
-        // in [startY, pathHeight))
-        const int r = t / g.nWin, rg = r - r % kRowGroup;
-        const int re = (rg + kRowGroup < g.rowCount ? rg + kRowGroup : g.rowCount) - 1;
-        int own = 0, chunk = 0;
-        if (banded) {
-          const int pr = band_of_row(F, g.rowStart + r), p0 = band_of_row(F, g.rowStart + rg),
-                    p1 = band_of_row(F, g.rowStart + re);
-          for (int pi = p0; pi <= p1; pi++) {
-            const int rc = pi < kLdsBandClasses ? cls[pi] : band_class(P, g, pi, heavyClass);
-            if (pi == pr) own = rc;
-            chunk = rc > chunk ? rc : chunk;
-          }
-        }
-        grouped = chunk <= kGroupMaxClass;
-        // a heavy row's item takes kHeavyWins windows at a time
-        if (own >= heavyClass) c = (t % g.nWin) % kHeavyWins == 0 ? own : -1;
-        else c = !grouped ? own : (r == rg ? chunk : -1);
-        P.taskItem[g.taskBase + t] = grouped ? (int32_t)((uint32_t)it | 0x80000000u) : it;
-        P.taskClass[g.taskBase + t] = (int8_t)c;
-      }
-      // one LDS atomic per class present in the wave
-      uint64_t pending = __ballot(c >= 0);
-      while (pending) {
-        const int leader = __builtin_ctzll(pending);
-        const int cl = __builtin_amdgcn_readlane(c, leader);
-        const uint64_t m = __ballot(c == cl);
-        if (lane == leader) atomicAdd(&hist[cl], (int)__popcll(m));
-        pending &= ~m;
-      }
-    }
-    __syncthreads();
+    const int unit = uni(ch.y) * 64 + lane, first = g.taskBase + unit % g.nWin;
+    unit_items(P, unit, g, P.fills[it], heavyClass, [&](int r, int c, bool grouped) {
+      if (c >= 0)
+        P.taskOrder[atomicAdd(&start[c], 1)] =
+            make_int2(first + r * g.nWin, grouped ? (int32_t)((uint32_t)it | 0x80000000u) : it);
+    });
   }
-  __syncthreads();
-  if (tid < kCostClasses && hist[tid]) atomicAdd(&P.counters[kCntClassHist + tid], hist[tid]);
-}
-
-// Block b's contiguous share of the work items.
-__device__ __forceinline__ int2 task_share(int ntasks) {
-  const int per = ((ntasks + (int)gridDim.x - 1) / (int)gridDim.x + 63) & ~63;
-  const int lo = (int)blockIdx.x * per;
-  return make_int2(lo, lo + per < ntasks ? lo + per : ntasks);
-}
-
-// Start of each cost class in the work-item order, largest class first, and
-// the number of items in the heavy classes.
-__global__ void scene_task_scan_kernel(ScenePools P) {
-  if (threadIdx.x != 0) return;
-  int32_t* const counters = P.counters;
-  const int heavyClass = heavy_class(P);
-  int off = 0;
-  for (int c = kCostClasses - 1; c >= 0; c--) {
-    if (c == heavyClass - 1) counters[kCntHeavy] = off;
-    counters[kCntClassCursor + c] = off;
-    off += counters[kCntClassHist + c];
-  }
-  counters[kCntGroups] = off;
-}
-
-// Places every work item in the order by its cost class: each block
-// reserves a range of every class for its share of the items, then deals it
-// out with LDS atomics.
-__global__ void __launch_bounds__(64) scene_task_order_kernel(ScenePools P) {
-  __shared__ int32_t cnt[kCostClasses], cur[kCostClasses];
-  const int lane = threadIdx.x;
-  if (P.counters[kCntError]) return;
-  if (lane < kCostClasses) cnt[lane] = 0;
-  __syncthreads();
-  const int2 r = task_share(P.counters[kCntTasks]);
-  for (int t = r.x + lane; t < r.y; t += 64)
-    if (P.taskClass[t] >= 0) atomicAdd(&cnt[P.taskClass[t]], 1);
-  __syncthreads();
-  if (lane < kCostClasses) cur[lane] = cnt[lane] ? atomicAdd(&P.counters[kCntClassCursor + lane], cnt[lane]) : 0;
-  __syncthreads();
-  for (int t = r.x + lane; t < r.y; t += 64)
-    if (P.taskClass[t] >= 0) P.taskOrder[atomicAdd(&cur[P.taskClass[t]], 1)] = t;
 }
 
 // A wave's place in the run pool: it appends its runs to chunks it takes one
@@ -1919,14 +2016,14 @@ constexpr int kHeavyMaxWidth = 1 << 22;  // 24.8 positions of a row item stay be
 
 // What the workgroup needs to know of a work item.
 struct HeavyItem {
-  int32_t first;       // task of its first window; -1 ends the kernel
+  int32_t first, it;   // task of its first window (-1 ends the kernel), call
   int32_t y, gx0, nw;  // row, first pixel, windows
   PartInfo part;       // the row's band
   int32_t mode, rule, xhi, covLo, covHi;
 };
 
 // Wave 0 reads the records of the next item while the workgroup is busy with
-// this one: each step's loads (order -> task -> call -> band) are issued a
+// this one: each step's loads (order -> call -> band) are issued a
 // phase before the next step needs them.  The items go round the workgroups
 // in their order, longest first; a shared queue would cost each item the
 // round trip of an atomic (8 to 14 thousand cycles of 70).
@@ -1937,10 +2034,9 @@ struct HeavyFetch {
   FillInfo F;
   PartInfo part;
   __device__ __forceinline__ void step_order(const ScenePools& P, int n) {
-    first = q < n ? P.taskOrder[q] : -1;
-  }
-  __device__ __forceinline__ void step_task(const ScenePools& P) {
-    it = first >= 0 ? P.taskItem[first] & 0x7fffffff : 0;
+    const int2 o = q < n ? P.taskOrder[q] : make_int2(-1, 0);
+    first = o.x;
+    it = o.y;  // never marked as grouped
   }
   __device__ __forceinline__ void step_call(const ScenePools& P) {
     g = P.geo[it];
@@ -1948,6 +2044,7 @@ struct HeavyFetch {
   }
   __device__ __forceinline__ void step_band(const ScenePools& P, HeavyItem* h) {
     h->first = first;  // every lane stores the same values
+    h->it = it;
     if (first < 0) return;
     const int local = first - g.taskBase, win0 = local % g.nWin, y = g.rowStart + local / g.nWin;
     part = P.parts[g.bandBase + band_of_row(F, y)];
@@ -1988,7 +2085,6 @@ __global__ void __launch_bounds__(kHeavyThreads, 5) scene_heavy_kernel(ScenePool
   if (wave == 0) {
     nx.q = blockIdx.x;
     nx.step_order(P, nHeavy);
-    nx.step_task(P);
     nx.step_call(P);
     nx.step_band(P, &sItems[0]);
   }
@@ -2099,9 +2195,8 @@ __global__ void __launch_bounds__(kHeavyThreads, 5) scene_heavy_kernel(ScenePool
         if (lane == 63 && total[m]) atomicAdd(&sTotal[m], total[m]);
       }
     }
-    if (wave == 0) nx.step_task(P);
-    __syncthreads();
     if (wave == 0) nx.step_call(P);
+    __syncthreads();
     ne = uni(sNe);
     leave = leave || (ne > 0 && !uni(sNotSpan) && (ne % 2) == 0) ||
             (uni(sTotal[0]) | uni(sTotal[1]) | uni(sTotal[2]) | uni(sTotal[3]) | uni(sTotal[4])) != 0;
@@ -2196,7 +2291,8 @@ __global__ void __launch_bounds__(kHeavyThreads, 5) scene_heavy_kernel(ScenePool
     if (leave) {  // to the rows kernel, window by window
       if (wave == 0) nx.step_band(P, next);
       for (int i = tid; i < kHeavyWins * (kWinA + 4); i += kHeavyThreads) ((int32_t*)D)[i] = 0;
-      if (tid < nw) P.taskOrder[P.taskCap + atomicAdd(&P.counters[kCntLeft], 1)] = first + tid;
+      if (tid < nw)
+        P.taskOrder[P.taskCap + atomicAdd(&P.counters[kCntLeft], 1)] = make_int2(first + tid, uni(sItem.it));
       continue;
     }
     if (ne == 0 && wave == 0) nx.step_band(P, next);
@@ -2231,8 +2327,8 @@ __global__ void __launch_bounds__(64, 4) scene_rows_kernel(ScenePools P) {
     if (q >= nItems) break;
     // Work item, call and the call's records are the same in every lane:
     // read them into scalar registers.
-    const int first = uni(q < nLeft ? P.taskOrder[P.taskCap + q] : P.taskOrder[nHeavy + q - nLeft]);
-    const int itw = uni(P.taskItem[first]);
+    const int2 item = P.taskOrder[q < nLeft ? P.taskCap + q : nHeavy + q - nLeft];
+    const int first = uni(item.x), itw = uni(item.y);
     const int it = itw & 0x7fffffff;
     ItemGeom g = P.geo[it];
     g.rowStart = uni(g.rowStart);
@@ -2333,8 +2429,8 @@ __global__ void __launch_bounds__(64) scene_compose_kernel(ScenePools P, void* c
     const int b1 = b0 + kWinB < W ? b0 + kWinB : W;
     bool loaded = false, dirty = false;
     const int bin = y / kBinRows;
-    const int l1 = P.binOff[bin + 1];
-    for (int i0 = P.binOff[bin]; i0 < l1; i0 += 64) {
+    const int l0 = P.binOff[bin], l1 = l0 + P.binCount[bin];
+    for (int i0 = l0; i0 < l1; i0 += 64) {
       const int li = i0 + lane;
       bool cov = false;
       int4 paint = make_int4(0, 0, 0, 0), span = paint;
@@ -2648,9 +2744,7 @@ int scene_launch_clear(const ScenePools& p, hipStream_t s) {
 
 int scene_launch_geometry(const ScenePools& p, hipStream_t s) {
   if (p.nItems <= 0) return 0;
-  // calls of more than kBlock commands (they come first in itemOrder):
-  // commands flattened by a thread each over the whole device, the rest in
-  // 1024-thread workgroups
+  // calls of more than kBlock commands (they come first in itemOrder)
   if (p.nBig > 0) {
     const int grid = (p.bigCmds + 255) / 256;
     hipLaunchKernelGGL(scene_big_cmd_kernel, dim3(grid), dim3(256), 0, s, p, 0);
@@ -2660,40 +2754,34 @@ int scene_launch_geometry(const ScenePools& p, hipStream_t s) {
     hipLaunchKernelGGL(scene_big_front_alloc_kernel, dim3(p.nBig), dim3(256), 0, s, p);
     hipLaunchKernelGGL(scene_big_front_kernel, dim3(kBigSegGrid), dim3(256), 0, s, p, 1);
     hipLaunchKernelGGL(scene_big_cmd_kernel, dim3(grid), dim3(256), 0, s, p, 1);
-    // fills: segments in chunks over the device; strokes: one workgroup
+    // fills: segments in chunks over the device
     hipLaunchKernelGGL(scene_big_plan_kernel, dim3(1), dim3(kScanBlock), 0, s, p, 0);
     hipLaunchKernelGGL(scene_big_seg_kernel, dim3(kBigSegGrid), dim3(256), 0, s, p, 0);
     hipLaunchKernelGGL(scene_big_seg_alloc_kernel, dim3(p.nBig), dim3(256), 0, s, p);
-    hipLaunchKernelGGL(scene_big_plan_kernel, dim3(1), dim3(kScanBlock), 0, s, p, 1);
     hipLaunchKernelGGL(scene_big_seg_kernel, dim3(kBigSegGrid), dim3(256), 0, s, p, 1);
-    hipLaunchKernelGGL(scene_big_band_kernel, dim3(kBigSegGrid), dim3(256), 0, s, p);
-    hipLaunchKernelGGL((scene_geom_kernel<kBigGeomBlock, kGeomBack>), dim3(p.nBig), dim3(kBigGeomBlock), 0, s,
-                       p, 0);
   }
   if (p.nItems > p.nBig)
-    hipLaunchKernelGGL((scene_geom_kernel<kBlock, kGeomAll>), dim3(p.nItems - p.nBig), dim3(kBlock), 0, s, p,
-                       p.nBig);
-  hipLaunchKernelGGL(scene_plan_kernel, dim3(1), dim3(kScanBlock), 0, s, p);
+    hipLaunchKernelGGL(scene_geom_kernel, dim3(p.nItems - p.nBig), dim3(kBlock), 0, s, p, p.nBig);
+  if (p.nStrokes > 0) {
+    hipLaunchKernelGGL(scene_stroke_kernel<false>, dim3(kStrokeGrid), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(scene_stroke_alloc_kernel, dim3(p.nStrokes), dim3(256), 0, s, p);
+    hipLaunchKernelGGL(scene_stroke_kernel<true>, dim3(kStrokeGrid), dim3(256), 0, s, p);
+  }
+  const int planBlocks = (p.nItems + kPlanCalls - 1) / kPlanCalls;
+  hipLaunchKernelGGL(scene_plan_kernel, dim3(planBlocks + kSegBandBlocks), dim3(256), 0, s, p, planBlocks);
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
 }
 
-int scene_launch_bands(const ScenePools& p, int grid, hipStream_t s) {
-  hipLaunchKernelGGL(scene_band_map_kernel, dim3(grid / 4 > 0 ? grid / 4 : 1), dim3(kBlock), 0, s, p);
-  hipLaunchKernelGGL(scene_band_count_kernel, dim3(grid), dim3(64), 0, s, p);
-  hipLaunchKernelGGL(scene_entry_tile_kernel, dim3(kEntryTiles), dim3(kBlock), 0, s, p);
-  hipLaunchKernelGGL(scene_entry_scan_kernel, dim3(1), dim3(kEntryTiles), 0, s, p);
-  hipLaunchKernelGGL(scene_entry_apply_kernel, dim3(kEntryTiles), dim3(kBlock), 0, s, p);
-  hipLaunchKernelGGL(scene_band_write_kernel, dim3(grid), dim3(64), 0, s, p);
+int scene_launch_bands(const ScenePools& p, hipStream_t s) {
+  const int bins = (p.H + kBinRows - 1) / kBinRows, binBlocks = (bins + kXcds - 1) / kXcds * kXcds;
+  hipLaunchKernelGGL(scene_band_kernel, dim3(binBlocks + kBandBlocks), dim3(256), 0, s, p, binBlocks);
+  hipLaunchKernelGGL(scene_band_write_kernel, dim3(kBandBlocks), dim3(256), 0, s, p);
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
 }
 
-int scene_launch_bins(const ScenePools& p, int grid, hipStream_t s) {
-  hipLaunchKernelGGL(scene_task_map_kernel, dim3(grid / 4 > 0 ? grid / 4 : 1), dim3(kTaskMapBlock), 0, s, p);
-  hipLaunchKernelGGL(scene_task_scan_kernel, dim3(1), dim3(64), 0, s, p);
-  hipLaunchKernelGGL(scene_task_order_kernel, dim3(grid >= 8 ? grid / 4 : grid), dim3(64), 0, s, p);
-  hipLaunchKernelGGL(scene_bin_kernel<false>, dim3(grid), dim3(64), 0, s, p);
-  hipLaunchKernelGGL(scene_bin_scan_kernel, dim3(1), dim3(kScanBlock), 0, s, p);
-  hipLaunchKernelGGL(scene_bin_kernel<true>, dim3(grid), dim3(64), 0, s, p);
+int scene_launch_tasks(const ScenePools& p, hipStream_t s) {
+  hipLaunchKernelGGL(scene_task_kernel<false>, dim3(kTaskBlocks), dim3(256), 0, s, p);
+  hipLaunchKernelGGL(scene_task_kernel<true>, dim3(kTaskBlocks), dim3(256), 0, s, p);
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
 }
 
