@@ -189,7 +189,11 @@ struct Ctx {
   };
   std::vector<Timed> evPairs;
   std::map<std::string, std::pair<double, int64_t>> kernelTimes;  // last profile: ms, launches
-  std::map<int, uint32_t*> luts;  // per radius: device weight table of the blur kernels
+  struct BlurTable {
+    uint32_t* dev;  // weight table of the blur kernels
+    int32_t bias;   // BlurArgs::bias
+  };
+  std::map<int, BlurTable> luts;  // per radius
   std::string arch;               // gcnArchName of the device
   // Autotuner results: (arch, target w, h, format, calls, commands bucket)
   // -> (phase-A shape, ms per render)
@@ -232,7 +236,6 @@ int init() {
   PXH_HIP(hipMemsetAsync(g.touched, 0, sizeof(unsigned long long), g.stream));
   for (auto& e : g.ev) PXH_HIP(hipEventCreate(&e));
   if (set_fill_lds_limit(g.maxLds) != 0) return fail(kErrDevice, "hipFuncSetAttribute(fill)");
-  if (set_blur_lds_limit(g.maxLds) != 0) return fail(kErrDevice, "hipFuncSetAttribute(blur)");
   if (scene_set_lds_limits(g.maxLds) != 0) return fail(kErrDevice, "hipFuncSetAttribute(scene)");
   g.inited = true;
   return 0;
@@ -465,39 +468,43 @@ void gaussian_lut(int radius, std::vector<uint32_t>* out) {
   gaussian_lut_into(radius, f.data(), out->data());
 }
 
-int get_lut(int radius, uint32_t** dev) {
+// 128 * the sum of the taps (the blur kernels' pixels are signed) + 256 (the
+// division by 255 starts from the quotient plus one)
+template <class T>
+int32_t blur_bias(const T* taps, int n) {
+  int64_t sum = 0;
+  for (int i = 0; i < n; i++) sum += taps[i];
+  return (int32_t)(128 * sum + 256);
+}
+
+int get_lut(int radius, Ctx::BlurTable* out) {
   std::lock_guard<std::mutex> lock(g.lutMu);
   auto it = g.luts.find(radius);
   if (it != g.luts.end()) {
-    *dev = it->second;
+    *out = it->second;
     return 0;
   }
   // taps, then the weight table the blur kernels read (built on the device)
   std::vector<uint32_t> lut;
   gaussian_lut(radius, &lut);
-  const size_t tabWords = 8 * (size_t)blur_table_dwords(radius);
   uint32_t* p = nullptr;
-  PXH_HIP(hipMalloc((void**)&p, (lut.size() + tabWords) * 4));
+  PXH_HIP(hipMalloc((void**)&p, (lut.size() + blur_table_dwords(radius)) * 4));
   PXH_HIP(hipMemcpy(p, lut.data(), lut.size() * 4, hipMemcpyHostToDevice));
   if (launch_blur_table(p, radius, p + lut.size(), g.stream) != 0)
     return fail(kErrDevice, "blur table launch failed");
   PXH_HIP(hipStreamSynchronize(g.stream));
-  g.luts[radius] = p + lut.size();
-  *dev = p + lut.size();
+  *out = g.luts[radius] = Ctx::BlurTable{p + lut.size(), blur_bias(lut.data(), (int)lut.size())};
   return 0;
 }
 
-int blur_impl(uint32_t* src_dst, uint32_t* out, int32_t w, int32_t h, int radius, uint32_t oob,
-              bool shadowColor, uint32_t color, int lane = 0) {
-  if (blur_x_lds(radius) > g.maxLds || blur_y_lds(radius) > g.maxLds)
-    return fail(kErrCapacity, "blur radius too large for the LDS tiles");
-  uint32_t* wtab = nullptr;
-  if (int r = get_lut(radius, &wtab)) return r;
+int blur_impl(uint32_t* img, int32_t w, int32_t h, int radius, uint32_t oob, int lane = 0) {
+  if (!blur_radius_fits(radius, g.maxLds)) return fail(kErrCapacity, "blur radius too large for the LDS tiles");
+  Ctx::BlurTable t;
+  if (int r = get_lut(radius, &t)) return r;
   DevBuf& tmp = lane == 0 ? g.tmp : g.laneTmp[lane];
   if (int e = tmp.ensure((size_t)w * h * 4)) return fail(e, "blur temporary allocation failed");
-  const int nd = blur_table_dwords(radius);
-  BlurArgs ax{src_dst, (uint32_t*)tmp.p, wtab, w, h, radius, oob, 0, 0, nd};
-  BlurArgs ay{(uint32_t*)tmp.p, out, wtab, w, h, radius, oob, shadowColor ? 1 : 0, color, nd};
+  BlurArgs ax{img, (uint32_t*)tmp.p, t.dev, w, h, radius, oob, t.bias};
+  BlurArgs ay{(uint32_t*)tmp.p, img, t.dev, w, h, radius, oob, t.bias};
   if (launch_blur(ax, ay, g.lane[lane]) != 0) return fail(kErrDevice, "blur launch failed");
   return 0;
 }
@@ -1903,8 +1910,7 @@ int pxh_blur(pxh_image* img, float radius, uint32_t oob_rgbx) {
   if (r == 0) return 0;
   if (r < 0) return fail(kErrNegBlur, "Cannot apply negative blur");
   if (r > 1 << 20) return fail(kErrCapacity, "blur radius too large");
-  uint32_t* p = (uint32_t*)img->dev;
-  return blur_impl(p, p, img->w, img->h, (int)r, oob_rgbx, false, 0);
+  return blur_impl((uint32_t*)img->dev, img->w, img->h, (int)r, oob_rgbx);
 }
 
 // blur with no device allocation: the intermediate image and the table live
@@ -1920,9 +1926,8 @@ int pxh_blur_noalloc(pxh_image* img, float radius, uint32_t oob_rgbx) {
   if (r < 0) return fail(kErrNegBlur, "Cannot apply negative blur");
   if ((size_t)img->w * (size_t)img->h > kNoAllocBlurPixels)
     return fail(kErrCapacity, "image larger than the allocation-free blur's scratch (4194304 pixels)");
-  if (2 * r + 1 > (int64_t)kMaxLutTaps ||
-      2 * r + 1 + 8 * (int64_t)blur_table_dwords((int)r) > (int64_t)kNoAllocLutWords ||
-      blur_x_lds((int)r) > g.maxLds || blur_y_lds((int)r) > g.maxLds)
+  if (2 * r + 1 > (int64_t)kMaxLutTaps || !blur_radius_fits((int)r, g.maxLds) ||
+      2 * r + 1 + blur_table_dwords((int)r) > (int64_t)kNoAllocLutWords)
     return fail(kErrCapacity, "blur radius too large for the LDS tiles");
   uint32_t* base = g.scratchPtr[g.device];
   if (!base) return fail(kErrDevice, "allocation-free scratch is not set up on this device");
@@ -1936,9 +1941,9 @@ int pxh_blur_noalloc(pxh_image* img, float radius, uint32_t oob_rgbx) {
   if (launch_lut_store(taps, lut, g.stream) != 0 || launch_blur_table(lut, (int)r, wtab, g.stream) != 0)
     return fail(kErrDevice, "table store launch failed");
   uint32_t* p = (uint32_t*)img->dev;
-  const int nd = blur_table_dwords((int)r);
-  BlurArgs ax{p, tmp, wtab, img->w, img->h, (int32_t)r, oob_rgbx, 0, 0, nd};
-  BlurArgs ay{tmp, p, wtab, img->w, img->h, (int32_t)r, oob_rgbx, 0, 0, nd};
+  const int32_t bias = blur_bias(taps.v, taps.n);
+  BlurArgs ax{p, tmp, wtab, img->w, img->h, (int32_t)r, oob_rgbx, bias};
+  BlurArgs ay{tmp, p, wtab, img->w, img->h, (int32_t)r, oob_rgbx, bias};
   if (launch_blur(ax, ay, g.stream) != 0) return fail(kErrDevice, "blur launch failed");
   return 0;
 }
@@ -1952,8 +1957,7 @@ int pxh_blur_on(pxh_image* img, float radius, uint32_t oob_rgbx, int32_t lane) {
   if (r == 0) return 0;
   if (r < 0) return fail(kErrNegBlur, "Cannot apply negative blur");
   if (r > 1 << 20) return fail(kErrCapacity, "blur radius too large");
-  uint32_t* p = (uint32_t*)img->dev;
-  return blur_impl(p, p, img->w, img->h, (int)r, oob_rgbx, false, 0, lane);
+  return blur_impl((uint32_t*)img->dev, img->w, img->h, (int)r, oob_rgbx, lane);
 }
 
 int32_t pxh_lanes(void) { return kLanes; }
@@ -1991,16 +1995,22 @@ pxh_image* pxh_image_view(void* device_ptr, int32_t width, int32_t height, int32
   return img;
 }
 
+static int32_t spread_window(int64_t s, int32_t w, int32_t h) {
+  return (int32_t)std::min<int64_t>(s < 0 ? -s : s, std::max(w, h));  // no window reaches further
+}
+
 int pxh_spread(pxh_image* img, float spread) {
   PXH_INIT();
   if (int r = check_image(img)) return r;
   if (img->fmt != PXH_FORMAT_RGBA8) return fail(kErrArg, "spread needs an RGBA8 image");
   int64_t s = nim_f2i(roundf(spread));  // images.nim:702
   if (s == 0) return 0;
-  if (int e = g.plane.ensure((size_t)img->w * img->h)) return fail(e, "plane allocation failed");
-  SpreadArgs a{(const uint32_t*)img->dev, (uint8_t*)g.plane.p, (uint32_t*)img->dev, img->w, img->h,
-               (int32_t)(s > 0 ? s : -s), s > 0 ? 1 : 0, 0, 0};
-  if (launch_spread(a, g.stream) != 0) return fail(kErrDevice, "spread launch failed");
+  const int32_t pitch = plane_pitch(img->w);
+  if (int e = g.plane.ensure((size_t)pitch * img->h)) return fail(e, "plane allocation failed");
+  SpreadArgs a{(const uint32_t*)img->dev, (uint8_t*)g.plane.p, nullptr, (uint32_t*)img->dev, img->w, img->h, pitch,
+               spread_window(s, img->w, img->h), s > 0 ? 1 : 0, 0, 0};
+  if (launch_spread_x(a, g.stream) != 0 || launch_spread_y(a, true, g.stream) != 0)
+    return fail(kErrDevice, "spread launch failed");
   return 0;
 }
 
@@ -2015,12 +2025,13 @@ int pxh_shadow(pxh_image* out, const pxh_image* src, float offset_x, float offse
   int64_t br = nim_f2i(roundf(blur));
   if (br < 0) return fail(kErrNegBlur, "Cannot apply negative blur");
   const int32_t w = src->w, h = src->h;
-  if (int e = g.tmp2.ensure((size_t)w * h * 4)) return fail(e, "shadow temporary allocation failed");
-  uint32_t* mask = (uint32_t*)g.tmp2.p;
+  if (br != 0 && (br > 1 << 20 || !blur_radius_fits((int)br, g.maxLds)))
+    return fail(kErrCapacity, "blur radius too large for the LDS tiles");
   int64_t s = nim_f2i(roundf(spread));
   // mask = draw(image, translate(offset), OverwriteBlend) onto transparent
   // (images.nim:765-768): whole-pixel offsets fold into the spread pass's
-  // reads; fractional ones go through drawSmooth first
+  // reads; fractional ones go through drawSmooth first.  From there on only
+  // the mask's alpha is used, as a plane of bytes.
   const bool whole = offset_x == floorf(offset_x) && offset_y == floorf(offset_y) &&
                      fabsf(offset_x) < 1073741824.0f && fabsf(offset_y) < 1073741824.0f;
   const uint32_t* from = (const uint32_t*)src->dev;
@@ -2029,30 +2040,27 @@ int pxh_shadow(pxh_image* out, const pxh_image* src, float offset_x, float offse
     dx = (int32_t)offset_x;
     dy = (int32_t)offset_y;
   } else {
+    if (int e = g.tmp2.ensure((size_t)w * h * 4)) return fail(e, "shadow temporary allocation failed");
+    uint32_t* mask = (uint32_t*)g.tmp2.p;
     PXH_HIP(hipMemsetAsync(mask, 0, (size_t)w * h * 4, g.stream));
     const float t[9] = {1, 0, 0, 0, 1, 0, offset_x, offset_y, 1};
     if (int r = draw_transform_impl(mask, w, h, (const uint32_t*)src->dev, w, h, t, kOverwrite, false))
       return r;
-    from = mask;  // spread in place: its passes read and write different buffers
+    from = mask;
   }
-  SpreadArgs sa{from, nullptr, mask, w, h, (int32_t)(s > 0 ? s : -s), s > 0 ? 1 : 0, dx, dy};
-  if (!whole && s == 0) {
-    // the drawn mask is ready
-  } else if (s != 0) {
-    // mask = draw(image, translate(offset), OverwriteBlend); spread(mask)
-    if (int e = g.plane.ensure((size_t)w * h)) return fail(e, "plane allocation failed");
-    sa.plane = (uint8_t*)g.plane.p;
-    if (launch_spread(sa, g.stream) != 0) return fail(kErrDevice, "spread launch failed");
-  } else {
-    if (launch_shift(sa, g.stream) != 0) return fail(kErrDevice, "shift launch failed");
-  }
-  if (br != 0) {
-    // blur(mask); result = fill(color).draw(mask, MaskBlend), fused into the Y pass
-    return blur_impl(mask, (uint32_t*)out->dev, w, h, (int)br, 0u, true, rgbx);
-  }
-  if (int r = pxh_image_fill(out, rgbx)) return r;
-  CompositeArgs c{(uint32_t*)out->dev, mask, w, h, w, h, 0, 0, 0, w, 0, h, kMask};
-  if (launch_composite(c, false, g.stream) != 0) return fail(kErrDevice, "composite launch failed");
+  const int32_t pitch = plane_pitch(w);
+  const size_t bytes = (size_t)pitch * h;
+  if (int e = g.plane.ensure(s != 0 ? 2 * bytes : bytes)) return fail(e, "plane allocation failed");
+  uint8_t* plane = (uint8_t*)g.plane.p;
+  SpreadArgs sa{from, plane, plane + bytes, nullptr, w, h, pitch, spread_window(s, w, h), s >= 0 ? 1 : 0, dx, dy};
+  if (launch_spread_x(sa, g.stream) != 0 || (s != 0 && launch_spread_y(sa, false, g.stream) != 0))
+    return fail(kErrDevice, "spread launch failed");
+  // blur(mask); result = fill(color).draw(mask, MaskBlend)
+  Ctx::BlurTable t = {};
+  if (br != 0)
+    if (int r = get_lut((int)br, &t)) return r;
+  ShadowArgs a{s != 0 ? sa.plane2 : sa.plane, (uint32_t*)out->dev, t.dev, w, h, pitch, (int32_t)br, t.bias, rgbx};
+  if (launch_shadow(a, g.stream) != 0) return fail(kErrDevice, "shadow launch failed");
   return 0;
 }
 

@@ -36,12 +36,10 @@ struct CompositeArgs {
 struct BlurArgs {
   const uint32_t* src;
   uint32_t* dst;
-  const uint32_t* wtab;  // weight table of blur_table_kernel (device)
+  const uint32_t* wtab;  // table of blur_table_kernel (device)
   int32_t w, h, radius;
   uint32_t oob;
-  int32_t shadowColor;   // Y pass only: write blendMask(color, result)
-  uint32_t color;
-  int32_t nd;            // blur_table_dwords(radius)
+  int32_t bias;          // 128 * the sum of the taps + 256
 };
 
 // Gaussian taps passed by value (kernel arguments stay under 4 KB).
@@ -51,12 +49,24 @@ struct LutTaps {
   int32_t n;
 };
 
+// Alpha planes: rows of `pitch` bytes (a multiple of 16, zeros past w).
+inline int32_t plane_pitch(int32_t w) { return (w + 15) & ~15; }
 struct SpreadArgs {
   const uint32_t* src;
-  uint8_t* plane;        // alpha plane scratch (w*h)
-  uint32_t* dst;
-  int32_t w, h, s, grow;
+  uint8_t* plane;        // the X pass's result
+  uint8_t* plane2;       // the Y pass's (a shadow)
+  uint32_t* dst;         // the Y pass's (an image)
+  int32_t w, h, pitch, s, grow;
   int32_t dx, dy;        // read src translated by (dx, dy)
+};
+
+struct ShadowArgs {
+  const uint8_t* plane;
+  uint32_t* dst;
+  const uint32_t* wtab;  // table of blur_table_kernel (radius > 0)
+  int32_t w, h, pitch, radius;
+  int32_t bias;          // 128 * the sum of the taps + 256
+  uint32_t color;
 };
 
 // Non-solid paint over the whole canvas (fillPath's route, paths.nim:
@@ -84,16 +94,15 @@ int launch_fill_rows(const FillArgs& a, int grid, size_t ldsBytes, bool a8, hipS
 int set_fill_lds_limit(size_t bytes);
 int launch_composite(const CompositeArgs& a, bool srcA8, hipStream_t s);
 int launch_blur(const BlurArgs& ax, const BlurArgs& ay, hipStream_t s);
-int set_blur_lds_limit(size_t bytes);
+bool blur_radius_fits(int r, size_t lds);
 int launch_lut_store(const LutTaps& t, uint32_t* dst, hipStream_t s);
-// Weight table of a blur of radius r (2 * 4 * blur_table_dwords(r) dwords)
-// built on the device from its 2r + 1 taps.
+// Weight table of a blur of radius r (blur_table_dwords(r) dwords) built on
+// the device from its 2r + 1 taps.
 int blur_table_dwords(int r);
 int launch_blur_table(const uint32_t* lut, int r, uint32_t* wtab, hipStream_t s);
-size_t blur_x_lds(int r);
-size_t blur_y_lds(int r);
-int launch_spread(const SpreadArgs& a, hipStream_t s);
-int launch_shift(const SpreadArgs& a, hipStream_t s);
+int launch_spread_x(const SpreadArgs& a, hipStream_t s);
+int launch_spread_y(const SpreadArgs& a, bool image, hipStream_t s);
+int launch_shadow(const ShadowArgs& a, hipStream_t s);
 int launch_opacity(uint32_t* img, int64_t n, uint32_t o, hipStream_t s);
 int launch_blend_pixels(const uint32_t* b, const uint32_t* s_, uint32_t* out, int64_t n,
                         int32_t mode, hipStream_t s);
