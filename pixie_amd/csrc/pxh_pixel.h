@@ -17,12 +17,41 @@
 
 namespace pxh {
 
+// x div 255 for x < 65535, without the multiplication that the compiler's
+// division takes (a quarter of the other instructions' rate).
+PXH_HD uint32_t div255(uint32_t x) { return (x + 1u + (x >> 8)) >> 8; }
+
+// (c * k + add) div 255 of each of a pixel's channels, k and add < 256: pairs
+// of channels in 16-bit halves (c * k + add + 1 + 254 < 2^16).
+PXH_HD uint32_t mul_div255(uint32_t c, uint32_t k, uint32_t add) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  const unsigned short k16 = (unsigned short)k, a16 = (unsigned short)add;
+  const u16x2 kk = {k16, k16}, aa = {a16, a16}, one = {1, 1}, eight = {8, 8};
+  u16x2 e = __builtin_bit_cast(u16x2, c & 0x00ff00ffu) * kk + aa;
+  u16x2 o = __builtin_bit_cast(u16x2, (c >> 8) & 0x00ff00ffu) * kk + aa;
+  e = e + one + (e >> eight);
+  o = o + one + (o >> eight);
+  // the results are the halves' high bytes
+  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, o), __builtin_bit_cast(uint32_t, e), 0x07030501u);
+#else
+  return pack(div255(ch_r(c) * k + add), div255(ch_g(c) * k + add), div255(ch_b(c) * k + add),
+              div255(ch_a(c) * k + add));
+#endif
+}
+
+// a + b of each channel, modulo 256
+PXH_HD uint32_t add_channels(uint32_t a, uint32_t b) {
+  return (((a & 0x00ff00ffu) + (b & 0x00ff00ffu)) & 0x00ff00ffu) |
+         (((a & 0xff00ff00u) + (b & 0xff00ff00u)) & 0xff00ff00u);
+}
+
 // `*`(ColorRGBX, uint8) common.nim:79-90, generalised to any uint32 factor x
 // (the float-opacity product common.nim:67-77 computes x = round(o*255) and
 // the same (c*x+127) div 255, wrapping modulo 2^32).
 PXH_HD uint32_t mul_cov(uint32_t c, uint32_t x) {
-  if (x == 0) return 0;
-  if (x == 255) return c;
+  // 0 gives 0 and 255 gives c, as the reference's shortcuts do
+  if (x <= 255u) return mul_div255(c, x, 127u);
   uint32_t r = (ch_r(c) * x + 127u) / 255u;
   uint32_t g = (ch_g(c) * x + 127u) / 255u;
   uint32_t b = (ch_b(c) * x + 127u) / 255u;
@@ -40,7 +69,7 @@ PXH_HD uint32_t area_factor(float area) {
 }
 
 PXH_HD uint32_t blend_alpha(uint32_t ba, uint32_t sa) {  // blends.nim:41-43
-  return (sa + ((ba * ((255u - sa) & 255u)) / 255u)) & 255u;
+  return (sa + div255(ba * ((255u - sa) & 255u))) & 255u;
 }
 
 PXH_HD uint32_t screen_c(uint32_t b, uint32_t s) {  // blends.nim:45-46
@@ -222,9 +251,7 @@ PXH_HD uint32_t blend(int32_t mode, uint32_t b, uint32_t s) {
     case kNormal: {  // 60-70
       if (ba == 0 || sa == 255) return s;
       if (sa == 0) return b;
-      uint32_t k = 255u - sa;
-      return pack(sr + (br * k) / 255u, sg + (bg * k) / 255u, sb + (bb * k) / 255u,
-                  blend_alpha(ba, sa));
+      return add_channels(s, mul_div255(b, 255u - sa, 0u));
     }
     case kDarken:
     case kLighten: {  // 72-84, 128-140
@@ -300,7 +327,7 @@ PXH_HD uint32_t blend(int32_t mode, uint32_t b, uint32_t s) {
     case kLuminosity:
       return blend_float(mode, b, s);
     case kMask:  // 227-232
-      return pack((br * sa) / 255u, (bg * sa) / 255u, (bb * sa) / 255u, (ba * sa) / 255u);
+      return mul_div255(b, sa, 0u);
     case kOverwrite:
       return s;
     case kSubtractMask: {  // 234-239
