@@ -178,7 +178,7 @@ struct Ctx {
   int32_t* laneErr = nullptr;
   std::set<pxh_scene*> scenes;  // live scenes (their pools are re-validated after an error)
   std::mutex scenesMu;
-  unsigned long long* touched = nullptr;  // N_touch counter of fills
+  unsigned long long* touched = nullptr;  // N_touch of fills: kTouchSlots counters, 8 words apart
   hipEvent_t ev[16] = {};
   // per-launch kernel timing (pxh_profile_begin / _end)
   bool profiling = false;
@@ -232,8 +232,8 @@ int init() {
   // kLanes words read at synchronize, then kLanes that checked renders write
   PXH_HIP(hipMalloc((void**)&g.laneErr, 2 * kLanes * sizeof(int32_t)));
   PXH_HIP(hipMemsetAsync(g.laneErr, 0, 2 * kLanes * sizeof(int32_t), g.stream));
-  PXH_HIP(hipMalloc((void**)&g.touched, sizeof(unsigned long long)));
-  PXH_HIP(hipMemsetAsync(g.touched, 0, sizeof(unsigned long long), g.stream));
+  PXH_HIP(hipMalloc((void**)&g.touched, kTouchSlots * 64));
+  PXH_HIP(hipMemsetAsync(g.touched, 0, kTouchSlots * 64, g.stream));
   for (auto& e : g.ev) PXH_HIP(hipEventCreate(&e));
   if (set_fill_lds_limit(g.maxLds) != 0) return fail(kErrDevice, "hipFuncSetAttribute(fill)");
   if (scene_set_lds_limits(g.maxLds) != 0) return fail(kErrDevice, "hipFuncSetAttribute(scene)");
@@ -310,6 +310,8 @@ int next_pow2(int v) {
   return p;
 }
 
+constexpr size_t kCuLds = 160 * 1024;  // LDS of a CU
+
 // Largest number of band entries any row of the fill selects (entries with
 // to.y > y and at.y < y + 1, the row program's selection), by a difference
 // array over each band's rows.
@@ -378,10 +380,20 @@ int raster_fill(pxh_image* img, FillGeom& geo) {
   // The row arrays hold one row's selection (the band entries that meet
   // [y, y + 1)), not the whole band: size them for the largest selection.
   const int maxSel = max_row_selection(geo);
-  const int ww = 512;
   const int cap = next_pow2(maxSel > 2 ? maxSel : 2);
-  const size_t fixedBytes = 8 * (size_t)ww + 16;
   const size_t capBytes = (size_t)cap * 24;
+  // Every window of a row repeats the row's hits and walk, so windows are made
+  // wider, up to 1,536 px, while the rows still give each CU the 12 waves that
+  // its registers hold, the LDS of 12 waves fits it, and no row selects more
+  // than 64 entries (beyond, the sample lines' keys hold positions in 512 px).
+  // A rounded rectangle over 3,686 x 3,686: 68 us in 512-px windows, 45 us in
+  // 1,024-px ones.
+  const int64_t spanPx = mask ? img->w : f.xhi - (f.xlo & ~3);
+  int ww = 512;
+  while (maxSel <= 64 && ww < 1536 && nRows * ((spanPx + ww + 511) / (ww + 512)) >= (int64_t)g.numCUs * 12 &&
+         12 * (8 * (size_t)(ww + 512) + 16 + capBytes) <= kCuLds)
+    ww += 512;
+  const size_t fixedBytes = 8 * (size_t)ww + 16;
   FillArgs a;
   a.F = (const FillInfo*)dp[0];
   a.parts = (const PartInfo*)dp[1];
@@ -1590,7 +1602,7 @@ static int draw_transform_impl(uint32_t* dst, int32_t aw, int32_t ah, const uint
   if (int e = g.drawRows.ensure(spanBytes + (size_t)ah * sa.nRuns * sizeof(float2)))
     return fail(e, "draw scratch allocation failed");
   sa.span = (int2*)g.drawRows.p;
-  sa.starts = (float2*)(g.drawRows.p + spanBytes);
+  sa.starts = (float*)(g.drawRows.p + spanBytes);
   if (launch_draw_smooth(sa, g.stream) != 0) return fail(kErrDevice, "draw launch failed");
   return 0;
 }
@@ -2371,11 +2383,13 @@ int pxh_scene_debug_geometry(pxh_scene* sc, int32_t i, int32_t* info16, int32_t*
 // the last reset (N_touch, the unit of the fill throughput metric).
 int pxh_touched_pixels(int64_t* out, int32_t reset) {
   PXH_INIT();
-  unsigned long long v = 0;
-  PXH_HIP(hipMemcpyAsync(&v, g.touched, sizeof(v), hipMemcpyDeviceToHost, g.stream));
+  std::vector<unsigned long long> v(kTouchSlots * 8);
+  PXH_HIP(hipMemcpyAsync(v.data(), g.touched, kTouchSlots * 64, hipMemcpyDeviceToHost, g.stream));
   PXH_HIP(hipStreamSynchronize(g.stream));
-  *out = (int64_t)v;
-  if (reset) PXH_HIP(hipMemsetAsync(g.touched, 0, sizeof(unsigned long long), g.stream));
+  unsigned long long sum = 0;
+  for (int i = 0; i < kTouchSlots; i++) sum += v[8 * (size_t)i];
+  *out = (int64_t)sum;
+  if (reset) PXH_HIP(hipMemsetAsync(g.touched, 0, kTouchSlots * 64, g.stream));
   return 0;
 }
 

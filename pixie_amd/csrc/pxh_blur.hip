@@ -25,7 +25,6 @@ namespace pxh {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));  // four pixels, wherever they start
 
 // ---------------------------------------------------------------------------
 // weights

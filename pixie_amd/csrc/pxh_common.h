@@ -97,6 +97,8 @@ PXH_HD uint32_t ch_a(uint32_t c) { return c >> 24; }
 // Device data layout of a fill (one fillShapes call)
 // ---------------------------------------------------------------------------
 
+constexpr int kTouchSlots = 512;  // counters of written pixels (touched_slot), 8 words apart
+
 // Per-fill header: the locals fillShapes derives before its scanline loop
 // (paths.nim:1602-1629), plus the paint.
 struct FillInfo {

@@ -29,8 +29,8 @@ struct MagnifyArgs {
 };
 
 // drawSmooth (images.nim:531-634) of src onto dst.  Rows are cut into runs
-// of kSmoothRun pixels; the running sample position at each run's start is
-// kept in `starts` (ah x nRuns).
+// of kSmoothRun pixels, at multiples of it; the running sample position at
+// each run's first pixel of the row's span is kept in `starts` (nRuns x 2 x ah).
 constexpr int kSmoothRun = 16;
 struct SmoothArgs {
   uint32_t* dst;
@@ -41,7 +41,7 @@ struct SmoothArgs {
   int32_t yStart, yEnd;       // clamped row range of the perimeter
   int32_t mode;
   int2* span;                 // per row: [xStart, xEnd) (scratch, ah entries)
-  float2* starts;             // per row and run: the start position (scratch)
+  float* starts;              // per run: its start's x in every row, then its y (scratch)
   int32_t nRuns;              // ceil(aw / kSmoothRun)
 };
 

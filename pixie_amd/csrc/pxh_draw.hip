@@ -24,10 +24,12 @@ namespace pxh {
 
 // mix(ColorRGBX, ColorRGBX, t), common.nim:59-65
 __device__ __forceinline__ uint32_t mix_rgbx(uint32_t a, uint32_t b, float t) {
-  const uint32_t x = nim_f2u32(roundf(t * 255.0f));
-  const uint32_t y = 255u - x;
-  return pack((ch_r(a) * y + ch_r(b) * x + 127u) / 255u, (ch_g(a) * y + ch_g(b) * x + 127u) / 255u,
-              (ch_b(a) * y + ch_b(b) * x + 127u) / 255u, (ch_a(a) * y + ch_a(b) * x + 127u) / 255u);
+  const float v = t * 255.0f;  // t in [0, 1): round half up is roundf
+  const uint32_t n = (uint32_t)v;
+  const uint32_t x = n + (v - (float)n >= 0.5f ? 1u : 0u);
+  // sums of two products of weights that add up to 255, plus 127: 16 bits,
+  // as the division's intermediate
+  return mix_div255(a, 255u - x, b, x);
 }
 
 // `*`(ColorRGBX, float32) for the constant opacities minifyBy2 uses
@@ -185,14 +187,14 @@ __device__ uint32_t wrapped_sample(const DrawSrc& s, float x, float y) {
 
 // ---------------------------------------------------------------------------
 // drawSmooth in three steps.  Each row's sample positions are the running sum
-// srcPos += dx from its first pixel, which float32 only reproduces when summed
-// in order, so:
-//   smooth_rows_kernel    one thread per row: the row's span from the
-//                         perimeter, then the running sum along it, storing
-//                         every kSmoothRun-th position (the start of each run)
-//   smooth_runs_kernel    one thread per run of kSmoothRun pixels: continues
-//                         the sum from the run's stored start, samples and
-//                         blends
+// srcPos += dx from its first pixel, in float32, so:
+//   smooth_rows_kernel    two threads per row (x and y): the row's span from
+//                         the perimeter, then the running sum along it,
+//                         storing the position at every multiple of
+//                         kSmoothRun and at the span's first pixel (the
+//                         starts of its runs)
+//   smooth_tiles_kernel   a wave per tile of pixels: continues the sums from
+//                         the runs' starts, samples and blends
 //   smooth_clear_kernel   MaskBlend only: clears the rows outside [yStart,
 //                         yEnd) and each row outside its span, skipping rows
 //                         whose span is empty (images.nim:560-561, 598-626)
@@ -216,7 +218,8 @@ __device__ __forceinline__ bool scan_hit(const float* seg, float ly, float* atx,
 }
 
 __global__ void __launch_bounds__(64) smooth_rows_kernel(SmoothArgs a) {
-  const int32_t y = blockIdx.x * 64 + threadIdx.x;
+  const int32_t y = blockIdx.x * 32 + (threadIdx.x & 31);
+  const int32_t axis = threadIdx.x >> 5;
   if (y >= a.ah) return;
   int32_t s = 0, e = 0;
   if (y >= a.yStart && y < a.yEnd) {
@@ -240,103 +243,112 @@ __global__ void __launch_bounds__(64) smooth_rows_kernel(SmoothArgs a) {
     s = a.aw;  // cleared whole: a span that ends before it starts
     e = 0;
   }
-  a.span[y] = make_int2(s, e);
+  if (axis == 0) a.span[y] = make_int2(s, e);
+  if (e <= s) return;
   // srcPos = p + dx * xStart + dy * y, then - h (images.nim:593-594)
-  float sx = a.p[0] + a.dx[0] * (float)s + a.dy[0] * (float)y;
-  float sy = a.p[1] + a.dx[1] * (float)s + a.dy[1] * (float)y;
-  sx = sx - 0.5f;
-  sy = sy - 0.5f;
-  float2* starts = a.starts + (size_t)y * a.nRuns;
-  const int32_t len = e - s;
-  const float ddx = a.dx[0], ddy = a.dx[1];
-  int32_t j = 0;
-  for (; j + kSmoothRun <= len; j += kSmoothRun) {
-    starts[j / kSmoothRun] = make_float2(sx, sy);
+  float p = a.p[axis] + a.dx[axis] * (float)s + a.dy[axis] * (float)y;
+  p = p - 0.5f;
+  // the x and the y sum are chains of dependent additions: a lane each.
+  // Neighbouring rows are neighbouring lanes and neighbours in memory.
+  float* starts = a.starts + (size_t)axis * a.ah + y;
+  const float d = a.dx[axis];
+  int32_t r = s / kSmoothRun, x = s;
+  starts[(size_t)2 * r * a.ah] = p;
+  for (int32_t next = (r + 1) * kSmoothRun; x < next; x++) p += d;
+  for (; x < e; x += kSmoothRun) {
+    r++;
+    starts[(size_t)2 * r * a.ah] = p;
 #pragma unroll
-    for (int k = 0; k < kSmoothRun; k++) {
-      sx += ddx;
-      sy += ddy;
-    }
+    for (int k = 0; k < kSmoothRun; k++) p += d;
   }
-  if (j < len) starts[j / kSmoothRun] = make_float2(sx, sy);
 }
 
-__device__ __noinline__ uint32_t blend_call(int32_t mode, uint32_t b, uint32_t s) { return blend(mode, b, s); }
-
-// A wave takes 64 consecutive runs of a row (64 * kSmoothRun pixels).  Each
-// lane continues the running sum along its own run and leaves the positions
-// in LDS; the wave then works through the pixels in order, lane l taking
-// pixel 64 j + l at step j, so that neighbouring lanes read neighbouring
-// source and destination pixels.  Three straight-line phases let the loads
-// issue together: every source read (pixels past the span read clamped
-// in-bounds addresses and are discarded), the bilinear mixes, then the
-// destination reads, blends and writes.
-__global__ void __launch_bounds__(64) smooth_runs_kernel(SmoothArgs a) {
-  __shared__ float2 pos[64 * kSmoothRun];
-  const int32_t y = blockIdx.y;
+// A wave takes a tile of 64 x 16 pixels: lane (row, quarter) continues the
+// running sum along its run of 16 and leaves the positions in LDS; the wave
+// then works through the tile in pieces of 16 x 4 pixels, four at a time, so
+// that a piece of a turned picture lies in about 14 of the source's lines
+// (128 bytes), not the 40 of 64 pixels in a row.  Straight-line phases let the
+// loads issue together: source reads (pixels outside the span read clamped
+// in-bounds addresses and are discarded), the mixes, destination reads, blends
+// and writes.  A 3,000 x 3,000 picture turned by 30 degrees onto 4,096 x
+// 4,096, Normal: 118 us by rows, 85 us by tiles (bound by the arithmetic of
+// the mixes).  The rows' sums: 26 us with x and y in one lane, 17 in two; a sum
+// that jumps through a binade by its constant step and stores scattered starts
+// took 75.
+constexpr int kTileW = 64, kTileH = 16, kPosStride = 66;
+__global__ void __launch_bounds__(64) smooth_tiles_kernel(SmoothArgs a) {
+  __shared__ float2 pos[kTileH * kPosStride];
+  __shared__ int2 spans[kTileH];
   const int32_t lane = threadIdx.x;
-  const int2 sp = a.span[y];
-  const int32_t xw = sp.x + blockIdx.x * 64 * kSmoothRun;  // the wave's first pixel
-  if (xw >= sp.y) return;                                  // uniform over the block
-  const int32_t run = blockIdx.x * 64 + lane;
-  float2 p = run < a.nRuns ? a.starts[(size_t)y * a.nRuns + run] : make_float2(0.0f, 0.0f);
+  const int32_t xt = blockIdx.x * kTileW, yt = (a.yStart & ~(kTileH - 1)) + blockIdx.y * kTileH;
+  {
+    const int32_t row = lane & 15, run = lane >> 4, y = yt + row;
+    int2 sp = make_int2(0, 0);
+    if (y < a.ah) sp = a.span[y];
+    const int32_t x = xt + run * kSmoothRun;
+    const bool meets = sp.x < x + kSmoothRun && sp.y > x && sp.x < sp.y;
+    if (__ballot(meets) == 0) return;  // the same in every lane
+    if (run == 0) spans[row] = sp;
+    float2 p = make_float2(0.0f, 0.0f);
+    if (meets) {
+      const float* starts = a.starts + (size_t)2 * (xt / kSmoothRun + run) * a.ah + y;
+      p = make_float2(starts[0], starts[a.ah]);
+    }
+    const int32_t skip = meets && sp.x > x ? sp.x - x : 0;  // pixels before the span
 #pragma unroll
-  for (int k = 0; k < kSmoothRun; k++) {
-    pos[lane * kSmoothRun + k] = p;
-    p.x += a.dx[0];
-    p.y += a.dx[1];
+    for (int k = 0; k < kSmoothRun; k++) {
+      pos[row * kPosStride + run * kSmoothRun + k] = p;
+      if (k >= skip) {
+        p.x += a.dx[0];
+        p.y += a.dx[1];
+      }
+    }
   }
   __syncthreads();
   const DrawSrc src = a.src;
   const uint32_t W = (uint32_t)src.w << src.mag, H = (uint32_t)src.h << src.mag;
-  uint32_t q[kSmoothRun][4];
-  float xf[kSmoothRun], yf[kSmoothRun];
+  const int32_t lx = lane & 15, ly = lane >> 4;
+  for (int32_t row = ly; row < kTileH; row += 4) {
+    const int2 sp = spans[row];
+    uint32_t q[4][4];
+    float xf[4], yf[4];
 #pragma unroll
-  for (int j = 0; j < kSmoothRun; j++) {
-    const float2 v = pos[j * 64 + lane];
-    const float fx = floorf(v.x), fy = floorf(v.y);
-    xf[j] = v.x - fx;
-    yf[j] = v.y - fy;
-    const int32_t px0 = pixel_coord(fx), py0 = pixel_coord(fy);
-    const bool vx0 = (uint32_t)px0 < W, vx1 = (uint32_t)(px0 + 1) < W;
-    const bool vy0 = (uint32_t)py0 < H, vy1 = (uint32_t)(py0 + 1) < H;
-    const uint32_t c0 = vx0 ? (uint32_t)px0 >> src.mag : 0u, c1 = vx1 ? (uint32_t)(px0 + 1) >> src.mag : 0u;
-    const size_t r0 = vy0 ? (size_t)((uint32_t)py0 >> src.mag) * src.w : 0;
-    const size_t r1 = vy1 ? (size_t)((uint32_t)(py0 + 1) >> src.mag) * src.w : 0;
-    const uint32_t a00 = src.px[r0 + c0], a10 = src.px[r0 + c1];
-    const uint32_t a01 = src.px[r1 + c0], a11 = src.px[r1 + c1];
-    q[j][0] = (vx0 && vy0) ? a00 : 0u;
-    q[j][1] = (vx1 && vy0) ? a10 : 0u;
-    q[j][2] = (vx0 && vy1) ? a01 : 0u;
-    q[j][3] = (vx1 && vy1) ? a11 : 0u;
+    for (int j = 0; j < 4; j++) {
+      const float2 v = pos[row * kPosStride + 16 * j + lx];
+      const float fx = floorf(v.x), fy = floorf(v.y);
+      xf[j] = v.x - fx;
+      yf[j] = v.y - fy;
+      const int32_t px0 = pixel_coord(fx), py0 = pixel_coord(fy);
+      const bool vx0 = (uint32_t)px0 < W, vx1 = (uint32_t)(px0 + 1) < W;
+      const bool vy0 = (uint32_t)py0 < H, vy1 = (uint32_t)(py0 + 1) < H;
+      const uint32_t c0 = vx0 ? (uint32_t)px0 >> src.mag : 0u, c1 = vx1 ? (uint32_t)(px0 + 1) >> src.mag : 0u;
+      const size_t r0 = vy0 ? (size_t)((uint32_t)py0 >> src.mag) * src.w : 0;
+      const size_t r1 = vy1 ? (size_t)((uint32_t)(py0 + 1) >> src.mag) * src.w : 0;
+      const uint32_t a00 = src.px[r0 + c0], a10 = src.px[r0 + c1];
+      const uint32_t a01 = src.px[r1 + c0], a11 = src.px[r1 + c1];
+      q[j][0] = (vx0 && vy0) ? a00 : 0u;
+      q[j][1] = (vx1 && vy0) ? a10 : 0u;
+      q[j][2] = (vx0 && vy1) ? a01 : 0u;
+      q[j][3] = (vx1 && vy1) ? a11 : 0u;
+    }
+    u32x4 smp;
+#pragma unroll
+    for (int j = 0; j < 4; j++) smp[j] = bilinear(q[j][0], q[j][1], q[j][2], q[j][3], xf[j], yf[j]);
+    uint32_t* dst = a.dst + (size_t)(yt + row) * a.aw + xt + lx;
+    bool in[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) in[j] = xt + 16 * j + lx >= sp.x && xt + 16 * j + lx < sp.y;
+    if (a.mode != kOverwrite) {
+      u32x4 d;
+#pragma unroll
+      for (int j = 0; j < 4; j++) d[j] = in[j] ? dst[16 * j] : 0u;
+      blend4(a.mode, &d, smp);
+      smp = d;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (in[j]) dst[16 * j] = smp[j];
   }
-  uint32_t smp[kSmoothRun];
-#pragma unroll
-  for (int j = 0; j < kSmoothRun; j++) smp[j] = bilinear(q[j][0], q[j][1], q[j][2], q[j][3], xf[j], yf[j]);
-  uint32_t* row = a.dst + (size_t)y * a.aw;
-  const int32_t lim = sp.y;  // pixels at or past the span's end are not touched
-  if (a.mode == kOverwrite) {
-#pragma unroll
-    for (int j = 0; j < kSmoothRun; j++)
-      if (xw + j * 64 + lane < lim) row[xw + j * 64 + lane] = smp[j];
-    return;
-  }
-  uint32_t d[kSmoothRun];
-#pragma unroll
-  for (int j = 0; j < kSmoothRun; j++) {
-    const int32_t x = xw + j * 64 + lane;
-    d[j] = row[x < lim ? x : xw];
-  }
-  if (a.mode == kNormal) {
-#pragma unroll
-    for (int j = 0; j < kSmoothRun; j++) d[j] = blend(kNormal, d[j], smp[j]);
-  } else {
-#pragma unroll
-    for (int j = 0; j < kSmoothRun; j++) d[j] = blend_call(a.mode, d[j], smp[j]);
-  }
-#pragma unroll
-  for (int j = 0; j < kSmoothRun; j++)
-    if (xw + j * 64 + lane < lim) row[xw + j * 64 + lane] = d[j];
 }
 
 __global__ void __launch_bounds__(256) smooth_clear_kernel(SmoothArgs a) {
@@ -349,8 +361,11 @@ __global__ void __launch_bounds__(256) smooth_clear_kernel(SmoothArgs a) {
 }
 
 int launch_draw_smooth(const SmoothArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(smooth_rows_kernel, dim3((a.ah + 63) / 64), dim3(64), 0, s, a);
-  hipLaunchKernelGGL(smooth_runs_kernel, dim3((a.nRuns + 63) / 64, a.ah), dim3(64), 0, s, a);
+  hipLaunchKernelGGL(smooth_rows_kernel, dim3((a.ah + 31) / 32), dim3(64), 0, s, a);
+  const int32_t y0 = a.yStart & ~(kTileH - 1), nRows = (a.yEnd < a.ah ? a.yEnd : a.ah) - y0;
+  if (nRows > 0)
+    hipLaunchKernelGGL(smooth_tiles_kernel, dim3((a.aw + kTileW - 1) / kTileW, (nRows + kTileH - 1) / kTileH), dim3(64),
+                       0, s, a);
   if (a.mode == kMask)
     hipLaunchKernelGGL(smooth_clear_kernel, dim3((a.aw + 255) / 256, a.ah), dim3(256), 0, s, a);
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
@@ -369,7 +384,7 @@ __global__ void __launch_bounds__(256) draw_correct_kernel(CorrectArgs a) {
   const uint32_t s = a.wrapped ? wrapped_sample(a.src, sx - 0.5f, sy - 0.5f)
                                : smooth_sample(a.src, sx - 0.5f, sy - 0.5f);
   uint32_t* d = a.dst + (size_t)y * a.aw + x;
-  *d = a.mode == kNormal ? blend(kNormal, *d, s) : blend_call(a.mode, *d, s);
+  *d = blend(a.mode, *d, s);
 }
 
 int launch_draw_correct(const CorrectArgs& a, hipStream_t s) {

@@ -40,6 +40,25 @@ PXH_HD uint32_t mul_div255(uint32_t c, uint32_t k, uint32_t add) {
 #endif
 }
 
+// (a * ka + b * kb + 127) div 255 of each channel, ka + kb = 255
+PXH_HD uint32_t mix_div255(uint32_t a, uint32_t ka, uint32_t b, uint32_t kb) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+  const unsigned short ka16 = (unsigned short)ka, kb16 = (unsigned short)kb;
+  const u16x2 va = {ka16, ka16}, vb = {kb16, kb16}, half = {127, 127}, one = {1, 1}, eight = {8, 8};
+  u16x2 e = __builtin_bit_cast(u16x2, a & 0x00ff00ffu) * va + half;
+  u16x2 o = __builtin_bit_cast(u16x2, (a >> 8) & 0x00ff00ffu) * va + half;
+  e = __builtin_bit_cast(u16x2, b & 0x00ff00ffu) * vb + e;
+  o = __builtin_bit_cast(u16x2, (b >> 8) & 0x00ff00ffu) * vb + o;
+  e = e + one + (e >> eight);
+  o = o + one + (o >> eight);
+  return __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, o), __builtin_bit_cast(uint32_t, e), 0x07030501u);
+#else
+  return pack(div255(ch_r(a) * ka + ch_r(b) * kb + 127u), div255(ch_g(a) * ka + ch_g(b) * kb + 127u),
+              div255(ch_b(a) * ka + ch_b(b) * kb + 127u), div255(ch_a(a) * ka + ch_a(b) * kb + 127u));
+#endif
+}
+
 // a + b of each channel, modulo 256
 PXH_HD uint32_t add_channels(uint32_t a, uint32_t b) {
   return (((a & 0x00ff00ffu) + (b & 0x00ff00ffu)) & 0x00ff00ffu) |
@@ -342,5 +361,22 @@ PXH_HD uint32_t blend(int32_t mode, uint32_t b, uint32_t s) {
       return b;
   }
 }
+
+#if defined(__HIPCC__) || defined(__HIP__)
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));  // four pixels, wherever they start
+
+// Four pixels with one choice of the mode, which is the same in every lane.
+template <int M = 0>
+__device__ __forceinline__ void blend4(int32_t mode, u32x4* b, u32x4 s) {
+  if constexpr (M < kNumBlendModes) {
+    if (mode == M) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) (*b)[k] = blend(M, (*b)[k], s[k]);
+    } else {
+      blend4<M + 1>(mode, b, s);
+    }
+  }
+}
+#endif
 
 }  // namespace pxh

@@ -162,7 +162,10 @@ constexpr int kBandTilesMax = 4096;
 // every fetch.
 constexpr int kQueues = 16;
 constexpr int kQueueStride = 64;  // ints between queue heads (256 B)
-// Queue sets: phase A's heavy rows, its other rows, phase B.
+// The first set of queue heads' place holds the counts of runs written.
+constexpr int kUsedSlots = 64;
+static_assert(kUsedSlots * 16 <= kQueues * kQueueStride, "the counts fit");
+// Sets: the counts of runs, phase A's rows, phase B.
 constexpr int kQueueSets = 3;
 
 // Grid of a queue-fed kernel: at least one wave per queue, a multiple of
@@ -239,7 +242,7 @@ struct ScenePools {
   int32_t* binList;          // call indices per bin
   int32_t binCap;
   int32_t binSlots;          // capacity of binCount / binOff (bins)
-  int32_t* queues;           // work-queue heads: 2 phases x kQueues, one per 256 B
+  int32_t* queues;           // kUsedSlots counts of runs, then work-queue heads: 2 phases x kQueues, one per 256 B
   int32_t* counters;         // SceneCounter
   // row scratch for bands larger than the LDS capacity
   char* gscratch;

@@ -18,8 +18,6 @@ constexpr int kStrokeGrid = 2048;  // workgroups of the stroke segment kernels (
 constexpr int kSegBandBlocks = 2048;  // workgroups of the band ranges (a wave per 64 segments)
 constexpr int kTaskBlocks = 1024;     // workgroups of the work-item kernels (a wave per 64 units)
 
-// A value that is the same in every lane, moved to a scalar register.
-__device__ __forceinline__ int32_t uni(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
 constexpr int kWinA = 512;    // phase-A column window
 constexpr int kWinB = 512;    // phase-B column window (2 chunks of 256 px)
 constexpr int kChunksB = kWinB / 256;
@@ -1788,6 +1786,13 @@ __device__ __forceinline__ int queue_next(int32_t* heads, int n) {
   return item < n ? (int)item : n;
 }
 
+// Where this workgroup counts the runs it wrote: one of kUsedSlots, 64 bytes
+// apart, which the composition adds up.  Thousands of waves that end together
+// and add to one address wait 10 to 20 ns each.
+__device__ __forceinline__ int32_t* used_slot(const ScenePools& P) {
+  return P.queues + (blockIdx.x % kUsedSlots) * 16;
+}
+
 // Takes n entries of a pool counter for the whole wave (also with every lane
 // in the atomic; once per chunk of runs).
 __device__ __forceinline__ int queue_take(int32_t* counter, int n) {
@@ -2309,7 +2314,7 @@ __global__ void __launch_bounds__(kHeavyThreads, 5) scene_heavy_kernel(ScenePool
       P.tasks[first + wave] = rr;  // every lane stores the same value
     }
   }
-  if (lane == 0 && rc.used) atomicAdd(&P.counters[kCntRunsUsed], rc.used);
+  if (lane == 0 && rc.used) atomicAdd(used_slot(P), rc.used);
 }
 
 __global__ void __launch_bounds__(64, 4) scene_rows_kernel(ScenePools P) {
@@ -2394,7 +2399,7 @@ __global__ void __launch_bounds__(64, 4) scene_rows_kernel(ScenePools P) {
       P.tasks[task] = rr;  // every lane stores the same value
     }
   }
-  if (threadIdx.x == 0 && rc.used) atomicAdd(&P.counters[kCntRunsUsed], rc.used);
+  if (threadIdx.x == 0 && rc.used) atomicAdd(used_slot(P), rc.used);
 }
 
 // ---------------------------------------------------------------------------
@@ -2424,6 +2429,10 @@ __global__ void __launch_bounds__(64) scene_compose_kernel(ScenePools P, void* c
   const int nUnits = H * winsPerRow;
   const bool vec = ((W & 3) == 0);
   uint32_t ntouch = 0;
+  if (blockIdx.x == 0) {  // the runs written, for the host
+    const int32_t used = wave_incl_sum(P.queues[lane * 16]);
+    if (lane == kWave - 1) P.counters[kCntRunsUsed] = used;
+  }
   if (const int32_t err = P.counters[kCntError]) {
     // an earlier stage ran out of a pool: the canvas stays untouched and the
     // error reaches the host through the lane's error word
@@ -2705,7 +2714,7 @@ __global__ void __launch_bounds__(64) scene_compose_kernel(ScenePools P, void* c
   if (touchedOut) {
     ntouch = (uint32_t)wave_incl_sum((int32_t)ntouch);
     ntouch = __builtin_amdgcn_readlane(ntouch, kWave - 1);
-    if (lane == 0 && ntouch) atomicAdd(touchedOut, (unsigned long long)ntouch);
+    if (lane == 0 && ntouch) atomicAdd(touched_slot(touchedOut), (unsigned long long)ntouch);
   }
 }
 
