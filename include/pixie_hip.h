@@ -187,8 +187,8 @@ int pxh_scene_stroke_path(pxh_scene* scene, const float* cmds, int32_t ncmds, co
 int pxh_scene_render(pxh_scene* scene, pxh_image* img);
 /* Autotuner (no reference counterpart): renders the scene onto a scratch
  * image of img's size with each phase-A launch shape (band entries kept in
- * LDS x row waves per CU, and whether tasks of large bands run in a launch
- * of their own), `reps` timed renders each, and keeps the fastest for later
+ * LDS, row waves per CU, and the size of band from which a workgroup takes a
+ * row), `reps` timed renders each, and keeps the fastest for later
  * renders.  *shape receives its index, *ms its time per render.  Results are
  * cached for the process, keyed by device arch, target size and format, and
  * the scene's call count and command count (to a power of two): a scene of

@@ -79,7 +79,7 @@ struct pxh_scene {
   pxh::ScenePools pools{};
   int32_t ptCap = 0, segCap = 0, bandCap = 0, entryCap = 0, taskCap = 0, runCap = 0, binCap = 0;
   int32_t binSlots = 0;  // row bins the pools hold (height / kBinRows)
-  int32_t gcap = 8192;   // band entries a large-band wave can hold in global row scratch
+  int32_t gcap = 8192;   // band entries a wave of the rows kernel can hold in global row scratch
 };
 
 namespace pxh {
@@ -546,9 +546,9 @@ int blur_impl(uint32_t* img, int32_t w, int32_t h, int radius, uint32_t oob, int
 
 // ---- scene (batched form) ----
 
-// A row whose selection exceeds the large-band launch's LDS capacity keeps
+// A row whose selection exceeds the rows kernel's LDS capacity keeps
 // its arrays in global row scratch, one slot of gcap entries per wave of that
-// launch.  gcap starts at 8192 and grows with the largest band a validated
+// kernel.  gcap starts at 8192 and grows with the largest band a validated
 // render meets, up to kMaxSceneGcap and 8 GiB of slots in all.
 const int kMaxSceneGcap = 1 << 18;
 

@@ -4,12 +4,16 @@
 // A scene is an ordered list of fillPath / strokePath calls whose canonical
 // commands stay resident in HBM.  Each render runs on the device:
 //   geometry  one workgroup per call: adaptive flattening (count -> scan ->
-//             emit), stroke expansion, shapesToSegments, bounds, band layout
-//   bands     one wave per y-band: ordered entry lists (partitionSegments)
+//             emit), shapesToSegments, bounds, band layout; strokes in
+//             chunks of their points
+//   bands     ordered entry lists of every y-band (partitionSegments), in
+//             tiles of bands, and the calls of every 16 canvas rows
+//   tasks     phase A's work items by cost, longest first
 //   rows      phase A: every (call, row, window) row program in parallel,
-//             each leaving its pixel codes as sparse (x, delta) runs
-//   compose   phase B: each wave owns a canvas row window in registers and
-//             applies the runs of every call covering it, in call order
+//             each leaving its pixel codes as sparse (x, delta) runs; rows
+//             of the largest bands take a workgroup
+//   compose   phase B: each wave owns a canvas row window in LDS and applies
+//             the runs of every call covering it, in call order
 #pragma once
 
 #include <hip/hip_runtime.h>
