@@ -662,7 +662,12 @@ __device__ __forceinline__ void walk32_borders(bool fillStart, bool fillEnd, int
   if (fillEnd) atomicAdd(&D[hi], -kSampleCov);
 }
 
-// A row window's place for the 32-bit walks.
+// A row window's place for the 32-bit walks, which take windows that end below
+// kWin32End: its 24.8 bounds must not leave 32 bits.  (Positions of 2^23 px
+// and more saturate to the lowest number, as pixie's conversion does; in a
+// window below them they count as hits left of it, which is where pixie's sort
+// puts them.)  The lines of a window beyond are walked whole.
+constexpr int32_t kWin32End = 1 << 23;
 struct Win32 {
   int32_t A, A1, B;  // 24.8 bounds of its hits (a hit at or left of x = 0 only counts)
   int32_t lo, hi;    // columns the coverage may write, from the window's start
@@ -1206,7 +1211,9 @@ __device__ int32_t row_program(const RowCtx& C, RowLds& L) {
     if (mask && lane == 0) add_run(C, L, covLo, covHi, -kClear);  // coverage range
     CovSpan cs{&C, &L, kSampleCov, (int32_t)covLo, (int32_t)covHi};
     uint32_t whole;
-    if (ne <= 8) {
+    if (Cp.wx1 >= kWin32End) {
+      whole = 0x1fu;
+    } else if (ne <= 8) {
       whole = row_coverage_seg<8>(Cp, L, ne, S, yLine, offset, F.rule);
     } else if (ne <= 16) {
       whole = row_coverage_seg<16>(Cp, L, ne, S, yLine, offset, F.rule);
