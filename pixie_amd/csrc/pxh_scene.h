@@ -20,6 +20,7 @@
 #include <stdint.h>
 
 #include "pxh_common.h"
+#include "pxh_queue.h"
 
 namespace pxh {
 
@@ -161,11 +162,6 @@ constexpr int kCounterInts = kNumCounters + 2 * kCostClasses;
 constexpr int kBinRows = 16;
 constexpr int kBandTilesMax = 4096;
 
-// Phase A and B deal out work through kQueues independent queues (queue q
-// serves work items q, q + kQueues, ...), so that no single counter takes
-// every fetch.
-constexpr int kQueues = 16;
-constexpr int kQueueStride = 64;  // ints between queue heads (256 B)
 // The first set of queue heads' place holds the counts of runs written.
 constexpr int kUsedSlots = 64;
 static_assert(kUsedSlots * 16 <= kQueues * kQueueStride, "the counts fit");

@@ -1759,33 +1759,6 @@ __global__ void __launch_bounds__(256) scene_band_kernel(ScenePools P, int binBl
 // phase A: row programs of every (call, row, window) -> sparse runs
 // ---------------------------------------------------------------------------
 
-// Next work item of this wave's queue, or a value >= n when it is empty.
-// The items are dealt to the kQueues queues in granules of G consecutive
-// items, round robin; a queue hands its items out in order.  Workgroups go
-// to the XCDs round robin, so queue q is served by XCD q % 8 alone: a
-// granule's items (neighbouring rows of one call, in phase A) share that
-// XCD's L2.
-// Every lane takes part in the atomic and the first lane's old value is taken:
-// broadcasting through LDS from a lane-0-only branch is not safe, because
-// __syncthreads() compiles to nothing in a one-wave workgroup and the compiler
-// may then let lanes 1..63 loop back to the LDS read without lane 0, spinning
-// on a stale value.  Every lane adds 1, so that a head counts in 64ths of an
-// item (to 2^26 items a queue): with the same value in every lane the compiler
-// sends one addition of 64, where a value of 1 in lane 0 and 0 elsewhere made
-// it sum the lanes in a loop of 64 rounds and 20 instructions, for every item.
-// 8,192 glyphs on 8,192 x 8,192: the composition 395 -> 279 us, the row
-// programs 516 -> 469 us.
-template <int G = 1>
-__device__ __forceinline__ int queue_next(int32_t* heads, int n) {
-  const int q = (int)(blockIdx.x % kQueues);
-  const uint32_t old = (uint32_t)atomicAdd(heads + q * kQueueStride, 1);
-  // the same in every lane: keep it (and what derives from it) scalar
-  const int k = (int)((uint32_t)__builtin_amdgcn_readfirstlane((int)old) >> 6);
-  // the item is increasing in k, so a queue is empty once one is >= n
-  const int64_t item = ((int64_t)(k / G) * kQueues + q) * G + k % G;
-  return item < n ? (int)item : n;
-}
-
 // Where this workgroup counts the runs it wrote: one of kUsedSlots, 64 bytes
 // apart, which the composition adds up.  Thousands of waves that end together
 // and add to one address wait 10 to 20 ns each.
