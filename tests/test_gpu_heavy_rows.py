@@ -1,6 +1,6 @@
 """Rows of bands with hundreds of entries in the batched form (the workgroup
-row kernel) against the per-call form, which runs the one-wave row program on
-the same shapes: the images must be equal byte for byte."""
+row kernel) against the oracle and against the per-call form, which runs the
+one-wave row program on the same shapes: the images must be equal byte for byte."""
 import numpy as np
 import pytest
 
@@ -35,11 +35,14 @@ def closed(shapes):
     return [np.concatenate([s, s[:1]]) for s in shapes]
 
 
-def both(px, shapes, w, h, rule, mode, a8=False):
+def both(px, orc, shapes, w, h, rule, mode, a8=False):
     color = (200, 90, 30, 220)
     back = np.random.default_rng(1).integers(0, 256, (h, w) if a8 else (h, w, 4), dtype=np.uint8)
     if not a8:
         back[..., :3] = np.minimum(back[..., :3], back[..., 3:])
+    want = np.repeat(back[..., None], 4, 2) if a8 else back.copy()
+    orc.fill_path(want, shape_cmds(shapes), color, winding=rule, mode=mode)
+    want = want[..., 3] if a8 else want
     one, two = px.Image.from_array(back), px.Image.from_array(back)
     one.fillShapes(closed(shapes), color, windingRule=rule, blendMode=mode)
     sc = px.Scene()
@@ -47,6 +50,7 @@ def both(px, shapes, w, h, rule, mode, a8=False):
     sc.render(two)
     a, b = one.download(), two.download()
     assert np.array_equal(a, b), "%d of %d bytes differ" % ((a != b).sum(), a.size)
+    assert np.array_equal(a, want), "%d of %d bytes differ from the oracle" % ((a != want).sum(), a.size)
     two.upload(back)
     sc.render(two)  # a replay
     assert np.array_equal(a, two.download())
@@ -75,24 +79,24 @@ def cases():
 
 @pytest.mark.parametrize("rule", [0, 1])
 @pytest.mark.parametrize("name,shapes,w,h", list(cases()), ids=[c[0] for c in cases()])
-def test_heavy_rows(gpu, name, shapes, w, h, rule):
-    both(gpu, shapes, w, h, rule, 0)
+def test_heavy_rows(gpu, orc, name, shapes, w, h, rule):
+    both(gpu, orc, shapes, w, h, rule, 0)
 
 
 @pytest.mark.parametrize("mode", [16, 17])
-def test_heavy_rows_mask_and_overwrite(gpu, mode):
-    both(gpu, [teeth(600, 30, 2500, 3, 40, 0.4, 1)], 2600, 48, 0, mode)
+def test_heavy_rows_mask_and_overwrite(gpu, orc, mode):
+    both(gpu, orc, [teeth(600, 30, 2500, 3, 40, 0.4, 1)], 2600, 48, 0, mode)
 
 
-def test_heavy_rows_a8(gpu):
-    both(gpu, [teeth(600, 30, 2500, 3, 40, 0.4, 1)], 2600, 48, 0, 0, a8=True)
+def test_heavy_rows_a8(gpu, orc):
+    both(gpu, orc, [teeth(600, 30, 2500, 3, 40, 0.4, 1)], 2600, 48, 0, 0, a8=True)
 
 
-def test_heavy_rows_sample_lines_through_vertices(gpu):
+def test_heavy_rows_sample_lines_through_vertices(gpu, orc):
     # beyond y = 4096 float32 rounds the middle sample line onto y + 0.5, so
     # vertices there count twice and a line's windings do not sum to 0
     z = teeth(600, 10, 900, 4100, 4140, 0.0, 2)
     z[:, 1] = np.floor(z[:, 1]) + 0.5
     mid = z.copy()
     mid[::2, 1] -= 20.0
-    both(gpu, [z, mid], 950, 4160, 0, 0)
+    both(gpu, orc, [z, mid], 950, 4160, 0, 0)

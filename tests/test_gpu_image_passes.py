@@ -1,6 +1,8 @@
 """Image passes at the edges of their tiles and vectors, against the oracle:
-transformed draws over long rows (the jumped running sum of positions, tiles
-cut by spans and borders), integer draws at every offset within a vector, and opacities.  All equal byte for byte."""
+transformed draws over long rows (the running sums of positions from run to run,
+tiles cut by spans and borders), integer draws at every offset within a vector,
+opacities, and per-call fills by the width of their windows.  All equal byte for
+byte."""
 import math
 
 import numpy as np
@@ -72,9 +74,9 @@ def test_opacity(gpu, orc, o):
 
 @pytest.mark.parametrize("teeth", [0, 1, 12, 31, 32, 33, 60])
 @pytest.mark.parametrize("w,h", [(500, 3300), (1537, 3100), (2049, 3100), (3300, 1600)])
-def test_window_widths(gpu, w, h, teeth):
+def test_window_widths(gpu, orc, w, h, teeth):
     """Per-call fills in windows of 512 to 1,536 px, of few and many entries a
-    row, against the recorded form (windows of 512 px)."""
+    row, against the oracle and the recorded form (windows of 512 px)."""
     d = "M 5.5 3 L %s 2.25 Q %s %s %s %s L 2 %s Z" % (w - 4, w - 1, h / 2, w - 9.5, h - 3, h - 1.5)
     for k in range(teeth):
         x = 20 + k * (w - 60) / teeth
@@ -87,4 +89,7 @@ def test_window_widths(gpu, w, h, teeth):
         sc.fillPath(d, color, blendMode=mode, windingRule=1)
         two = px.Image.from_array(base)
         sc.render(two)
-        assert np.array_equal(img.download(), two.download())
+        got, want = img.download(), base.copy()
+        assert np.array_equal(got, two.download())
+        orc.fill_path(want, d, color, winding=1, mode=mode)
+        assert np.array_equal(got, want)
