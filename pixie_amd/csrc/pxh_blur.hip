@@ -415,8 +415,9 @@ int launch_lut_store(const LutTaps& t, uint32_t* dst, hipStream_t s) {
 // spread, on alpha bytes in a plane whose rows are padded with zeros to a
 // multiple of 16.  The window is clamped to the image.  A negative spread
 // takes the least of the window: the greatest of the complements.  Bytes are
-// compared as the 16-bit halves of even and odd bytes.  1,921 x 1,081, spread
-// 4: 9 us (X, it reads the RGBA8) and 8 us; a pixel to a thread, 16 and 13 us.
+// compared as the 16-bit halves of even and odd bytes.  Bound by latency at the
+// sizes of layers, so each pass has several loads in flight.  1,921 x 1,081,
+// both passes: 16 us at spread 4 and 31 at 20; a pixel to a thread 27 and 82.
 // ---------------------------------------------------------------------------
 struct MaxBytes {
   u16x2 even = {0, 0}, odd = {0, 0};
@@ -430,26 +431,47 @@ struct MaxBytes {
   }
 };
 
-// The alphas of four pixels from x of a row of the translated source, flipped
-// by `flip` inside the image and 0 outside it.
-__device__ __forceinline__ uint32_t alphas4(const SpreadArgs& a, const uint32_t* row, int32_t x, uint32_t flip) {
+// Four pixels from x of a row of the translated source: loaded at once, or
+// one by one at clamped addresses where they reach over a border (kSingles:
+// always, so that lanes at a border and lanes inside take one way), so that
+// several of these are in flight before the first is used.
+struct Quad {
+  u32x4 v;
+  bool inside;
+};
+template <bool kSingles>
+__device__ __forceinline__ Quad load_quad(const SpreadArgs& a, const uint32_t* row, int32_t x) {
   const int32_t sx = x - a.dx;
-  if (x >= 0 && x + 4 <= a.w && row && sx >= 0 && sx + 4 <= a.w) {
-    const u32x4 v = *(const u32x4*)(row + sx);
-    return (__builtin_amdgcn_perm(v[1], v[0], 0x0c0c0703u) | __builtin_amdgcn_perm(v[3], v[2], 0x07030c0cu)) ^ flip;
-  }
-  uint32_t out = 0;
+  Quad q;
+  q.inside = x >= 0 && x + 4 <= a.w && row && sx >= 0 && sx + 4 <= a.w;
+  if (!kSingles && q.inside) {
+    q.v = *(const u32x4*)(row + sx);
+  } else {
+    const uint32_t* from = row ? row : a.src;
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    if (x + i < 0 || x + i >= a.w) continue;
-    uint32_t al = 0;
-    if (row && sx + i >= 0 && sx + i < a.w) al = row[sx + i] >> 24;
-    out |= (al ^ (flip & 255u)) << (8 * i);
+    for (int i = 0; i < 4; i++) q.v[i] = from[sx + i < 0 ? 0 : sx + i < a.w ? sx + i : a.w - 1];
   }
-  return out;
+  return q;
+}
+// Their alphas, flipped by `flip` inside the image and 0 outside it.
+__device__ __forceinline__ uint32_t alphas4(const SpreadArgs& a, const uint32_t* row, int32_t x, const Quad& q,
+                                            uint32_t flip) {
+  uint32_t out = __builtin_amdgcn_perm(q.v[1], q.v[0], 0x0c0c0703u) | __builtin_amdgcn_perm(q.v[3], q.v[2], 0x07030c0cu);
+  if (!q.inside) {
+    const int32_t sx = x - a.dx;
+    uint32_t in = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      if (!(row && sx + i >= 0 && sx + i < a.w)) out &= ~(255u << (8 * i));
+      if (x + i >= 0 && x + i < a.w) in |= 255u << (8 * i);
+    }
+    return (out ^ flip) & in;
+  }
+  return out ^ flip;
 }
 
 // X pass, four pixels to a thread; s = 0 only takes the translated alphas.
+template <bool kSingles>
 __global__ void __launch_bounds__(256) spread_x_kernel(SpreadArgs a) {
   const int32_t y = blockIdx.y, x = ((int32_t)blockIdx.x * 256 + (int32_t)threadIdx.x) * 4;
   if (x >= a.pitch) return;
@@ -463,15 +485,27 @@ __global__ void __launch_bounds__(256) spread_x_kernel(SpreadArgs a) {
     int32_t m0 = -((s + 3) / 4), m1 = s / 4;
     m0 = m0 < -x / 4 - 1 ? -x / 4 - 1 : m0;
     m1 = m1 > (a.w - 1 - x) / 4 ? (a.w - 1 - x) / 4 : m1;
-    uint32_t cur = alphas4(a, row, x + 4 * m0, flip);
+    auto get = [&](int32_t m, const Quad& q) { return alphas4(a, row, x + 4 * m, q, flip); };
+    Quad q0 = load_quad<kSingles>(a, row, x + 4 * m0);
     MaxBytes best;
-    for (int32_t m = m0; m <= m1; m++) {
-      const uint32_t next = s ? alphas4(a, row, x + 4 * (m + 1), flip) : 0u;
+    auto take = [&](int32_t m, uint32_t cur, uint32_t next) {
       if (4 * m >= -s) best.add(cur);
       if (4 * m + 1 >= -s && 4 * m + 1 <= s) best.add(__builtin_amdgcn_alignbyte(next, cur, 1));
       if (4 * m + 2 >= -s && 4 * m + 2 <= s) best.add(__builtin_amdgcn_alignbyte(next, cur, 2));
       if (4 * m + 3 >= -s && 4 * m + 3 <= s) best.add(__builtin_amdgcn_alignbyte(next, cur, 3));
-      cur = next;
+    };
+    if (s == 0) {
+      best.add(get(0, q0));
+    } else {
+      uint32_t cur = 0;
+      for (int32_t m = m0; m <= m1; m += 2) {
+        const Quad q1 = load_quad<kSingles>(a, row, x + 4 * (m + 1)), q2 = load_quad<kSingles>(a, row, x + 4 * (m + 2));
+        if (m == m0) cur = get(m, q0);
+        const uint32_t n1 = get(m + 1, q1), n2 = get(m + 2, q2);
+        take(m, cur, n1);
+        if (m < m1) take(m + 1, n1, n2);
+        cur = n2;
+      }
     }
     out = best.get() ^ flip;
     if (x + 4 > a.w) out &= (1u << (8 * (a.w - x))) - 1u;
@@ -479,26 +513,33 @@ __global__ void __launch_bounds__(256) spread_x_kernel(SpreadArgs a) {
   *(uint32_t*)(a.plane + (size_t)y * a.pitch + x) = out;
 }
 
-// Y pass, four pixels of four rows to a thread: into the second plane, or
+// Y pass, four pixels of kRows rows to a thread: into the second plane, or
 // into an image of black with that alpha.
-template <bool kImage>
+template <bool kImage, int kRows>
 __global__ void __launch_bounds__(256) spread_y_kernel(SpreadArgs a) {
-  const int32_t y0 = (int32_t)blockIdx.y * 4, x = ((int32_t)blockIdx.x * 256 + (int32_t)threadIdx.x) * 4;
+  const int32_t y0 = (int32_t)blockIdx.y * kRows, x = ((int32_t)blockIdx.x * 256 + (int32_t)threadIdx.x) * 4;
   if (x >= (kImage ? a.w : a.pitch)) return;
   const uint32_t flip = a.grow ? 0u : ~0u;
   const int32_t s = a.s;
-  const int32_t lo = y0 - s > 0 ? y0 - s : 0, hi = (int64_t)y0 + 3 + s < a.h - 1 ? y0 + 3 + s : a.h - 1;
-  MaxBytes best[4];
-  for (int32_t yy = lo; yy <= hi; yy++) {
-    const uint32_t v = *(const uint32_t*)(a.plane + (size_t)yy * a.pitch + x) ^ flip;
+  const int32_t lo = y0 - s > 0 ? y0 - s : 0, hi = (int64_t)y0 + kRows - 1 + s < a.h - 1 ? y0 + kRows - 1 + s : a.h - 1;
+  MaxBytes best[kRows];
+  for (int32_t yb = lo; yb <= hi; yb += 4) {  // four rows in flight; the last again past the end
+    uint32_t v[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int32_t d = yy - (y0 + i);
-      if (d >= -s && d <= s) best[i].add(v);
+    for (int u = 0; u < 4; u++)
+      v[u] = *(const uint32_t*)(a.plane + (size_t)(yb + u < hi ? yb + u : hi) * a.pitch + x) ^ flip;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int32_t yy = yb + u < hi ? yb + u : hi;
+#pragma unroll
+      for (int i = 0; i < kRows; i++) {
+        const int32_t d = yy - (y0 + i);
+        if (d >= -s && d <= s) best[i].add(v[u]);
+      }
     }
   }
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
+  for (int i = 0; i < kRows; i++) {
     if (y0 + i >= a.h) break;
     const uint32_t v = best[i].get() ^ flip;
     if (!kImage) {
@@ -516,16 +557,32 @@ __global__ void __launch_bounds__(256) spread_y_kernel(SpreadArgs a) {
   }
 }
 
+// A small image does not fill the chip with four rows to a thread, and each of
+// its waves reaches over a border: its Y pass takes a row to a thread, its X
+// pass loads single pixels.  257 x 199, spread 1 and 20: 5.9 and 12.1 us,
+// 6.8 and 15.9 as larger images; 1,023 x 767 fills the chip either way.
+constexpr int64_t kSmallPlane = 1 << 19;  // bytes
 int launch_spread_x(const SpreadArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(spread_x_kernel, dim3((a.pitch + 1023) / 1024, a.h), dim3(256), 0, s, a);
+  const dim3 grid((a.pitch + 1023) / 1024, a.h);
+  if ((int64_t)a.pitch * a.h <= kSmallPlane)
+    hipLaunchKernelGGL(spread_x_kernel<true>, grid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL(spread_x_kernel<false>, grid, dim3(256), 0, s, a);
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
 }
-int launch_spread_y(const SpreadArgs& a, bool image, hipStream_t s) {
-  const dim3 grid((a.pitch + 1023) / 1024, (a.h + 3) / 4);
+template <int kRows>
+static void go_spread_y(const SpreadArgs& a, bool image, hipStream_t s) {
+  const dim3 grid((a.pitch + 1023) / 1024, (a.h + kRows - 1) / kRows);
   if (image)
-    hipLaunchKernelGGL(spread_y_kernel<true>, grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((spread_y_kernel<true, kRows>), grid, dim3(256), 0, s, a);
   else
-    hipLaunchKernelGGL(spread_y_kernel<false>, grid, dim3(256), 0, s, a);
+    hipLaunchKernelGGL((spread_y_kernel<false, kRows>), grid, dim3(256), 0, s, a);
+}
+int launch_spread_y(const SpreadArgs& a, bool image, hipStream_t s) {
+  if ((int64_t)a.pitch * a.h <= kSmallPlane)
+    go_spread_y<1>(a, image, s);
+  else
+    go_spread_y<4>(a, image, s);
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
 }
 

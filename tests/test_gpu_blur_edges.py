@@ -31,6 +31,7 @@ def picture(w, h, seed):
 
 
 SIZES = [(1, 1), (2, 63), (3, 5), (47, 49), (48, 48), (64, 64), (65, 33), (97, 193), (195, 130), (256, 70)]
+PLANES = SIZES + [(1040, 520), (1041, 517)]  # and beyond the small alpha planes
 
 
 @pytest.mark.parametrize("w,h", SIZES)
@@ -44,7 +45,7 @@ def test_blur(gpu, orc, r, w, h):
     assert np.array_equal(img.download(), want)
 
 
-@pytest.mark.parametrize("w,h", SIZES)
+@pytest.mark.parametrize("w,h", PLANES)
 @pytest.mark.parametrize("s", [1, 2, 3, 4, 5, 8, 31, 300, -1, -2, -7, -300])
 def test_spread(gpu, orc, s, w, h):
     a = picture(w, h, abs(s))
@@ -55,7 +56,7 @@ def test_spread(gpu, orc, s, w, h):
     assert np.array_equal(img.download(), want)
 
 
-@pytest.mark.parametrize("w,h", SIZES)
+@pytest.mark.parametrize("w,h", PLANES)
 @pytest.mark.parametrize("offset,spread,blur", [((0, 0), 0, 0), ((1, -2), 0, 1), ((7, 3), 3, 0), ((-5, 2), 2, 8),
                                                 ((2.5, -5.25), 0, 16), ((64, 1), -2, 17), ((0, 3), 1, 24),
                                                 ((2, 2), 5, 40), ((3, 900), 1, 2)])
