@@ -141,16 +141,19 @@ struct Ctx {
   // take turns in slots 1 .. kStageSlots - 1, so that a fill is prepared and
   // queued while those before it run; a larger one takes slot 0, whose size
   // follows it.  A frame of 24 calls on 1,280 x 720: 827 us with one slot,
-  // 643 us with these.
+  // 643 us with these.  The small slots lie in one allocation on either side,
+  // made for the first of them: one by one they made each of the first eight
+  // calls of a process wait for two allocations (150 us each, not 60).
   struct StageSlot {
     char* host = nullptr;
     size_t hostCap = 0;
-    DevBuf dev;
+    char* dev = nullptr;
     hipEvent_t free = nullptr;
   };
   static constexpr int kStageSlots = 9;
   static constexpr size_t kSmallStage = 256 << 10;
   StageSlot stage[kStageSlots];
+  DevBuf stageDev;   // slot 0's
   unsigned stageTurn = 0;
   DevBuf gscratch;   // per-workgroup row scratch when it does not fit in LDS
   // Execution lanes: independent streams (lane 0 is `stream`), each with its
@@ -271,23 +274,39 @@ int stage(const std::vector<std::pair<const void*, size_t>>& parts, std::vector<
     total += (p.second + 255) & ~(size_t)255;
   }
   const bool small = total <= Ctx::kSmallStage;
+  if (small && !g.stage[1].host) {
+    const size_t all = (Ctx::kStageSlots - 1) * Ctx::kSmallStage;
+    char *host = nullptr, *dev = nullptr;
+    PXH_HIP(hipMalloc((void**)&dev, all));
+    if (hipHostMalloc((void**)&host, all, hipHostMallocDefault) != hipSuccess) {
+      (void)hipFree(dev);
+      return fail(kErrNoMem, "host staging allocation failed");
+    }
+    for (int i = 1; i < Ctx::kStageSlots; i++) {
+      g.stage[i].host = host + (i - 1) * Ctx::kSmallStage;
+      g.stage[i].dev = dev + (i - 1) * Ctx::kSmallStage;
+    }
+  }
   Ctx::StageSlot& slot = g.stage[small ? 1 + g.stageTurn++ % (Ctx::kStageSlots - 1) : 0];
   PXH_HIP(hipEventSynchronize(slot.free));
-  if (total > slot.hostCap) {
-    if (slot.host) PXH_HIP(hipHostFree(slot.host));
-    slot.host = nullptr;
-    slot.hostCap = 0;
-    const size_t c = small ? Ctx::kSmallStage : total + total / 2 + (1 << 20);
-    PXH_HIP(hipHostMalloc((void**)&slot.host, c, hipHostMallocDefault));
-    slot.hostCap = c;
+  if (!small) {
+    if (total > slot.hostCap) {
+      if (slot.host) PXH_HIP(hipHostFree(slot.host));
+      slot.host = nullptr;
+      slot.hostCap = 0;
+      const size_t c = total + total / 2 + (1 << 20);
+      PXH_HIP(hipHostMalloc((void**)&slot.host, c, hipHostMallocDefault));
+      slot.hostCap = c;
+    }
+    if (int r = g.stageDev.ensure(total)) return fail(r, "device staging allocation failed");
+    slot.dev = g.stageDev.p;
   }
-  if (int r = slot.dev.ensure(small ? Ctx::kSmallStage : total)) return fail(r, "device staging allocation failed");
   for (size_t i = 0; i < parts.size(); i++)
     if (parts[i].second) memcpy(slot.host + offs[i], parts[i].first, parts[i].second);
-  PXH_HIP(hipMemcpyAsync(slot.dev.p, slot.host, total, hipMemcpyHostToDevice, g.stream));
+  PXH_HIP(hipMemcpyAsync(slot.dev, slot.host, total, hipMemcpyHostToDevice, g.stream));
   *free = slot.free;
   out->clear();
-  for (size_t i = 0; i < parts.size(); i++) out->push_back(slot.dev.p + offs[i]);
+  for (size_t i = 0; i < parts.size(); i++) out->push_back(slot.dev + offs[i]);
   return 0;
 }
 
