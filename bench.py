@@ -84,8 +84,8 @@ def timed(px, fn, steps, profile=True):
     return wall, touched, stages
 
 
-STAGES = ("fill_rows_kernel", "scene_geometry", "scene_bands", "scene_bins", "scene_rows_kernel",
-          "scene_compose_kernel")
+STAGES = ("fill_rows_kernel", "scene_geometry", "scene_bands", "scene_bins", "scene_heavy_kernel",
+          "scene_rows_kernel", "scene_compose_kernel")
 
 
 def glyph_extra(px, WL, reps=5, cpu_seconds=5.0):

@@ -443,8 +443,8 @@ int pxh_event_elapsed(int32_t a, int32_t b, float* ms);
 int pxh_profile_begin(void);
 int pxh_profile_end(double* kernel_ms, int64_t* launches);
 /* The share of one kernel (or scene stage) in the last profile: names are
- * fill_rows_kernel, scene_geometry, scene_bands, scene_rows_kernel,
- * scene_compose_kernel. */
+ * fill_rows_kernel, scene_geometry, scene_bands, scene_bins (the work items),
+ * scene_heavy_kernel, scene_rows_kernel, scene_compose_kernel. */
 int pxh_profile_kernel(const char* name, double* kernel_ms, int64_t* launches);
 
 /* Host geometry of one fillPath (stroke = 0) or strokePath (stroke = 1) call

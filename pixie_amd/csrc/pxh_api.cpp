@@ -1162,6 +1162,10 @@ int scene_launch(pxh_scene* sc, pxh_image* img, int lane, bool checked = false) 
     r = scene_launch_tasks(p, st);
   }
   if (!r) {
+    LaunchTimer t("scene_heavy_kernel", st);
+    r = scene_launch_heavy(p, g.numCUs, st);
+  }
+  if (!r) {
     LaunchTimer t("scene_rows_kernel", st);
     r = scene_launch_rows(p, shape, g.numCUs, st);
   }

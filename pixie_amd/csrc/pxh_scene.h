@@ -287,7 +287,8 @@ int scene_launch_clear(const ScenePools& p, hipStream_t s);
 int scene_launch_geometry(const ScenePools& p, hipStream_t s);
 int scene_launch_bands(const ScenePools& p, hipStream_t s);  // band entries and row bins
 int scene_launch_tasks(const ScenePools& p, hipStream_t s);  // phase A's work items and their order
-// Phase A in the given shape: the heavy rows, then the others.
+// Phase A: the rows of the largest bands, then the others in the given shape.
+int scene_launch_heavy(const ScenePools& p, int numCUs, hipStream_t s);
 int scene_launch_rows(const ScenePools& p, const RowShape& shape, int numCUs, hipStream_t s);
 int scene_launch_compose(const ScenePools& p, void* canvas, bool a8, unsigned long long* touched,
                          int32_t* errOut, int grid, hipStream_t s);

@@ -2828,9 +2828,13 @@ int scene_launch_tasks(const ScenePools& p, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
 }
 
-int scene_launch_rows(const ScenePools& p, const RowShape& shape, int numCUs, hipStream_t s) {
+int scene_launch_heavy(const ScenePools& p, int numCUs, hipStream_t s) {
   hipLaunchKernelGGL(scene_heavy_kernel, dim3(scene_queue_grid(numCUs * kHeavyGroupsPerCU)), dim3(kHeavyThreads), 0,
                      s, p);
+  return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
+}
+
+int scene_launch_rows(const ScenePools& p, const RowShape& shape, int numCUs, hipStream_t s) {
   const size_t lds = row_lds_fixed_bytes(kWinA) + row_cap_bytes(shape.ldsCap);
   hipLaunchKernelGGL(scene_rows_kernel, dim3(scene_queue_grid(numCUs * shape.wavesPerCU)), dim3(64), lds, s, p);
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;

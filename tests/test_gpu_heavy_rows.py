@@ -100,3 +100,15 @@ def test_heavy_rows_sample_lines_through_vertices(gpu, orc):
     mid = z.copy()
     mid[::2, 1] -= 20.0
     both(gpu, orc, [z, mid], 950, 4160, 0, 0)
+
+
+def test_profile_names_each_row_kernel(gpu):
+    sc, img = gpu.Scene(), gpu.Image(2600, 48)
+    sc.fillPath(shape_cmds([teeth(600, 30, 2500, 3, 40, 0.4, 1)]), (200, 90, 30, 220))
+    sc.render(img)
+    gpu.profile_begin()
+    sc.render(img)
+    gpu.profile_end()
+    for name in ("scene_heavy_kernel", "scene_rows_kernel"):
+        ms, launches = gpu.profile_kernel(name)
+        assert launches == 1 and ms > 0, (name, ms, launches)
