@@ -393,32 +393,11 @@ int max_row_selection(const FillGeom& geo) {
   return best;
 }
 
-// Launches the raster of one built fill onto img.
-int raster_fill(pxh_image* img, FillGeom& geo) {
-  FillInfo& f = geo.info;
-  if (f.pathWidth == 0) return 0;
+// Launches the raster of one fill whose header, bands, entries and windings
+// are on the device at dp.
+int raster_staged(pxh_image* img, const FillGeom& geo, const std::vector<char*>& dp, int32_t rowBase, int32_t nRows) {
+  const FillInfo& f = geo.info;
   const bool mask = f.mode == kMask;
-  int32_t rowBase, nRows;
-  if (mask) {
-    rowBase = 0;
-    nRows = img->h;
-  } else {
-    rowBase = f.startY;
-    nRows = f.pathHeight - f.startY;
-  }
-  if (nRows <= 0) return 0;
-  std::vector<char*> dp;
-  hipEvent_t staged;
-  int r = stage({{&f, sizeof(FillInfo)},
-                 {geo.parts.data(), geo.parts.size() * sizeof(PartInfo)},
-                 {geo.entries.data(), geo.entries.size() * sizeof(Entry)},
-                 {geo.windings.data(), geo.windings.size()}},
-                &dp, &staged);
-  if (r) return r;
-  struct Release {  // on every way out, also where no kernel follows the copy
-    hipEvent_t e;
-    ~Release() { (void)hipEventRecord(e, g.stream); }
-  } release{staged};
   // The row arrays hold one row's selection (the band entries that meet
   // [y, y + 1)), not the whole band: size them for the largest selection.
   const int maxSel = max_row_selection(geo);
@@ -472,6 +451,36 @@ int raster_fill(pxh_image* img, FillGeom& geo) {
       return fail(kErrDevice, std::string("fill launch: ") + hipGetErrorString(hipGetLastError()));
   }
   return 0;
+}
+
+// Launches the raster of one built fill onto img.
+int raster_fill(pxh_image* img, FillGeom& geo) {
+  FillInfo& f = geo.info;
+  if (f.pathWidth == 0) return 0;
+  int32_t rowBase, nRows;
+  if (f.mode == kMask) {
+    rowBase = 0;
+    nRows = img->h;
+  } else {
+    rowBase = f.startY;
+    nRows = f.pathHeight - f.startY;
+  }
+  if (nRows <= 0) return 0;
+  std::vector<char*> dp;
+  hipEvent_t staged;
+  int r = stage({{&f, sizeof(FillInfo)},
+                 {geo.parts.data(), geo.parts.size() * sizeof(PartInfo)},
+                 {geo.entries.data(), geo.entries.size() * sizeof(Entry)},
+                 {geo.windings.data(), geo.windings.size()}},
+                &dp, &staged);
+  if (r) return r;
+  r = raster_staged(img, geo, dp, rowBase, nRows);
+  // the slot is free behind the kernel, or the copy where none was launched
+  if (const hipError_t e = hipEventRecord(staged, g.stream); e != hipSuccess) {
+    (void)hipStreamSynchronize(g.stream);  // nothing marks the slot as read
+    return r ? r : fail(kErrDevice, std::string("hipEventRecord: ") + hipGetErrorString(e));
+  }
+  return r;
 }
 
 int check_image(const pxh_image* img) {
