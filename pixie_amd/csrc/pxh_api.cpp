@@ -404,14 +404,18 @@ int raster_staged(pxh_image* img, const FillGeom& geo, const std::vector<char*>&
   const int cap = next_pow2(maxSel > 2 ? maxSel : 2);
   const size_t capBytes = (size_t)cap * 24;
   // Every window of a row repeats the row's hits and walk, so windows are made
-  // wider, up to 1,536 px, while the rows still give each CU the 12 waves that
-  // its registers hold, the LDS of 12 waves fits it, and no row selects more
-  // than 64 entries (beyond, the sample lines' keys hold positions in 512 px).
-  // A rounded rectangle over 3,686 x 3,686: 68 us in 512-px windows, 45 us in
-  // 1,024-px ones.
+  // wider, up to 1,536 px, where that leaves a row fewer of them, the rows still
+  // give each CU 12 waves (of the 16 that its registers hold), the LDS of 12
+  // waves fits it, and no row selects more than 64 entries (beyond, the sample
+  // lines' keys hold positions in 512 px).  A rounded rectangle over 3,686 x
+  // 3,686 of an 8-bit canvas: 68 us in 512-px windows, 45 us in 1,024-px ones.
+  // 12 waves: opaque ones of RGBA8 over 3,539 x 3,539 and 2,016 x 3,840 take 77 and 39 us, with 8 waves 95
+  // and 49; of 960 x 3,840 28 us, with 16 waves 30.
   const int64_t spanPx = mask ? img->w : f.xhi - (f.xlo & ~3);
+  const auto windows = [spanPx](int w) { return (spanPx + w - 1) / w; };
   int ww = 512;
-  while (maxSel <= 64 && ww < 1536 && nRows * ((spanPx + ww + 511) / (ww + 512)) >= (int64_t)g.numCUs * 12 &&
+  while (maxSel <= 64 && ww < 1536 && windows(ww + 512) < windows(ww) &&
+         nRows * windows(ww + 512) >= (int64_t)g.numCUs * 12 &&
          12 * (8 * (size_t)(ww + 512) + 16 + capBytes) <= kCuLds)
     ww += 512;
   const size_t fixedBytes = 8 * (size_t)ww + 16;
