@@ -564,7 +564,7 @@ int get_lut(int radius, Ctx::BlurTable* out) {
 }
 
 int blur_impl(uint32_t* img, int32_t w, int32_t h, int radius, uint32_t oob, int lane = 0) {
-  if (!blur_radius_fits(radius, g.maxLds)) return fail(kErrCapacity, "blur radius too large for the LDS tiles");
+  if (!blur_radius_fits(radius, g.maxLds)) return fail(kErrCapacity, "blur radius too large");
   Ctx::BlurTable t;
   if (int r = get_lut(radius, &t)) return r;
   DevBuf& tmp = lane == 0 ? g.tmp : g.laneTmp[lane];
@@ -1998,7 +1998,7 @@ int pxh_blur_noalloc(pxh_image* img, float radius, uint32_t oob_rgbx) {
     return fail(kErrCapacity, "image larger than the allocation-free blur's scratch (4194304 pixels)");
   if (2 * r + 1 > (int64_t)kMaxLutTaps || !blur_radius_fits((int)r, g.maxLds) ||
       2 * r + 1 + blur_table_dwords((int)r) > (int64_t)kNoAllocLutWords)
-    return fail(kErrCapacity, "blur radius too large for the LDS tiles");
+    return fail(kErrCapacity, "blur radius too large");
   uint32_t* base = g.scratchPtr[g.device];
   if (!base) return fail(kErrDevice, "allocation-free scratch is not set up on this device");
   LutTaps taps;
@@ -2096,7 +2096,7 @@ int pxh_shadow(pxh_image* out, const pxh_image* src, float offset_x, float offse
   if (br < 0) return fail(kErrNegBlur, "Cannot apply negative blur");
   const int32_t w = src->w, h = src->h;
   if (br != 0 && (br > 1 << 20 || !blur_radius_fits((int)br, g.maxLds)))
-    return fail(kErrCapacity, "blur radius too large for the LDS tiles");
+    return fail(kErrCapacity, "blur radius too large");
   int64_t s = nim_f2i(roundf(spread));
   // mask = draw(image, translate(offset), OverwriteBlend) onto transparent
   // (images.nim:765-768): whole-pixel offsets fold into the spread pass's

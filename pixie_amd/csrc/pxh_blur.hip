@@ -34,7 +34,7 @@ typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 // line is there four times, copy s shifted by s bytes: byte x is read at
 // x - s of copy s = x & 3.
 constexpr int kTapPad = 64;
-__host__ __device__ __forceinline__ int tap_line(int r) { return (2 * r + 224) & ~15; }  // bytes
+constexpr __host__ __device__ __forceinline__ int tap_line(int r) { return (2 * r + 224) & ~15; }  // bytes
 int blur_table_dwords(int r) { return 3 * tap_line(r); }
 
 __global__ void __launch_bounds__(256) blur_table_kernel(const uint32_t* lut, int r, int8_t* tab) {
@@ -361,16 +361,22 @@ __global__ void __launch_bounds__(256, kWhole ? 3 : 2) blur_y_kernel(BlurArgs a)
   }
 }
 
+// LDS that a workgroup asks for: the lines of two digits (streamed blocks), and
+// a shadow's columns.
+constexpr size_t blur_lds(int r) { return 8 * (size_t)tap_line(r); }
+constexpr int shadow_blocks(int r) { return (16 + 2 * ((r + 15) & ~15) + 63) / 64; }
+constexpr size_t shadow_lds(int r) { return 64 * (48 + 64 * (size_t)shadow_blocks(r)); }
+
 template <int NT, bool kWhole, bool kThree = false>
 static void go_x(const BlurArgs& a, hipStream_t s) {
   const dim3 grid((a.w + 64 * NT - 1) / (64 * NT), (a.h + 15) / 16);
-  const size_t lds = kWhole ? NT * 3072 : 8 * (size_t)tap_line(a.radius);
+  const size_t lds = kWhole ? NT * 3072 : blur_lds(a.radius);
   hipLaunchKernelGGL((blur_x_kernel<NT, kWhole, kThree>), grid, dim3(256), lds, s, a);
 }
 template <int NT, int NC, bool kWhole, bool kThree = false>
 static void go_y(const BlurArgs& a, hipStream_t s) {
   const dim3 grid((a.w + 16 * NC - 1) / (16 * NC), (a.h + 64 * NT - 1) / (64 * NT));
-  const size_t lds = kWhole ? NT * 3072 : 8 * (size_t)tap_line(a.radius);
+  const size_t lds = kWhole ? NT * 3072 : blur_lds(a.radius);
   hipLaunchKernelGGL((blur_y_kernel<NT, NC, kWhole, kThree>), grid, dim3(256), lds, s, a);
 }
 
@@ -392,13 +398,19 @@ int launch_blur(const BlurArgs& ax, const BlurArgs& ay, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? 0 : kErrDevice;
 }
 
-// The radii that are accepted, by the size of a workgroup's LDS: those whose
-// 1,024-pixel row segments and 64 x 64 tiles of four channel planes, with
-// their borders and weights, fit it.
-bool blur_radius_fits(int r, size_t lds) {
+// The radii that are accepted stay those of the form before the matrix
+// products: 1,024-pixel row segments and 64 x 64 tiles of four channel planes,
+// with their borders and weights, in a workgroup's LDS (276 at 160 KB).  All of
+// them ask for less than the 64 KB that a launch gets without an attribute.
+constexpr bool blur_radius_accepted(int r, size_t lds) {
   const size_t nd = (size_t)(2 * (int64_t)r + 10) / 4;
   return (256 + 3 * nd) * 16 <= lds && (15 + nd) * 1024 + nd * 32 <= lds;
 }
+constexpr int kMaxRadius = 276;
+static_assert(blur_radius_accepted(kMaxRadius, 160 << 10) && !blur_radius_accepted(kMaxRadius + 1, 160 << 10),
+              "the largest radius");
+static_assert(blur_lds(kMaxRadius) <= 64 << 10 && shadow_lds(kMaxRadius) + 1024 <= 64 << 10, "no LDS attribute is set");
+bool blur_radius_fits(int r, size_t lds) { return r <= kMaxRadius && blur_radius_accepted(r, lds); }
 
 // Writes a Gaussian table passed by value into device memory (the
 // allocation-free blur keeps its table in static device scratch).
@@ -597,7 +609,6 @@ int launch_spread_y(const SpreadArgs& a, bool image, hipStream_t s) {
 // r = 16 takes 8 us, where the two passes on RGBA8 took 15 and 20 us.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ int shadow_border(int r) { return (r + 15) & ~15; }
-static int shadow_blocks(int r) { return (16 + 2 * ((r + 15) & ~15) + 63) / 64; }
 
 __device__ __forceinline__ uint32_t bytes_of(const Sums& s) {
   return high_bytes(div2(s.lo[0], s.hi[0], s.lo[1], s.hi[1]), div2(s.lo[2], s.hi[2], s.lo[3], s.hi[3]));
@@ -673,7 +684,7 @@ int launch_shadow(const ShadowArgs& a, hipStream_t s) {
     hipLaunchKernelGGL(shadow_color_kernel, dim3((a.w + 1023) / 1024, a.h), dim3(256), 0, s, a);
   } else {
     const int nb = shadow_blocks(a.radius);
-    const size_t lds = (size_t)64 * (48 + 64 * nb);
+    const size_t lds = shadow_lds(a.radius);
     if (nb == 1)
       hipLaunchKernelGGL(shadow_blur_kernel<true>, grid, dim3(256), lds, s, a);
     else

@@ -65,3 +65,19 @@ def test_shadow(gpu, orc, offset, spread, blur, w, h):
     color = (9, 120, 30, 200)
     got = gpu.Image.from_array(a).shadow(offset, spread, blur, color).download()
     assert np.array_equal(got, orc.shadow(a, offset, spread, blur, color))
+
+
+def test_largest_radius(gpu, orc):
+    a = picture(65, 133, 5)
+    want = a.copy()
+    orc.blur(want, 276, (1, 2, 3, 4))
+    img = gpu.Image.from_array(a)
+    img.blur(276, (1, 2, 3, 4))
+    assert np.array_equal(img.download(), want)
+    assert np.array_equal(img.shadow((1, 1), 0, 276, (9, 9, 9, 99)).download(),
+                          orc.shadow(want, (1, 1), 0, 276, (9, 9, 9, 99)))
+    for call in (lambda: img.blur(277), lambda: img.shadow((1, 1), 0, 277, (9, 9, 9, 99))):
+        with pytest.raises(gpu.PixieError) as e:
+            call()
+        assert e.value.code == 9
+    assert np.array_equal(img.download(), want)
