@@ -1782,9 +1782,11 @@ __device__ __forceinline__ int band_of_row(const FillInfo& F, int y) {
 // First cost class of the heavy kernel: one later for a scene of many tasks,
 // whose other rows keep the chip busy beside a row that takes one wave long
 // (the heavy kernel runs more instructions per row: its benefit is latency).
-// 1,023 x 767 with 100 paths (13 k tasks): 694 us from class 10, 928 from 11;
-// 4096 x 4096 with 2,000 paths (291 k): 1,849 and 1,741 us.
-constexpr int kManyTasks = 1 << 16;
+// Fills, three in ten stroked, by their tasks, from class 10 and 11: 45 k 606
+// and 866 us, 69 k 618 and 792, 92 k 738 and 871, 147 k 937 and 1,031, 200 k
+// 1,142 and 1,135, 266 k 1,451 and 1,310; all stroked, 102 k 909 and 1,009,
+// 147 k 1,145 and 1,142, 228 k 1,598 and 1,472.
+constexpr int kManyTasks = 3 << 16;
 __device__ __forceinline__ int heavy_class(const ScenePools& P) {
   return P.heavyClass + (P.counters[kCntTasks] > kManyTasks ? 1 : 0);
 }
