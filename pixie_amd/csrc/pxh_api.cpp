@@ -409,8 +409,8 @@ int raster_staged(pxh_image* img, const FillGeom& geo, const std::vector<char*>&
   // waves fits it, and no row selects more than 64 entries (beyond, the sample
   // lines' keys hold positions in 512 px).  A rounded rectangle over 3,686 x
   // 3,686 of an 8-bit canvas: 68 us in 512-px windows, 45 us in 1,024-px ones.
-  // 12 waves: opaque ones of RGBA8 over 3,539 x 3,539 and 2,016 x 3,840 take 77 and 39 us, with 8 waves 95
-  // and 49; of 960 x 3,840 28 us, with 16 waves 30.
+  // 12 waves: opaque ones of RGBA8 over 3,539 x 3,539 and 2,016 x 3,840 take 77
+  // and 39 us, with 8 waves 95 and 49; of 960 x 3,840 28 us, with 16 waves 30.
   const int64_t spanPx = mask ? img->w : f.xhi - (f.xlo & ~3);
   const auto windows = [spanPx](int w) { return (spanPx + w - 1) / w; };
   int ww = 512;
@@ -1074,26 +1074,18 @@ int scene_upload(pxh_scene* sc, int lane) {
   if (!sc->dashes.empty())
     PXH_HIP(hipMemcpyAsync(sc->dDashes, sc->dashes.data(), sc->dashes.size() * sizeof(float),
                            hipMemcpyHostToDevice, st));
-  // Geometry workgroups start longest call first, so that a long stroke does
-  // not start late and hold the kernel's end: estimated cost = commands,
-  // times the work of a stroke point (heavier with round joins or caps).
+  // Geometry workgroups start longest call first, so that a long call does
+  // not start late and hold the kernel's end.
   {
     const size_t n = sc->items.size();
-    std::vector<int64_t> cost(n);
-    for (size_t i = 0; i < n; i++) {
-      const SceneItem& it = sc->items[i];
-      int64_t c = it.cmdCount;
-      if (it.stroke && !it.strokeNone) c *= (it.join == 1 || it.cap == 1) ? 16 : 4;
-      cost[i] = c;
-    }
-    // calls of more than 256 commands first: their geometry runs in
-    // 1024-thread workgroups of a launch of its own
+    // calls of more than 256 commands first: their geometry is spread over the
+    // device, in launches of its own
     auto big = [&](int32_t i) { return sc->items[i].cmdCount > 256; };
     sc->order.resize(n);
     for (size_t i = 0; i < n; i++) sc->order[i] = (int32_t)i;
     std::stable_sort(sc->order.begin(), sc->order.end(), [&](int32_t a, int32_t b) {
       if (big(a) != big(b)) return big(a);
-      return cost[a] > cost[b];
+      return sc->items[a].cmdCount > sc->items[b].cmdCount;
     });
     sc->nBig = 0;
     for (size_t i = 0; i < n; i++) sc->nBig += big((int32_t)i) ? 1 : 0;
