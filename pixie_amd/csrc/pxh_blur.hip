@@ -429,7 +429,7 @@ int launch_lut_store(const LutTaps& t, uint32_t* dst, hipStream_t s) {
 // takes the least of the window: the greatest of the complements.  Bytes are
 // compared as the 16-bit halves of even and odd bytes.  Bound by latency at the
 // sizes of layers, so each pass has several loads in flight.  1,921 x 1,081,
-// both passes: 16 us at spread 4 and 31 at 20; a pixel to a thread 27 and 82.
+// both passes: 15 us at spread 4 and 29 at 20; a pixel to a thread 27 and 82.
 // ---------------------------------------------------------------------------
 struct MaxBytes {
   u16x2 even = {0, 0}, odd = {0, 0};
@@ -535,21 +535,23 @@ __global__ void __launch_bounds__(256) spread_y_kernel(SpreadArgs a) {
   const int32_t s = a.s;
   const int32_t lo = y0 - s > 0 ? y0 - s : 0, hi = (int64_t)y0 + kRows - 1 + s < a.h - 1 ? y0 + kRows - 1 + s : a.h - 1;
   MaxBytes best[kRows];
-  for (int32_t yb = lo; yb <= hi; yb += 4) {  // four rows in flight; the last again past the end
+  // four rows in flight; past the end the last again
+  auto four = [&](int32_t yb, bool clamp) {
     uint32_t v[4];
 #pragma unroll
     for (int u = 0; u < 4; u++)
-      v[u] = *(const uint32_t*)(a.plane + (size_t)(yb + u < hi ? yb + u : hi) * a.pitch + x) ^ flip;
+      v[u] = *(const uint32_t*)(a.plane + (size_t)(clamp && yb + u > hi ? hi : yb + u) * a.pitch + x) ^ flip;
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      const int32_t yy = yb + u < hi ? yb + u : hi;
+    for (int u = 0; u < 4; u++)
 #pragma unroll
       for (int i = 0; i < kRows; i++) {
-        const int32_t d = yy - (y0 + i);
+        const int32_t d = (clamp && yb + u > hi ? hi : yb + u) - (y0 + i);
         if (d >= -s && d <= s) best[i].add(v[u]);
       }
-    }
-  }
+  };
+  int32_t yb = lo;
+  for (; yb + 3 <= hi; yb += 4) four(yb, false);
+  if (yb <= hi) four(yb, true);
 #pragma unroll
   for (int i = 0; i < kRows; i++) {
     if (y0 + i >= a.h) break;

@@ -24,7 +24,7 @@ namespace pxh {
 
 // mix(ColorRGBX, ColorRGBX, t), common.nim:59-65
 __device__ __forceinline__ uint32_t mix_rgbx(uint32_t a, uint32_t b, float t) {
-  const float v = t * 255.0f;  // t in [0, 1): round half up is roundf
+  const float v = t * 255.0f;  // t in [0, 1] (v - floor(v) rounds to 1 just below 0): half up is roundf
   const uint32_t n = (uint32_t)v;
   const uint32_t x = n + (v - (float)n >= 0.5f ? 1u : 0u);
   // sums of two products of weights that add up to 255, plus 127: 16 bits,

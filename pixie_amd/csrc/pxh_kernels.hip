@@ -6,7 +6,7 @@
 //   composite_kernel   blendRect (images.nim:468-529), all 20 blend modes
 //   opacity_kernel     applyOpacity (images.nim:261-277)
 //
-// Every kernel is memory-bound integer / float32 work: no MFMA.
+// No kernel here is a contraction: integer and float32 arithmetic, no MFMA.
 #include <hip/hip_runtime.h>
 
 #include "pxh_kernels.h"
@@ -14,10 +14,11 @@
 
 namespace pxh {
 
-
 // ---------------------------------------------------------------------------
 // fill: one wave (64 threads) per workgroup, grid-stride over (row, window)
-// units
+// units.  100 KB of code with the twenty blend modes and the row program's
+// forms in line; at the 128 VGPRs of four waves a SIMD it spills 11 VGPRs and
+// 194 SGPRs (48 B of scratch a lane).
 // ---------------------------------------------------------------------------
 template <bool kA8>
 __global__ void __launch_bounds__(64, 4) fill_rows_kernel(FillArgs a) {

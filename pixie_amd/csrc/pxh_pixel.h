@@ -21,8 +21,8 @@ namespace pxh {
 // division takes (a quarter of the other instructions' rate).
 PXH_HD uint32_t div255(uint32_t x) { return (x + 1u + (x >> 8)) >> 8; }
 
-// (c * k + add) div 255 of each of a pixel's channels, k and add < 256: pairs
-// of channels in 16-bit halves (c * k + add + 1 + 254 < 2^16).
+// (c * k + add) div 255 of each of a pixel's channels, k < 256, add <= 254: pairs
+// of channels in 16-bit halves (255 * 255 + add + 1 + 254 < 2^16).
 PXH_HD uint32_t mul_div255(uint32_t c, uint32_t k, uint32_t add) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));

@@ -253,11 +253,12 @@ struct ScenePools {
 
 // Phase-A launch shapes: the band entries the rows kernel's waves keep in LDS
 // (larger selections in the global row scratch), its waves per CU, and the
-// first cost class of the heavy kernel.  16 waves per CU are what 128 VGPRs
-// allow; 20 waves of 96 spilled 39 of them and ran no faster (scene of 2,000
-// paths on 4096 x 4096 1,742 and 1,749 us, paragraph of 820 glyphs 576 and
-// 541 us).  A scene's autotuner picks one;
-// run-pool sizing assumes the most waves any shape has.
+// first cost class of the heavy kernel (one later in scenes of many tasks).
+// 16 waves per CU are what 128 VGPRs allow, where the rows kernel spills 4 of
+// them (20 B of scratch a lane) and keeps about 200 SGPRs in VGPR lanes; 20
+// waves of 96 spilled 39 and ran no faster (scene of 2,000 paths on 4096 x 4096
+// 1,742 and 1,749 us, paragraph of 820 glyphs 576 and 541 us).  A scene's
+// autotuner picks one; run-pool sizing assumes the most waves any shape has.
 constexpr int kHeavyWins = 2;          // windows of a heavy row's work item
 constexpr int kHeavyWavesPerGroup = 4;  // waves of a heavy kernel workgroup
 constexpr int kHeavyGroupsPerCU = 5;

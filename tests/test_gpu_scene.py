@@ -330,8 +330,8 @@ def test_scene_band_over_capacity_renders(gpu):
 
 
 def test_scene_big_calls(gpu, orc):
-    # calls of more than 256 commands take the 1024-thread geometry
-    # workgroups: 300 circles in one fill (1,800 commands), a 400-segment
+    # calls of more than 256 commands are laid out across the device, in
+    # chunks: 300 circles in one fill (1,800 commands), a 400-segment
     # polyline stroked with round joins and dashes, a 600-command EvenOdd
     # fill, each between small calls
     rng = np.random.default_rng(31)
@@ -508,9 +508,8 @@ def test_scene_heavy_runs_replayed(gpu):
 
 @pytest.mark.parametrize("shape", range(6))
 def test_scene_every_phase_a_shape(gpu, shape):
-    # every phase-A launch shape the autotuner may pick (one launch, or the
-    # large-band tasks in a second launch beside or before the rest) draws
-    # the per-call image, on a mixed scene with large bands and on combs
+    # every phase-A launch shape the autotuner may pick (entries in LDS, waves
+    # per CU, the bands whose rows take a workgroup) draws the per-call image, on a mixed scene with large bands and on combs
     cmds, canvas = WL.mixed_scene(seed=13, n_paths=120, W=768, H=512)
     ref = px.Image.from_array(canvas)
     sc = px.Scene()
