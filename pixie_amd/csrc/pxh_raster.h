@@ -1227,7 +1227,7 @@ __device__ int32_t row_program(const RowCtx& C, RowLds& L) {
       whole = 0;
       row_coverage_presorted(Cp, L, ne, yLine, offset, F.rule, cs);
     }
-    for (int m = 0; whole != 0; m++, whole >>= 1) {
+    for (; whole != 0; whole >>= 1) {
       yLine += offset;
       if (whole & 1u) {  // pixie's walk of the whole line
         wave_walk(L, row_hits(Cp, L, ne, yLine, S), F.rule, cs);
